@@ -309,7 +309,7 @@ def line_search_ms(mdz, hot, ctx, reps):
 
 def device_solve(mdz, hot, ncx, ncz, seed, penalty=1e5):
     """The device solve of the Newton correction (KillerSolver: Powell-Hestenes
-    iterations around GCR, preconditioned by the band Cholesky factor of the
+    iterations around GCR, preconditioned by the sparse Cholesky factor of the
     penalised Picard operator) on the blocks of one Newton-iteration unit of
     a lithosphere model; the second of two solves is reported (the first
     one initialises the dense-algebra libraries).  Not the metric."""
@@ -330,8 +330,7 @@ def device_solve(mdz, hot, ncx, ncz, seed, penalty=1e5):
         return {"workload": "lithosphere %dx%d cells, penalty %g, first Newton iteration" % (ncx, ncz, penalty),
                 "momentum_unknowns": nu.value, "ms": round(wall, 1), "factor_ms": round(info.factor_ms, 1),
                 "iterate_ms": round(info.iterate_ms, 1), "ph_its": info.ph_its,
-                "ksp_its": list(info.ksp_its[:info.ph_its]), "kd": info.kd, "nb": info.nb,
-                "band_GB": round((info.kd + info.nb) * nu.value * 8 / 1e9, 2),
+                "ksp_its": list(info.ksp_its[:info.ph_its]), "kd": info.kd,
                 "ms_per_gcr_iteration": round(info.iterate_ms / max(1, info.ksp_its_total), 2)}
     finally:
         hot.mdz_ctx_destroy(ctx)

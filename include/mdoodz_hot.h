@@ -292,7 +292,7 @@ typedef struct _DirectSolver DirectSolver;
  * system with the Picard blocks matA..matD (preconditioner) and the
  * Jacobian blocks JmatA..JmatC (operator): sol[0 .. neq_mom) = du,
  * sol[neq_mom ..) = dp.  Powell-Hestenes iterations around the restarted
- * GCR of kspgcr, preconditioned by a band Cholesky factor of the penalised
+ * GCR of kspgcr, preconditioned by a sparse Cholesky factor of the penalised
  * operator on the device (in place of CHOLMOD's); pardi is not read.
  * Penalty, tolerances and pc_type come from model, the equation numbering
  * from Stokes, the grid dimensions, comp_cells and bet_n from mesh. */
@@ -521,7 +521,7 @@ typedef struct {
     int    ph_its;        /* Powell-Hestenes iterations */
     int    ksp_its_total; /* GCR iterations, counted as kspgcr counts them */
     int    ksp_its[20];   /* per Powell-Hestenes iteration */
-    int    kd, nb;        /* lower bandwidth of the factor in its ordering; block size */
+    int    kd, nb;        /* half bandwidth of Jts by grid columns or rows (the narrower); nb as asked (1024 for 0) */
     double maxdiv0, maxdiv, maxru0, maxru; /* the reference's stopping quantities */
     double resx, resz, resp; /* rms of the final residual over the u, v, p equations */
     double factor_ms, iterate_ms; /* host wall time of the factorisation and the iterations */
@@ -532,8 +532,9 @@ typedef struct {
  * and the residual F of the last unit, then ScaleVelocitiesRHSBack where
  * the blocks are scaled.  The correction stays on the device for
  * mdz_ctx_line_search (dx = NULL) and is copied to dx (neq_mom + neq_cont
- * values by equation number) when dx is not NULL.  nb: block size of the
- * triangular solves (0: 1024; a multiple of 64).  Penalty (default 1e10), abs_tol_div
+ * values by equation number) when dx is not NULL.  nb: 0 or a
+ * multiple of 64, reported in info; the factor's layout does not depend on
+ * it.  Penalty (default 1e10), abs_tol_div
  * (1e-14), rel_tol_div (1e-5) and rel_tol_KSP (1e-4) from the context's
  * params, the reference's input defaults where they are 0, and pc_type (0:
  * the Picard operator as preconditioner, 1: the symmetrised Jacobian).

@@ -43,12 +43,12 @@ struct SolverPattern {
     const int *Ic, *J;
 };
 
-/* Band ordering of the momentum unknowns from the node of each momentum
- * row (u node k + l Nx, v node Nx (Nz + 1) + k + l (Nx + 1)), and the
- * patterns of Jts and Js, from the host patterns of the Picard A, B, C and
+/* Analysis of the factor from the node of each momentum row (u node
+ * k + l Nx, v node Nx (Nz + 1) + k + l (Nx + 1)), and the patterns of Jts and Js, from the host patterns of the Picard A, B, C and
  * Jacobian A, B blocks, for the preconditioner pc_type (0: PC = A; 1:
- * PC = (AJ + AJ^T) / 2); nb is the block size of the triangular solves (0:
- * default).  Kept until the next call. */
+ * PC = (AJ + AJ^T) / 2); nb (0, or a multiple of 64) is
+ * checked and reported only: the factor's tiles do not depend on it.  Kept
+ * until the next call. */
 int mdz_solver_order(MdzSolver *sv, int Nx, int Nz, int nu, int np, const int *mom_node, const SolverPattern &A,
                      const SolverPattern &B, const SolverPattern &C, const SolverPattern &AJ, const SolverPattern &BJ,
                      int pc_type, int nb);

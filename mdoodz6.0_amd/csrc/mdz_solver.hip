@@ -18,22 +18,8 @@
  * the residuals (Solvers.c:2536-2560).
  *
  * MI355X design:
- *  - the factor replaces CHOLMOD's supernodal one by a band Cholesky: the
- *    momentum unknowns are ordered column by column of the staggered grid
- *    (or row by row, whichever gives the narrower band), so that Jts has a
- *    lower bandwidth kd of about twice the shorter grid dimension.  Storage
- *    is LAPACK band storage with ldab = kd + nb rows per column (element
- *    (r, c) at ab[(r - c) + c ldab]); rows kd+1 .. ldab-1 of each column
- *    are zero padding, so that every window of the blocked right-looking
- *    factorisation is a dense column-major matrix with leading dimension
- *    ldab - 1 (for any step width up to nb).  Each factor step of 64
- *    columns is one potrf (64 x 64), one trsm (kd x 64) and one syrk
- *    (kd x kd, rank 64) on the matrix cores (rocSOLVER, rocBLAS);
- *  - the inverses of the nb x nb diagonal blocks (nb = 1024 by default,
- *    the triangular solves' block) are formed once per
- *    factorisation (batched trtri), so that each block step of the
- *    triangular solves is two matrix-vector products that spread over the
- *    whole chip (no sequential substitution inside a block);
+ *  - the factor replaces CHOLMOD's supernodal one by a sparse Cholesky on
+ *    the matrix cores (mdz_factor.hip);
  *  - Jts and Js are assembled once per solve, by one value function on
  *    patterns built with the ordering: their penalty entries are about
  *    penalty / celvol times larger than the viscous ones, and a
@@ -45,8 +31,6 @@
  *    fixed order (results independent of scheduling).
  */
 #include <hip/hip_runtime.h>
-#include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <math.h>
 #include <stdarg.h>
@@ -56,8 +40,11 @@
 
 #include <algorithm>
 #include <chrono>
+#include <mutex>
 #include <vector>
 
+#include "mdz_factor.h"
+#include "mdz_host_parallel.h"
 #include "mdz_solver.h"
 
 int mdz_error(int code, const char *msg);
@@ -66,9 +53,6 @@ int mdz_error(int code, const char *msg);
 #define SV_MAXIT 1000
 #define SV_NITMAX 20
 #define SV_NB_DEFAULT 1024
-#ifndef SV_NBF
-#define SV_NBF 64 /* columns per factor step */
-#endif
 #define SV_RED 512 /* blocks of the reduction kernels (fixed: deterministic sums) */
 #define SV_BLK 256
 
@@ -89,19 +73,11 @@ static int sv_err(int code, const char *fmt, ...) {
         hipError_t _e = (x);                                                                       \
         if (_e != hipSuccess) return sv_err(MDZ_EHIP, "%s: %s", #x, hipGetErrorString(_e));        \
     } while (0)
-#define SVBLAS(x)                                                                                  \
-    do {                                                                                           \
-        rocblas_status _s = (x);                                                                   \
-        if (_s != rocblas_status_success) return sv_err(MDZ_EHIP, "%s: rocBLAS status %d", #x, (int)_s); \
-    } while (0)
-
 struct MdzSolver {
     hipStream_t s = nullptr;
-    rocblas_handle h = nullptr;
-    int n = 0, np = 0, kd = 0, nb = 0, nblk = 0, nequ = 0;
-    long long ldab = 0;
-    int *pos = nullptr; /* band position of each momentum equation */
-    int *eq = nullptr;  /* momentum equation at each band position */
+    int n = 0, np = 0, kd = 0, nb = 0, nequ = 0;
+    MdzFactor *fac = nullptr; /* factor of Jts */
+    bool ordered = false;
     /* patterns of Jts = A - B Dpen C and Js = AJ - BJ Dpen C (unique sorted
      * columns per row), their values */
     int *ts_Ic = nullptr, *ts_J = nullptr, *js_Ic = nullptr, *js_J = nullptr;
@@ -110,22 +86,16 @@ struct MdzSolver {
     /* pc_type 1: AJ's transpose (row i: the entries of AJ's column i, their rows) */
     int pc_type = 0;
     int *tr_Ic = nullptr, *tr_J = nullptr, *tr_src = nullptr;
-    double *ab = nullptr;
-    size_t ab_len = 0;
-    double *linv = nullptr; /* inverses of the diagonal blocks, nb x nb column-major each */
-    size_t linv_len = 0;
-    int *info = nullptr; /* potrf then trtri status per block */
-    size_t info_len = 0;
     /* vectors */
     double *work = nullptr;
     size_t work_len = 0;
-    double *udum, *f, *sv, *v, *r, *y, *t, *xb, *fu, *pdum, *fp, *tc, *VV, *SS;
+    double *udum, *f, *sv, *v, *fu, *pdum, *fp, *tc, *VV, *SS;
     size_t ldv = 0;
     /* captured preconditioner application (f -> sv), and what it was captured for */
     hipGraph_t pc_graph = nullptr;
     hipGraphExec_t pc_exec = nullptr;
-    const void *pc_key[6] = {};
-    long long pc_dims[3] = {};
+    const void *pc_key[2] = {};
+    unsigned long long pc_version = 0;
     double *partial = nullptr; /* SV_RED * 32 */
     double *dscal = nullptr;   /* device scalars: 0..31 dots, 32.. misc */
     double *hscal = nullptr;   /* pinned host copy */
@@ -178,7 +148,7 @@ __global__ void __launch_bounds__(SV_BLK) k_final(const double *partial, int nq,
 }
 
 /* ------------------------------------------------------------------ */
-/* band matrix                                                          */
+/* the assembled operators                                              */
 /* ------------------------------------------------------------------ */
 struct CsrView {
     const int *Ic, *J;
@@ -227,159 +197,6 @@ __global__ void __launch_bounds__(SV_BLK) k_schur_values(int n, const int *Ic, c
     for (int e = e0; e < e1; e++) val[e] = -val[e];
 }
 
-/* The factor's matrix: the lower triangle (column <= row, equation order)
- * of Jts placed at the band positions of its rows and columns (one writer
- * per element: the pattern has unique columns in a row) */
-__global__ void __launch_bounds__(SV_BLK) k_band_fill(int n, const int *pos, const int *Ic, const int *J,
-                                                      const double *val, double *ab, long long ldab) {
-    const int i = blockIdx.x * SV_BLK + threadIdx.x;
-    if (i >= n) return;
-    const long long pi = pos[i];
-    for (int e = Ic[i]; e < Ic[i + 1]; e++) {
-        const int j = J[e];
-        if (j > i) continue;
-        const long long pj = pos[j];
-        const long long r = pi > pj ? pi : pj, c = pi > pj ? pj : pi;
-        ab[(r - c) + c * ldab] = val[e];
-    }
-}
-
-/* Diagonal block b of the factor (lower triangle) into linv[b] (nb x nb),
- * upper triangle zero, the rows beyond a short last block set to identity. */
-__global__ void __launch_bounds__(SV_BLK) k_diag_blocks(const double *ab, long long ldab, int n, int nb, double *linv) {
-    const int b = blockIdx.x;
-    const long long i0 = (long long)b * nb;
-    const int ib = (int)min((long long)nb, n - i0);
-    double *L = linv + (size_t)b * nb * nb;
-    for (int e = threadIdx.x; e < nb * nb; e += SV_BLK) {
-        const int r = e % nb, c = e / nb;
-        double x;
-        if (r < ib && c < ib) x = r >= c ? ab[(r - c) + (i0 + c) * ldab] : 0.0;
-        else x = r == c ? 1.0 : 0.0;
-        L[e] = x;
-    }
-}
-
-/* ------------------------------------------------------------------ */
-/* triangular solves, one block step per launch                         */
-/* ------------------------------------------------------------------ */
-/* Row-block products of the forward solve: 16 rows per block of 256
- * threads, the column range split over 16 column groups (a wave reads 16
- * contiguous rows of 4 adjacent columns), partial sums added in a fixed
- * order through LDS. */
-#define TS_R 16
-#define TS_S 16
-
-/* sum over j = j0, j0 + TS_S, .. < j1 of p[j * ld] * v[j]: up to 32 terms
- * per thread (nb <= 512) are loaded in one batch before any is used, so
- * that a block step's whole panel is in flight at once (a step moves only a
- * few MB: its time is one memory latency, not a bandwidth); longer ranges
- * continue in further batches.  Partial sums are added in a fixed order. */
-#define SD_U 32
-__device__ __forceinline__ double strided_dot(const double *__restrict__ p, long long ld,
-                                              const double *__restrict__ v, int j0, int j1) {
-    double acc = 0.0;
-    for (int jb = j0; jb < j1; jb += SD_U * TS_S) {
-        double a[SD_U], b[SD_U];
-#pragma unroll
-        for (int u = 0; u < SD_U; u++) {
-            const int j = jb + u * TS_S;
-            a[u] = j < j1 ? p[(long long)j * ld] : 0.0;
-            b[u] = j < j1 ? v[j] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < SD_U; u++) acc += a[u] * b[u];
-    }
-    return acc;
-}
-
-/* y[0..ib) = Linv r[0..ib) (Linv's upper triangle is zero) */
-__global__ void __launch_bounds__(SV_BLK) k_fwd_diag(const double *Linv, int nb, int ib, const double *r, double *y) {
-    __shared__ double red[TS_S][TS_R];
-    const int lr = threadIdx.x % TS_R, cg = threadIdx.x / TS_R;
-    const int row = blockIdx.x * TS_R + lr;
-    const int jend = min(ib, (int)blockIdx.x * TS_R + TS_R);
-    const double acc = row < ib ? strided_dot(Linv + row, nb, r, cg, jend) : 0.0;
-    red[cg][lr] = acc;
-    __syncthreads();
-    if (cg == 0 && row < ib) {
-        double sum = 0.0;
-#pragma unroll
-        for (int q = 0; q < TS_S; q++) sum += red[q][lr];
-        y[row] = sum;
-    }
-}
-
-/* r[i0 + ib + a] -= sum_j L(i0 + ib + a, i0 + j) y[i0 + j], a < m: the panel
- * below the diagonal block, column by column (contiguous in a); the band's
- * zero padding covers the elements beyond kd */
-__global__ void __launch_bounds__(SV_BLK) k_fwd_panel(const double *ab, long long ldab, int kd, long long i0, int ib,
-                                                      int m, const double *y, double *r) {
-    __shared__ double red[TS_S][TS_R];
-    const int lr = threadIdx.x % TS_R, cg = threadIdx.x / TS_R;
-    const int a0 = blockIdx.x * TS_R, a = a0 + lr;
-    const int j0 = max(0, ib + a0 - kd);
-    const double acc = a < m ? strided_dot(ab + i0 * ldab + ib + a, ldab - 1, y + i0, j0 + cg, ib) : 0.0;
-    red[cg][lr] = acc;
-    __syncthreads();
-    if (cg == 0 && a < m) {
-        double sum = 0.0;
-#pragma unroll
-        for (int q = 0; q < TS_S; q++) sum += red[q][lr];
-        r[i0 + ib + a] -= sum;
-    }
-}
-
-/* sum over a = l, l + 64, .. < a1 of p[a] v[a]: 16 terms per lane loaded
- * in one batch (a column of kd <= 1024 rows at once) */
-#define LD_U 16
-__device__ __forceinline__ double lane_dot(const double *__restrict__ p, const double *__restrict__ v, int l, int a1) {
-    double acc = 0.0;
-    for (int ab = l; ab < a1; ab += LD_U * 64) {
-        double x[LD_U], w[LD_U];
-#pragma unroll
-        for (int u = 0; u < LD_U; u++) {
-            const int a = ab + u * 64;
-            x[u] = a < a1 ? p[a] : 0.0;
-            w[u] = a < a1 ? v[a] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < LD_U; u++) acc += x[u] * w[u];
-    }
-    return acc;
-}
-
-/* t[i0 + j] = y[i0 + j] - sum_a L(i0 + ib + a, i0 + j) x[i0 + ib + a]: one
- * wave per column j (contiguous in a) */
-__global__ void __launch_bounds__(SV_BLK) k_bwd_panel(const double *ab, long long ldab, int kd, long long i0, int ib,
-                                                      int m, const double *x, const double *y, double *t) {
-    const int j = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
-    if (j >= ib) return;
-    const int aend = min(m, kd + j - ib + 1);
-    const double *col = ab + (i0 + j) * ldab + (ib - j);
-    const double acc = wave_sum(lane_dot(col, x + i0 + ib, l, aend));
-    if (l == 0) t[i0 + j] = y[i0 + j] - acc;
-}
-
-/* x[i0 + j] = sum_{r >= j} Linv(r, j) t[i0 + r]: one wave per column */
-__global__ void __launch_bounds__(SV_BLK) k_bwd_diag(const double *Linv, int nb, int ib, long long i0, const double *t,
-                                                     double *x) {
-    const int j = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
-    if (j >= ib) return;
-    const double *col = Linv + (size_t)j * nb + j;
-    const double acc = wave_sum(lane_dot(col, t + i0 + j, l, ib - j));
-    if (l == 0) x[i0 + j] = acc;
-}
-
-__global__ void k_gather(int n, const int *eq, const double *f, double *r) {
-    const int p = blockIdx.x * SV_BLK + threadIdx.x;
-    if (p < n) r[p] = f[eq[p]];
-}
-__global__ void k_scatter(int n, const int *eq, const double *x, double *s) {
-    const int p = blockIdx.x * SV_BLK + threadIdx.x;
-    if (p < n) s[eq[p]] = x[p];
-}
-
 /* ------------------------------------------------------------------ */
 /* sparse products and the iteration's vector steps                     */
 /* ------------------------------------------------------------------ */
@@ -389,12 +206,34 @@ __device__ __forceinline__ double row_dot(const CsrView &M, int i, const double 
     return s;
 }
 
-/* out = M x, or b - M x where b is not null */
-__global__ void __launch_bounds__(SV_BLK) k_csr_apply(int n, CsrView M, const double *x, const double *b, double *out) {
+/* b - row i of M x with products and sums carried in two doubles (the error
+ * of each is exact: Ogita, Rump and Oishi 2005, Dot2).  The penalty entries
+ * make a residual the difference of terms about 1e5 times larger, whose
+ * rounding the soft modes amplify: in plain doubles it is what bounds the
+ * correction's accuracy.  The rows are read at memory speed either way. */
+__device__ __forceinline__ double row_residual(const CsrView &M, int i, const double *x, double b) {
+    double s = b, c = 0.0;
+    for (int e = M.Ic[i]; e < M.Ic[i + 1]; e++) {
+        const double a = -M.A[e], y = x[M.J[e]];
+        const double p = a * y, q = __builtin_fma(a, y, -p);
+        const double t = s + p, z = t - s;
+        c += ((s - (t - z)) + (p - z)) + q;
+        s = t;
+    }
+    return s + c;
+}
+
+/* out = M x */
+__global__ void __launch_bounds__(SV_BLK) k_csr_apply(int n, CsrView M, const double *x, double *out) {
     const int i = blockIdx.x * SV_BLK + threadIdx.x;
-    if (i >= n) return;
-    const double mx = row_dot(M, i, x);
-    out[i] = b ? b[i] - mx : mx;
+    if (i < n) out[i] = row_dot(M, i, x);
+}
+
+/* out = b - M x */
+__global__ void __launch_bounds__(SV_BLK) k_csr_residual(int n, CsrView M, const double *x, const double *b,
+                                                         double *out) {
+    const int i = blockIdx.x * SV_BLK + threadIdx.x;
+    if (i < n) out[i] = row_residual(M, i, x, b[i]);
 }
 
 /* udum = (bu - BJ (Dpen bp)) - BJ (incomp dp)  (Solvers.c:2510-2516) */
@@ -417,7 +256,7 @@ __global__ void __launch_bounds__(SV_BLK) k_ph_dp(int np, CsrView CJ, const doub
                                                   const double *D1, const double *Dpen, double *dp) {
     const int k = blockIdx.x * SV_BLK + threadIdx.x;
     if (k >= np) return;
-    const double pd = (bp[k] - row_dot(CJ, k, du)) - D1[k] * dp[k];
+    const double pd = row_residual(CJ, k, du, bp[k]) - D1[k] * dp[k];
     dp[k] = Dpen[k] * pd + dp[k];
 }
 
@@ -593,11 +432,11 @@ int mdz_solver_create(MdzSolver **out, hipStream_t s) {
     if (!out) return sv_err(MDZ_EINVAL, "solver: null output");
     MdzSolver *S = new MdzSolver();
     S->s = s;
-    if (rocblas_create_handle(&S->h) != rocblas_status_success) {
+    const int rc = mdz_factor_create(&S->fac, s);
+    if (rc) {
         delete S;
-        return sv_err(MDZ_EHIP, "rocblas_create_handle failed");
+        return rc;
     }
-    rocblas_set_stream(S->h, s);
     hipError_t e = hipMalloc((void **)&S->partial, (size_t)SV_RED * 32 * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void **)&S->dscal, 128 * sizeof(double));
     if (e == hipSuccess) e = hipHostMalloc((void **)&S->hscal, 128 * sizeof(double), hipHostMallocDefault);
@@ -609,23 +448,16 @@ int mdz_solver_create(MdzSolver **out, hipStream_t s) {
     return MDZ_OK;
 }
 
-static void free_factor(MdzSolver *S) {
-    hipFree(S->ab); S->ab = nullptr; S->ab_len = 0;
-    hipFree(S->linv); S->linv = nullptr; S->linv_len = 0;
-    hipFree(S->info); S->info = nullptr; S->info_len = 0;
-}
-
 void mdz_solver_destroy(MdzSolver *S) {
     if (!S) return;
     if (S->s) hipStreamSynchronize(S->s);
-    free_factor(S);
     if (S->pc_exec) hipGraphExecDestroy(S->pc_exec);
     if (S->pc_graph) hipGraphDestroy(S->pc_graph);
-    hipFree(S->pos); hipFree(S->eq); hipFree(S->work); hipFree(S->partial); hipFree(S->dscal);
+    mdz_factor_destroy(S->fac);
+    hipFree(S->work); hipFree(S->partial); hipFree(S->dscal);
     hipFree(S->ts_Ic); hipFree(S->ts_J); hipFree(S->js_Ic); hipFree(S->js_J); hipFree(S->ts_val); hipFree(S->js_val);
     hipFree(S->tr_Ic); hipFree(S->tr_J); hipFree(S->tr_src);
     if (S->hscal) hipHostFree(S->hscal);
-    if (S->h) rocblas_destroy_handle(S->h);
     delete S;
 }
 
@@ -661,27 +493,46 @@ static void band_order(int Nx, int Nz, int n, const int *mom_node, bool by_x, st
 static void schur_pattern(int n, const int *Pi, const int *Pj, const int *Bi, const int *Bj, const int *Ci,
                           const int *Cj, std::vector<int> &Ic, std::vector<int> &J) {
     Ic.assign((size_t)n + 1, 0);
-    J.clear();
-    std::vector<int> row;
-    for (int i = 0; i < n; i++) {
-        row.clear();
-        for (int e = Pi[i]; e < Pi[i + 1]; e++) row.push_back(Pj[e]);
-        for (int eb = Bi[i]; eb < Bi[i + 1]; eb++) {
-            const int k = Bj[eb];
-            for (int ec = Ci[k]; ec < Ci[k + 1]; ec++) row.push_back(Cj[ec]);
+    std::mutex mu;
+    std::vector<std::pair<long long, std::vector<int>>> part; /* (first row, columns of the chunk's rows) */
+    mdz_host_parallel(n, 8192, [&](long long i0, long long i1) {
+        std::vector<int> out, row;
+        for (long long i = i0; i < i1; i++) {
+            row.clear();
+            for (int e = Pi[i]; e < Pi[i + 1]; e++) row.push_back(Pj[e]);
+            for (int eb = Bi[i]; eb < Bi[i + 1]; eb++) {
+                const int k = Bj[eb];
+                for (int ec = Ci[k]; ec < Ci[k + 1]; ec++) row.push_back(Cj[ec]);
+            }
+            std::sort(row.begin(), row.end());
+            row.erase(std::unique(row.begin(), row.end()), row.end());
+            out.insert(out.end(), row.begin(), row.end());
+            Ic[(size_t)i + 1] = (int)row.size();
         }
-        std::sort(row.begin(), row.end());
-        row.erase(std::unique(row.begin(), row.end()), row.end());
-        J.insert(J.end(), row.begin(), row.end());
-        Ic[(size_t)i + 1] = (int)J.size();
-    }
+        std::lock_guard<std::mutex> g(mu);
+        part.emplace_back(i0, std::move(out));
+    });
+    for (int i = 0; i < n; i++) Ic[(size_t)i + 1] += Ic[i];
+    J.resize((size_t)Ic[n]);
+    mdz_host_parallel((long long)part.size(), 1, [&](long long q0, long long q1) {
+        for (long long q = q0; q < q1; q++)
+            std::copy(part[(size_t)q].second.begin(), part[(size_t)q].second.end(),
+                      J.begin() + Ic[(size_t)part[(size_t)q].first]);
+    });
 }
 
 /* largest |pos(i) - pos(j)| over a pattern */
 static long long band_width(int n, const std::vector<int> &pos, const std::vector<int> &Ic, const std::vector<int> &J) {
     long long kd = 0;
-    for (int i = 0; i < n; i++)
-        for (int e = Ic[i]; e < Ic[(size_t)i + 1]; e++) kd = std::max(kd, std::llabs((long long)pos[i] - pos[J[e]]));
+    std::mutex mu;
+    mdz_host_parallel(n, 20000, [&](long long i0, long long i1) {
+        long long k = 0;
+        for (long long i = i0; i < i1; i++)
+            for (int e = Ic[(size_t)i]; e < Ic[(size_t)i + 1]; e++)
+                k = std::max(k, std::llabs((long long)pos[(size_t)i] - pos[(size_t)J[(size_t)e]]));
+        std::lock_guard<std::mutex> g(mu);
+        kd = std::max(kd, k);
+    });
     return kd;
 }
 
@@ -704,9 +555,9 @@ static int check_pattern(const SolverPattern &p, int nrow, int ncol, const char 
     return MDZ_OK;
 }
 
-int mdz_solver_order(MdzSolver *S, int Nx, int Nz, int nu, int np, const int *mom_node, const SolverPattern &A,
-                     const SolverPattern &B, const SolverPattern &C, const SolverPattern &AJ, const SolverPattern &BJ,
-                     int pc_type, int nb) {
+static int order_system(MdzSolver *S, int Nx, int Nz, int nu, int np, const int *mom_node, const SolverPattern &A,
+                        const SolverPattern &B, const SolverPattern &C, const SolverPattern &AJ,
+                        const SolverPattern &BJ, int pc_type, int nb) {
     if (pc_type != 0 && pc_type != 1) return sv_err(MDZ_EUNSUPPORTED, "pc_type = %d", pc_type);
     if (!S || nu < 1 || np < 1 || !mom_node) return sv_err(MDZ_EINVAL, "solver ordering: bad arguments");
     int rc;
@@ -752,14 +603,11 @@ int mdz_solver_order(MdzSolver *S, int Nx, int Nz, int nu, int np, const int *mo
     band_order(Nx, Nz, nu, mom_node, true, px);
     band_order(Nx, Nz, nu, mom_node, false, pz);
     const long long kx = band_width(nu, px, tsI, tsJ), kz = band_width(nu, pz, tsI, tsJ);
-    std::vector<int> &pos = kx <= kz ? px : pz;
     const long long kd = std::max(1LL, std::min(kx, kz));
     if (nb <= 0) nb = SV_NB_DEFAULT;
     if (nb < 64 || nb % 64) return sv_err(MDZ_EINVAL, "solver block size %d (a multiple of 64)", nb);
-    if (kd + nb >= (1LL << 30)) return sv_err(MDZ_EUNSUPPORTED, "solver band width %lld", kd);
-    std::vector<int> eq(nu);
-    for (int i = 0; i < nu; i++) eq[pos[i]] = i;
-    if ((rc = upload_ints(&S->pos, pos)) || (rc = upload_ints(&S->eq, eq)) || (rc = upload_ints(&S->ts_Ic, tsI)) ||
+    S->ordered = false;
+    if ((rc = mdz_factor_analyse(S->fac, Nx, Nz, nu, mom_node, tsI, tsJ)) || (rc = upload_ints(&S->ts_Ic, tsI)) ||
         (rc = upload_ints(&S->ts_J, tsJ)) || (rc = upload_ints(&S->js_Ic, jsI)) || (rc = upload_ints(&S->js_J, jsJ)) ||
         (rc = upload_ints(&S->tr_Ic, trI)) || (rc = upload_ints(&S->tr_J, trJ)) || (rc = upload_ints(&S->tr_src, trS)))
         return rc;
@@ -775,30 +623,24 @@ int mdz_solver_order(MdzSolver *S, int Nx, int Nz, int nu, int np, const int *mo
     S->nequ = nequ;
     S->kd = (int)kd;
     S->nb = nb;
-    S->ldab = kd + nb;
-    S->nblk = mdz_div_up_sv(nu, nb);
+    S->ordered = true;
     return MDZ_OK;
+}
+
+int mdz_solver_order(MdzSolver *S, int Nx, int Nz, int nu, int np, const int *mom_node, const SolverPattern &A,
+                     const SolverPattern &B, const SolverPattern &C, const SolverPattern &AJ, const SolverPattern &BJ,
+                     int pc_type, int nb) {
+    try {
+        return order_system(S, Nx, Nz, nu, np, mom_node, A, B, C, AJ, BJ, pc_type, nb);
+    } catch (const std::exception &e) {
+        return sv_err(MDZ_ENOMEM, "solver ordering: %s", e.what());
+    }
 }
 
 static int ensure_buffers(MdzSolver *S) {
     const size_t n = S->n, np = S->np > 0 ? S->np : 1;
-    const size_t ab_len = (size_t)S->ldab * n, linv_len = (size_t)S->nblk * S->nb * S->nb;
-    if (S->ab_len != ab_len) {
-        hipFree(S->ab); S->ab = nullptr; S->ab_len = 0;
-        SVHIP(hipMalloc((void **)&S->ab, ab_len * sizeof(double)));
-        S->ab_len = ab_len;
-    }
-    if (S->linv_len != linv_len) {
-        hipFree(S->linv); S->linv = nullptr; S->linv_len = 0;
-        SVHIP(hipMalloc((void **)&S->linv, linv_len * sizeof(double)));
-        S->linv_len = linv_len;
-        hipFree(S->info); S->info = nullptr;
-        /* potrf status per factor step (at most nblk (nb / 64 + 1)), then trtri status per block */
-        S->info_len = (size_t)S->nblk * (S->nb / 64 + 1) + S->nblk;
-        SVHIP(hipMalloc((void **)&S->info, S->info_len * sizeof(int)));
-    }
     const size_t ldv = (n + 63) & ~(size_t)63, ldp = (np + 63) & ~(size_t)63;
-    const size_t work_len = 9 * ldv + 3 * ldp + 2 * SV_RESTART * ldv;
+    const size_t work_len = 5 * ldv + 3 * ldp + 2 * SV_RESTART * ldv;
     if (S->work_len != work_len) {
         hipFree(S->work); S->work = nullptr; S->work_len = 0;
         SVHIP(hipMalloc((void **)&S->work, work_len * sizeof(double)));
@@ -806,9 +648,8 @@ static int ensure_buffers(MdzSolver *S) {
     }
     double *w = S->work;
     S->ldv = ldv;
-    S->udum = w; S->f = w + ldv; S->sv = w + 2 * ldv; S->v = w + 3 * ldv; S->r = w + 4 * ldv; S->y = w + 5 * ldv;
-    S->t = w + 6 * ldv; S->xb = w + 7 * ldv; S->fu = w + 8 * ldv;
-    S->pdum = w + 9 * ldv; S->fp = S->pdum + ldp; S->tc = S->fp + ldp;
+    S->udum = w; S->f = w + ldv; S->sv = w + 2 * ldv; S->v = w + 3 * ldv; S->fu = w + 4 * ldv;
+    S->pdum = w + 5 * ldv; S->fp = S->pdum + ldp; S->tc = S->fp + ldp;
     S->VV = S->tc + ldp; S->SS = S->VV + SV_RESTART * ldv;
     return MDZ_OK;
 }
@@ -823,10 +664,8 @@ static int read_scalars(MdzSolver *S, int first, int count) {
 }
 
 static int factorise(MdzSolver *S, const SolverInput &in) {
-    const int n = S->n, nb = S->nb, kd = S->kd;
-    const long long ldab = S->ldab;
+    const int n = S->n;
     hipStream_t s = S->s;
-    SVHIP(hipMemsetAsync(S->ab, 0, S->ab_len * sizeof(double), s));
     const dim3 gN(mdz_div_up_sv(n, SV_BLK)), blk(SV_BLK);
     const bool sym = S->pc_type == 1;
     hipLaunchKernelGGL(k_schur_values, gN, blk, 0, s, n, (const int *)S->ts_Ic, (const int *)S->ts_J,
@@ -835,81 +674,17 @@ static int factorise(MdzSolver *S, const SolverInput &in) {
     hipLaunchKernelGGL(k_schur_values, gN, blk, 0, s, n, (const int *)S->js_Ic, (const int *)S->js_J, view(in.AJ), 1.0,
                        (const int *)nullptr, (const int *)nullptr, (const int *)nullptr, view(in.BJ), view(in.C),
                        in.Dpen, S->js_val);
-    hipLaunchKernelGGL(k_band_fill, gN, blk, 0, s, n, (const int *)S->pos, (const int *)S->ts_Ic,
-                       (const int *)S->ts_J, (const double *)S->ts_val, S->ab, ldab);
     SVHIP(hipGetLastError());
-    const double one = 1.0, mone = -1.0;
-    const int ld = (int)(ldab - 1);
-    /* factor steps of nbf columns (any nbf <= nb keeps every window inside
-     * the band storage); the diagonal blocks of the solves are nb wide */
-    const int nbf = std::min(SV_NBF, nb);
-    const int nsteps = mdz_div_up_sv(n, nbf);
-    for (int b = 0; b < nsteps; b++) {
-        const long long i0 = (long long)b * nbf;
-        const int ib = (int)std::min((long long)nbf, n - i0);
-        const int m = (int)std::min((long long)kd, n - i0 - ib);
-        double *d = S->ab + i0 * ldab;
-        SVBLAS(rocsolver_dpotrf(S->h, rocblas_fill_lower, ib, d, ld, S->info + b));
-        if (m > 0) {
-            SVBLAS(rocblas_dtrsm(S->h, rocblas_side_right, rocblas_fill_lower, rocblas_operation_transpose,
-                                 rocblas_diagonal_non_unit, m, ib, &one, d, ld, d + ib, ld));
-            SVBLAS(rocblas_dsyrk(S->h, rocblas_fill_lower, rocblas_operation_none, m, ib, &mone, d + ib, ld, &one,
-                                 d + (long long)ib * ldab, ld));
-        }
-    }
-    hipLaunchKernelGGL(k_diag_blocks, dim3(S->nblk), dim3(SV_BLK), 0, s, (const double *)S->ab, ldab, n, nb, S->linv);
-    SVHIP(hipGetLastError());
-    SVBLAS(rocsolver_dtrtri_strided_batched(S->h, rocblas_fill_lower, rocblas_diagonal_non_unit, nb, S->linv, nb,
-                                            (rocblas_stride)nb * nb, S->info + S->nblk * (size_t)(nb / nbf + 1),
-                                            S->nblk));
-    std::vector<int> inf((size_t)nsteps + S->nblk);
-    SVHIP(hipMemcpyAsync(inf.data(), S->info, (size_t)nsteps * sizeof(int), hipMemcpyDeviceToHost, s));
-    SVHIP(hipMemcpyAsync(inf.data() + nsteps, S->info + S->nblk * (size_t)(nb / nbf + 1), S->nblk * sizeof(int),
-                         hipMemcpyDeviceToHost, s));
-    SVHIP(hipStreamSynchronize(s));
-    for (int b = 0; b < nsteps; b++)
-        if (inf[b] != 0)
-            return sv_err(MDZ_ESOLVE, "Cholesky factor of Jts: leading minor %d of block %d is not positive definite",
-                          inf[b], b);
-    for (int b = 0; b < S->nblk; b++)
-        if (inf[nsteps + b] != 0) return sv_err(MDZ_ESOLVE, "inverse of diagonal block %d is singular", b);
+    int bad = -1;
+    const int rc = mdz_factor_numeric(S->fac, S->ts_Ic, S->ts_J, S->ts_val, &bad);
+    if (rc) return rc;
+    if (bad >= 0)
+        return sv_err(MDZ_ESOLVE, "Cholesky factor of Jts: the pivot of momentum equation %d is not positive", bad);
     return MDZ_OK;
 }
 
-/* sv = Jts^-1 f through the factor (band order in between) */
-static void precondition(MdzSolver *S, const double *f, double *out) {
-    const int n = S->n, nb = S->nb, kd = S->kd;
-    const long long ldab = S->ldab;
-    hipStream_t s = S->s;
-    hipLaunchKernelGGL(k_gather, dim3(mdz_div_up_sv(n, SV_BLK)), dim3(SV_BLK), 0, s, n, (const int *)S->eq, f, S->r);
-    for (int b = 0; b < S->nblk; b++) {
-        const long long i0 = (long long)b * nb;
-        const int ib = (int)std::min((long long)nb, n - i0);
-        const int m = (int)std::min((long long)kd, n - i0 - ib);
-        const double *L = S->linv + (size_t)b * nb * nb;
-        hipLaunchKernelGGL(k_fwd_diag, dim3(mdz_div_up_sv(ib, TS_R)), dim3(SV_BLK), 0, s, L, nb, ib,
-                           (const double *)(S->r + i0), S->y + i0);
-        if (m > 0)
-            hipLaunchKernelGGL(k_fwd_panel, dim3(mdz_div_up_sv(m, TS_R)), dim3(SV_BLK), 0, s, (const double *)S->ab, ldab,
-                               kd, i0, ib, m, (const double *)S->y, S->r);
-    }
-    for (int b = S->nblk - 1; b >= 0; b--) {
-        const long long i0 = (long long)b * nb;
-        const int ib = (int)std::min((long long)nb, n - i0);
-        const int m = (int)std::min((long long)kd, n - i0 - ib);
-        const double *L = S->linv + (size_t)b * nb * nb;
-        hipLaunchKernelGGL(k_bwd_panel, dim3(mdz_div_up_sv(ib, 4)), dim3(SV_BLK), 0, s, (const double *)S->ab, ldab, kd,
-                           i0, ib, m, (const double *)S->xb, (const double *)S->y, S->t);
-        hipLaunchKernelGGL(k_bwd_diag, dim3(mdz_div_up_sv(ib, 4)), dim3(SV_BLK), 0, s, L, nb, ib, i0,
-                           (const double *)S->t, S->xb);
-    }
-    hipLaunchKernelGGL(k_scatter, dim3(mdz_div_up_sv(n, SV_BLK)), dim3(SV_BLK), 0, s, n, (const int *)S->eq,
-                       (const double *)S->xb, out);
-}
-
-/* sv = Jts^-1 f as one graph launch: about 4 n / nb small kernels, whose
- * launch cost would otherwise exceed their run time; captured again when
- * the factor's buffers or dimensions change */
+/* sv = Jts^-1 f as one graph launch (two launches per level of the
+ * elimination tree); captured again when the factor's layout changes */
 static int run_precondition(MdzSolver *S) {
     /* MDZ_SOLVER_GRAPH=0 launches the same kernels one by one (for tracing
      * tools that do not follow graph launches) */
@@ -918,25 +693,25 @@ static int run_precondition(MdzSolver *S) {
         return e && e[0] == '0' ? 0 : 1;
     }();
     if (!use_graph) {
-        precondition(S, S->f, S->sv);
+        mdz_factor_apply(S->fac, S->f, S->sv);
         return MDZ_OK;
     }
-    const void *key[6] = {S->ab, S->linv, S->r, S->f, S->sv, S->eq};
-    const long long dims[3] = {S->n, S->nb, S->kd};
-    if (!S->pc_exec || memcmp(key, S->pc_key, sizeof(key)) || memcmp(dims, S->pc_dims, sizeof(dims))) {
+    const void *key[2] = {S->f, S->sv};
+    const unsigned long long version = mdz_factor_version(S->fac);
+    if (!S->pc_exec || memcmp(key, S->pc_key, sizeof(key)) || version != S->pc_version) {
         if (S->pc_exec) hipGraphExecDestroy(S->pc_exec);
         if (S->pc_graph) hipGraphDestroy(S->pc_graph);
         S->pc_exec = nullptr;
         S->pc_graph = nullptr;
         SVHIP(hipStreamBeginCapture(S->s, hipStreamCaptureModeThreadLocal));
-        precondition(S, S->f, S->sv);
+        mdz_factor_apply(S->fac, S->f, S->sv);
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamEndCapture(S->s, &g);
         if (e != hipSuccess) return sv_err(MDZ_EHIP, "preconditioner capture: %s", hipGetErrorString(e));
         S->pc_graph = g;
         SVHIP(hipGraphInstantiate(&S->pc_exec, g, nullptr, nullptr, 0));
         memcpy(S->pc_key, key, sizeof(key));
-        memcpy(S->pc_dims, dims, sizeof(dims));
+        S->pc_version = version;
     }
     SVHIP(hipGraphLaunch(S->pc_exec, S->s));
     return MDZ_OK;
@@ -945,7 +720,9 @@ static int run_precondition(MdzSolver *S) {
 /* out = Js x, or b - Js x */
 static void apply_js(MdzSolver *S, const double *x, const double *b, double *out) {
     const CsrView js{S->js_Ic, S->js_J, S->js_val};
-    hipLaunchKernelGGL(k_csr_apply, dim3(mdz_div_up_sv(S->n, SV_BLK)), dim3(SV_BLK), 0, S->s, S->n, js, x, b, out);
+    const dim3 grid(mdz_div_up_sv(S->n, SV_BLK)), blk(SV_BLK);
+    if (b) hipLaunchKernelGGL(k_csr_residual, grid, blk, 0, S->s, S->n, js, x, b, out);
+    else hipLaunchKernelGGL(k_csr_apply, grid, blk, 0, S->s, S->n, js, x, out);
 }
 
 static int final_sum(MdzSolver *S, int nq, int max_mask, int slot) {
@@ -1024,7 +801,7 @@ static int residuals(MdzSolver *S, const SolverInput &in, const double *du, cons
 }
 
 int mdz_solver_solve(MdzSolver *S, const SolverInput &in, double *du, double *dp, mdz_solve_info *info) {
-    if (!S || !S->pos) return sv_err(MDZ_EINVAL, "solver: no ordering");
+    if (!S || !S->ordered) return sv_err(MDZ_EINVAL, "solver: no ordering");
     if (in.nu != S->n || in.np != S->np) return sv_err(MDZ_EINVAL, "solver: ordering of another system");
     if (in.pc_type != S->pc_type)
         return sv_err(MDZ_EINVAL, "solver: ordering built for pc_type %d, solve asks for %d", S->pc_type, in.pc_type);
