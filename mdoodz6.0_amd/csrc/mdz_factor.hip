@@ -27,6 +27,7 @@
  * other in a solve): factor 703 -> 6.5 ms, a GCR direction 5.6 -> 0.55 ms;
  * at 257 x 129 cells 168 -> 3 ms and 1.17 -> 0.18 ms.
  */
+#include <limits.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -60,128 +61,144 @@ __device__ __forceinline__ double nd_lane(double x, int l) {
 
 /* LDS of the tile kernels: two 64 x 64 operands (column k of row r at
  * k 64 + (r ^ 16 (k & 1)): the two columns a half wave reads lie in
- * different banks), or the diagonal tile (65 doubles a column) and its
- * inverse */
-#define ND_LDS (ND_T * (ND_T + 1) + ND_T * ND_T)
+ * different banks), or the diagonal tile (65 doubles a column), its inverse
+ * and the column buffers of its factorisation */
+#define ND_DIAG (ND_T * (ND_T + 1))
+#define ND_LDS (ND_DIAG + ND_T * ND_T + 640)
 __device__ __forceinline__ int nd_sw(int k, int r) { return k * ND_T + (r ^ ((k & 1) << 4)); }
 
-/* Cholesky factor of the w x w lower triangle in S and its inverse, written
- * to out (64 x 64 column-major, identity beyond w); called by a whole
- * workgroup of 256 after a barrier.  16-column steps: wave 0 factors the
- * diagonal block and inverts it in registers (lane exchange by readlane),
- * the workgroup forms the rows below and the trailing update. */
-__device__ __forceinline__ void nd_potrf(double *S, double *V, int w, double *__restrict__ out, int pos0, int *bad) {
-    const int tid = threadIdx.x;
-    const int nb = (w + 15) >> 4, R = nb << 4;
-    for (int e = tid; e < ND_T * ND_T; e += ND_BLK) V[e] = (e & 63) == (e >> 6) ? 1.0 : 0.0;
-    for (int e = tid; e < R * R; e += ND_BLK) {
-        const int c = e / R, r = e - c * R;
-        if (r >= w || c >= w) S[c * 65 + r] = r == c ? 1.0 : 0.0;
+/* 1 / p and 1 / sqrt(p) of a positive normal p: the hardware's estimate and
+ * two Newton steps (a divide or a square root is a chain twice as long) */
+__device__ __forceinline__ double nd_rcp(double p) {
+    double y = __builtin_amdgcn_rcp(p);
+#pragma unroll
+    for (int i = 0; i < 2; i++) y = __builtin_fma(y, __builtin_fma(-p, y, 1.0), y);
+    return y;
+}
+__device__ __forceinline__ double nd_rsqrt(double p) {
+    double y = __builtin_amdgcn_rsq(p);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const double e = __builtin_fma(-p * y, y, 1.0);
+        y = __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+    }
+    return y;
+}
+
+/* Inverse of the Cholesky factor of the w x w lower triangle in S (LDS, 65
+ * doubles a column; overwritten), written to out (64 x 64 column-major,
+ * identity beyond w) and, where T is not null, to its place in a front;
+ * called by a whole workgroup of 256 after a barrier.  Bound by the chain of
+ * w columns.
+ *
+ * Elimination: lane = row, wave q holds columns 16 q .. 16 q + 15 in
+ * registers.  Four columns a step: their owner eliminates among them
+ * (pivots by readlane; unit-lower multipliers, no square root), passes them
+ * through LDS, and after one barrier the waves take four rank-one terms off
+ * the columns to the right.  The loop is rolled (straight-line steps run at
+ * the pace of cold instruction fetches): the owner moves its columns down by
+ * four, so that the step's are always the first four.
+ *
+ * Inverse: wave q inverts diagonal block q (16 x 16, lane = column), then a
+ * barrier per block row and V(i, j) = -V(i, i) sum_k L(i, k) V(k, j) on the
+ * matrix instructions, whose result registers are the second product's
+ * operand as they are; rows are scaled by 1 / sqrt(pivot) on the way out.
+ *
+ * Measured for 64 columns: 22 us (with its launch); 33 with the inverse eliminated
+ * along by readlane, 50 for 16-column blocks through LDS with six barriers
+ * each. */
+__device__ __forceinline__ void nd_potrf(double *S, int w, double *__restrict__ out, double *T, int ldt, int pos0,
+                                         int *bad) {
+    double *V = S + ND_DIAG, *buf = V + ND_T * ND_T;
+    double *piv = buf; /* 64 pivots; then two buffers of four columns and four reciprocal pivots */
+    const int r = threadIdx.x & 63, q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nb = (w + 15) >> 4, W = nb << 4;
+    double a[16];
+    int fail = INT_MAX;
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        const int c = 16 * q + k;
+        V[c * ND_T + r] = r == c ? 1.0 : 0.0;
+        a[k] = r < w && c <= r ? S[c * 65 + r] : c < w ? 0.0 : r == c ? 1.0 : 0.0;
+    }
+#pragma unroll 1
+    for (int j0 = 0; j0 < W; j0 += 4) {
+        const int ow = j0 >> 4;
+        double *B = buf + 64 + (j0 & 4) * 72;
+        if (q == ow) { /* (its own columns of S: the other waves read theirs only) */
+            double y[4];
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                double p = nd_lane(a[t], j0 + t);
+                fail = p > 0.0 ? fail : min(fail, j0 + t);
+                p = p > 0.0 ? p : 1.0;
+                y[t] = nd_rcp(p);
+                const double f = r > j0 + t ? a[t] * y[t] : 0.0;
+                if (r == 0) piv[j0 + t] = p;
+#pragma unroll
+                for (int u = t + 1; u < 4; u++) a[u] = __builtin_fma(-f, nd_lane(a[t], j0 + u), a[u]);
+                S[(j0 + t) * 65 + r] = f;
+                B[t * 64 + r] = a[t];
+            }
+#pragma unroll
+            for (int k = 0; k < 12; k++) a[k] = a[k + 4];
+        }
+        __syncthreads();
+        if (q >= ow) { /* (the owner's last columns are past its sixteen: never used) */
+            const double *Bc = B + (q == ow ? j0 + 4 : 16 * q);
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const double f = S[(j0 + t) * 65 + r];
+                double b[16];
+#pragma unroll
+                for (int k = 0; k < 16; k++) b[k] = Bc[t * 64 + k];
+                __builtin_amdgcn_sched_barrier(0); /* all reads in flight before the first use */
+#pragma unroll
+                for (int k = 0; k < 16; k++) a[k] = __builtin_fma(-f, b[k], a[k]);
+            }
+        }
+    }
+    if (fail < w && r == 0) atomicMin(bad, pos0 + fail);
+    __syncthreads();
+    const int li = r & 15, lk = r >> 4;
+    if (q < nb) {
+        double x[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            double t = li == i ? 1.0 : 0.0;
+#pragma unroll
+            for (int k = 0; k < i; k++) t = __builtin_fma(-S[(16 * q + k) * 65 + 16 * q + i], x[k], t);
+            x[i] = t;
+        }
+        if (lk == 0)
+#pragma unroll
+            for (int i = 0; i < 16; i++) V[(16 * q + li) * ND_T + 16 * q + i] = x[i];
+    }
+    for (int ib = 1; ib < nb; ib++) {
+        __syncthreads();
+        if (q >= ib) continue;
+        nd_d4 g = {}, z = {};
+        for (int kb = q; kb < ib; kb++)
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                const int k = 16 * kb + 4 * ks + lk;
+                g = __builtin_amdgcn_mfma_f64_16x16x4f64(S[k * 65 + 16 * ib + li], V[(16 * q + li) * ND_T + k], g, 0, 0, 0);
+            }
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++)
+            z = __builtin_amdgcn_mfma_f64_16x16x4f64(V[(16 * ib + 4 * ks + lk) * ND_T + 16 * ib + li], g[ks], z, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 4; v++) V[(16 * q + li) * ND_T + 16 * ib + 4 * v + lk] = -z[v];
     }
     __syncthreads();
-    for (int kb = 0; kb < nb; kb++) {
-        const int o = kb << 4;
-        if (tid < 64) {
-            const int l = tid & 15;
-            double a[16], ri[16], x[16];
+    const double rs = r < w ? nd_rsqrt(piv[r]) : 1.0;
 #pragma unroll
-            for (int c = 0; c < 16; c++) a[c] = S[(o + c) * 65 + o + l];
-#pragma unroll
-            for (int c = 0; c < 16; c++) {
-                double p = nd_lane(a[c], c);
-                if (!(p > 0.0)) {
-                    if (tid == 0) atomicMin(bad, pos0 + o + c);
-                    p = 1.0;
-                }
-                const double d = sqrt(p);
-                ri[c] = 1.0 / d;
-                a[c] = l == c ? d : a[c] * ri[c];
-#pragma unroll
-                for (int c2 = c + 1; c2 < 16; c2++) a[c2] -= a[c] * nd_lane(a[c], c2);
-            }
-            /* lane l: column l of the inverse */
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                double t = l == r ? 1.0 : 0.0;
-#pragma unroll
-                for (int k = 0; k < r; k++) t -= nd_lane(a[k], r) * x[k];
-                x[r] = t * ri[r];
-            }
-            if (tid < 16) {
-#pragma unroll
-                for (int c = 0; c < 16; c++)
-                    if (c <= l) S[(o + c) * 65 + o + l] = a[c];
-#pragma unroll
-                for (int r = 0; r < 16; r++) V[(o + l) * ND_T + o + r] = r >= l ? x[r] : 0.0;
-            }
-        }
-        __syncthreads();
-        const int nr = R - o - 16;
-        if (nr > 0) {
-            double g[3];
-#pragma unroll
-            for (int q = 0; q < 3; q++) {
-                const int e = tid + q * ND_BLK;
-                if (e < nr * 16) {
-                    const int c = e / nr, r = o + 16 + e - c * nr;
-                    double t = 0.0;
-                    for (int k = 0; k <= c; k++) t += S[(o + k) * 65 + r] * V[(o + k) * ND_T + o + c];
-                    g[q] = t;
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int q = 0; q < 3; q++) {
-                const int e = tid + q * ND_BLK;
-                if (e < nr * 16) {
-                    const int c = e / nr, r = o + 16 + e - c * nr;
-                    S[(o + c) * 65 + r] = g[q];
-                }
-            }
-            __syncthreads();
-            for (int e = tid; e < nr * nr; e += ND_BLK) {
-                const int cc = e / nr, c = o + 16 + cc, r = o + 16 + e - cc * nr;
-                if (r < c) continue;
-                double t = 0.0;
-#pragma unroll
-                for (int k = 0; k < 16; k++) t += S[(o + k) * 65 + r] * S[(o + k) * 65 + c];
-                S[c * 65 + r] -= t;
-            }
-            __syncthreads();
-        }
+    for (int k = 0; k < 16; k++) {
+        const int c = 16 * q + k;
+        const double x = V[c * ND_T + r] * rs;
+        out[c * ND_T + r] = x;
+        if (T && r < w && c < w) T[(long long)c * ldt + r] = x;
     }
-    /* off-diagonal blocks of the inverse, block row by block row */
-    const int r = tid & 15, c = tid >> 4;
-    for (int ib = 1; ib < nb; ib++) {
-        const int ri0 = ib << 4;
-        double g[3];
-#pragma unroll
-        for (int jb = 0; jb < 3; jb++)
-            if (jb < ib) {
-                double t = 0.0;
-                for (int k = jb << 4; k < ri0; k++) t += S[k * 65 + ri0 + r] * V[((jb << 4) + c) * ND_T + k];
-                g[jb] = t;
-            }
-        __syncthreads();
-#pragma unroll
-        for (int jb = 0; jb < 3; jb++)
-            if (jb < ib) V[((jb << 4) + c) * ND_T + ri0 + r] = g[jb];
-        __syncthreads();
-#pragma unroll
-        for (int jb = 0; jb < 3; jb++)
-            if (jb < ib) {
-                double t = 0.0;
-                for (int k = 0; k <= r; k++)
-                    t += V[(ri0 + k) * ND_T + ri0 + r] * V[((jb << 4) + c) * ND_T + ri0 + k];
-                g[jb] = -t;
-            }
-        __syncthreads();
-#pragma unroll
-        for (int jb = 0; jb < 3; jb++)
-            if (jb < ib) V[((jb << 4) + c) * ND_T + ri0 + r] = g[jb];
-        __syncthreads();
-    }
-    for (int e = tid; e < ND_T * ND_T; e += ND_BLK) out[e] = V[e];
 }
 
 /* rows of a row tile: first row of the front and how many */
@@ -247,7 +264,8 @@ __global__ void __launch_bounds__(ND_BLK) k_nd_scatter(int n, const int *__restr
 __global__ void __launch_bounds__(ND_BLK) k_nd_assemble(const NdTask *__restrict__ task,
                                                         const NdNode *__restrict__ nodes,
                                                         const int *__restrict__ inv, const double *__restrict__ Uc,
-                                                        double *__restrict__ P, double *__restrict__ Linv, int *bad) {
+                                                        double *__restrict__ P, double *__restrict__ Lb,
+                                                        double *__restrict__ Linv, int *bad) {
     __shared__ double sh[ND_LDS];
     const NdTask t = task[blockIdx.x];
     const NdNode N = nodes[t.node];
@@ -265,7 +283,8 @@ __global__ void __launch_bounds__(ND_BLK) k_nd_assemble(const NdTask *__restrict
     }
     if (!first) return;
     __syncthreads();
-    nd_potrf(sh, sh + ND_T * 65, nc, Linv + (size_t)N.lin * (ND_T * ND_T), N.ooff, bad);
+    nd_potrf(sh, nc, Linv + (size_t)N.lin * (ND_T * ND_T), N.np == 1 ? Lb + N.poff : nullptr, N.ld,
+             N.ooff, bad);
 }
 
 /* Panel j of the nodes of a level: task = (row tile, column tile) of the
@@ -322,7 +341,7 @@ __global__ void __launch_bounds__(ND_BLK) k_nd_panel(const NdTask *__restrict__ 
                 for (int ri = 0; ri < 2; ri++)
                     acc[ci][ri] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ci], b[ri], acc[ci][ri], 0, 0, 0);
         }
-        const bool keep = q == 0 && t.a == t.b;
+        const bool keep = q == 0 && t.a == t.b && N.np > 1;
 #pragma unroll
         for (int ci = 0; ci < 2; ci++)
 #pragma unroll
@@ -336,6 +355,34 @@ __global__ void __launch_bounds__(ND_BLK) k_nd_panel(const NdTask *__restrict__ 
                 }
     }
     __syncthreads();
+    if (N.np == 1 && t.a == t.b) {
+        /* a front of one panel: its rows of T = L21 L11^-1 at once */
+        nd_d4 tw[2][2] = {};
+#pragma unroll 4
+        for (int ks = 0; ks < w4; ks += 4) {
+            const int k = ks + lk;
+            double a[2], b[2];
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                a[q] = Vj[(cq + 16 * q + li) * ND_T + k];
+                b[q] = Lr[nd_sw(k, rq + 16 * q + li)];
+            }
+#pragma unroll
+            for (int ci = 0; ci < 2; ci++)
+#pragma unroll
+                for (int ri = 0; ri < 2; ri++)
+                    tw[ci][ri] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ci], b[ri], tw[ci][ri], 0, 0, 0);
+        }
+#pragma unroll
+        for (int ci = 0; ci < 2; ci++)
+#pragma unroll
+            for (int ri = 0; ri < 2; ri++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int c = cq + 16 * ci + 4 * v + lk, r = rq + 16 * ri + li;
+                    if (c < w && r < tnr) Lb[N.poff + (long long)c * N.ld + tr0 + r] = tw[ci][ri][v];
+                }
+    }
     nd_d4 acc[2][2] = {};
 #pragma unroll 4
     for (int ks = 0; ks < w4; ks += 4) {
@@ -374,12 +421,13 @@ __global__ void __launch_bounds__(ND_BLK) k_nd_panel(const NdTask *__restrict__ 
             }
     if (!next) return;
     __syncthreads();
-    nd_potrf(sh, sh + ND_T * 65, tnc, Linv + ((size_t)N.lin + j + 1) * (ND_T * ND_T), N.ooff + tc0, bad);
+    nd_potrf(sh, tnc, Linv + ((size_t)N.lin + j + 1) * (ND_T * ND_T), nullptr, 0, N.ooff + tc0, bad);
 }
 
-/* T = [L11^-1; L21 L11^-1] over the panel storage, column tiles from the
- * last to the first (all nodes of all levels at once): task = (column tile
- * j, row tile); T(:, j) = (E - sum_{i > j} T(:, i) L(i, j)) Linv_j with E
+/* T = [L11^-1; L21 L11^-1] of the fronts of several panels, over the panel
+ * storage (a front of one panel has its T in Lb already), column tiles from
+ * the last to the first (all nodes of all levels at once): task = (column
+ * tile j, row tile); T(:, j) = (E - sum_{i > j} T(:, i) L(i, j)) Linv_j with E
  * the rows of L21, and T(j, j) = Linv_j. */
 __global__ void __launch_bounds__(ND_BLK) k_nd_invert(const NdTask *__restrict__ task,
                                                       const NdNode *__restrict__ nodes, double *P,
@@ -496,7 +544,8 @@ template <int RT>
 __global__ void __launch_bounds__(ND_BLK) k_nd_forward(const NdTask *__restrict__ task,
                                                        const NdNode *__restrict__ nodes, const int *__restrict__ inv,
                                                        const int *__restrict__ eq, const double *__restrict__ P,
-                                                       const double *__restrict__ f, double *__restrict__ y,
+                                                       const double *__restrict__ Lb, const double *__restrict__ f,
+                                                       double *__restrict__ y,
                                                        double *g) {
     constexpr int CG = ND_BLK / RT;
     __shared__ double rs[ND_CH];
@@ -505,7 +554,7 @@ __global__ void __launch_bounds__(ND_BLK) k_nd_forward(const NdTask *__restrict_
     const NdNode N = nodes[t.node];
     const int lr = threadIdx.x % RT, cg = threadIdx.x / RT;
     const int m = N.s + N.b, row0 = t.a * RT, row = row0 + lr;
-    const double *Tr = P + N.poff + (row < m ? row : 0);
+    const double *Tr = (N.np > 1 ? P : Lb) + N.poff + (row < m ? row : 0);
     /* own rows end at the diagonal tile of the last row */
     const int last = min(row0 + RT, m) - 1;
     const int cend = last < N.s ? min(N.s, (last / ND_T + 1) * ND_T) : N.s;
@@ -538,7 +587,8 @@ template <int CT>
 __global__ void __launch_bounds__(ND_BLK) k_nd_backward(const NdTask *__restrict__ task,
                                                         const NdNode *__restrict__ nodes,
                                                         const int *__restrict__ blist, const int *__restrict__ eq,
-                                                        const double *__restrict__ P, const double *__restrict__ y,
+                                                        const double *__restrict__ P,
+                                                        const double *__restrict__ Lb, const double *__restrict__ y,
                                                         double *x, double *__restrict__ out) {
     constexpr int NC = CT / 16;
     __shared__ double vs[ND_CH];
@@ -560,7 +610,7 @@ __global__ void __launch_bounds__(ND_BLK) k_nd_backward(const NdTask *__restrict
         for (int q = 0; q < NC; q++) {
             const int c = c0 + cl + 16 * q;
             if (c < N.s) {
-                const double *Tc = P + N.poff + (long long)c * N.ld;
+                const double *Tc = (N.np > 1 ? P : Lb) + N.poff + (long long)c * N.ld;
                 const int rs = max(rb, (c / ND_T) * ND_T);
                 double a = 0.0;
 #pragma unroll 8
@@ -680,7 +730,7 @@ int mdz_factor_numeric(MdzFactor *F, const int *Ic, const int *J, const double *
         if (L.assemble.count)
             hipLaunchKernelGGL(k_nd_assemble, dim3(L.assemble.count), dim3(ND_BLK), 0, s,
                                (const NdTask *)F->tasks.p + L.assemble.first, nodes, (const int *)F->inv.p,
-                               (const double *)Uc, F->P.p, F->Linv.p, F->bad.p);
+                               (const double *)Uc, F->P.p, F->Lb.p, F->Linv.p, F->bad.p);
         for (size_t j = 0; j < L.panel.size(); j++)
             if (L.panel[j].count)
                 hipLaunchKernelGGL(k_nd_panel, dim3(L.panel[j].count), dim3(ND_BLK), 0, s,
@@ -708,7 +758,7 @@ void mdz_factor_apply(MdzFactor *F, const double *f, double *x) {
         const dim3 grid(L.forward.count), blk(ND_BLK);
 #define FWD(RT)                                                                                                   \
     hipLaunchKernelGGL((k_nd_forward<RT>), grid, blk, 0, s, t, nodes, (const int *)F->inv.p, (const int *)F->eq.p, \
-                       (const double *)F->P.p, f, F->y.p, F->g.p)
+                       (const double *)F->P.p, (const double *)F->Lb.p, f, F->y.p, F->g.p)
         if (L.rt == 64) FWD(64);
         else if (L.rt == 32) FWD(32);
         else FWD(16);
@@ -721,7 +771,7 @@ void mdz_factor_apply(MdzFactor *F, const double *f, double *x) {
         const dim3 grid(L.backward.count), blk(ND_BLK);
 #define BWD(CT)                                                                                                      \
     hipLaunchKernelGGL((k_nd_backward<CT>), grid, blk, 0, s, t, nodes, (const int *)F->blist.p, (const int *)F->eq.p, \
-                       (const double *)F->P.p, (const double *)F->y.p, F->x.p, x)
+                       (const double *)F->P.p, (const double *)F->Lb.p, (const double *)F->y.p, F->x.p, x)
         if (L.ct == 64) BWD(64);
         else if (L.ct == 32) BWD(32);
         else BWD(16);

@@ -396,12 +396,12 @@ static int nd_plan(NdPlan &plan, int Nx, int Nz, int n, const int *mom_node, con
             for (int c = 0; c < N[q].s; c += L.ct) task.push_back({q, c / L.ct, 0});
         L.backward = end(first);
     }
-    for (int p = 0; p < npmax; p++) {
+    for (int p = 0; p < (npmax > 1 ? npmax : 0); p++) { /* (fronts of one panel need none) */
         const int first = (int)task.size();
         for (int q = 0; q < nt; q++) {
             const NdNode &k = N[q];
             const int j = k.np - 1 - p, tiles = k.np + (k.b + ND_T - 1) / ND_T;
-            if (j < 0) continue;
+            if (j < 0 || k.np < 2) continue;
             for (int r = j; r < tiles; r++) task.push_back({q, j, r});
         }
         plan.invert.push_back({first, (int)task.size() - first});
