@@ -22,9 +22,11 @@ int mdz_factor_analyse(MdzFactor *F, int Nx, int Nz, int n, const int *mom_node,
                        const std::vector<int> &J);
 
 /* Numeric factor of the symmetric matrix whose lower triangle (column <=
- * row, equation order) is that of (Ic, J, val) on the device; *bad = an
+ * row, equation order) is that of the pattern (Ic, J), given on the device in
+ * slices of 64 rows (entry e of row i at base[i / 64] + 64 e + i % 64, row
+ * lengths from Ic); *bad = an
  * equation whose pivot is not positive, or -1.  Synchronises. */
-int mdz_factor_numeric(MdzFactor *F, const int *Ic, const int *J, const double *val, int *bad);
+int mdz_factor_numeric(MdzFactor *F, const int *base, const int *Ic, const int *J, const double *val, int *bad);
 
 /* x = (L L^T)^-1 f in equation order, on device vectors; enqueues only */
 void mdz_factor_apply(MdzFactor *F, const double *f, double *x);

@@ -231,15 +231,16 @@ __device__ __forceinline__ double nd_children(const NdNode *__restrict__ nodes, 
 
 /* matrix entries to their places in the panels: one row of the lower
  * triangle per thread (one writer per element) */
-__global__ void __launch_bounds__(ND_BLK) k_nd_scatter(int n, const int *__restrict__ Ic, const int *__restrict__ J,
-                                                       const double *__restrict__ val, const int *__restrict__ pos,
+__global__ void __launch_bounds__(ND_BLK) k_nd_scatter(int n, const int *__restrict__ base, const int *__restrict__ Ic,
+                                                       const int *__restrict__ J, const double *__restrict__ val, const int *__restrict__ pos,
                                                        const int *__restrict__ node_of,
                                                        const NdNode *__restrict__ nodes,
                                                        const int *__restrict__ blist, double *__restrict__ P) {
     const int i = blockIdx.x * ND_BLK + threadIdx.x;
     if (i >= n) return;
-    const int pi = pos[i];
-    for (int e = Ic[i]; e < Ic[i + 1]; e++) {
+    const int pi = pos[i], len = Ic[i + 1] - Ic[i];
+    for (int q = 0; q < len; q++) {
+        const int e = base[i >> 6] + 64 * q + (i & 63);
         const int j = J[e];
         if (j > i) continue;
         const int pj = pos[j], lo = min(pi, pj), hi = max(pi, pj);
@@ -715,14 +716,14 @@ int mdz_factor_analyse(MdzFactor *F, int Nx, int Nz, int n, const int *mom_node,
     return MDZ_OK;
 }
 
-int mdz_factor_numeric(MdzFactor *F, const int *Ic, const int *J, const double *val, int *bad) {
+int mdz_factor_numeric(MdzFactor *F, const int *base, const int *Ic, const int *J, const double *val, int *bad) {
     if (!F || F->n < 1) return mdz_error(MDZ_EINVAL, "factor: not analysed");
     hipStream_t s = F->s;
     const NdNode *nodes = F->nodes.p;
     const int none = INT_MAX;
     FCHK(hipMemcpyAsync(F->bad.p, &none, sizeof(int), hipMemcpyHostToDevice, s));
     FCHK(hipMemsetAsync(F->P.p, 0, F->plan.panel_len * sizeof(double), s));
-    hipLaunchKernelGGL(k_nd_scatter, dim3((F->n + ND_BLK - 1) / ND_BLK), dim3(ND_BLK), 0, s, F->n, Ic, J, val,
+    hipLaunchKernelGGL(k_nd_scatter, dim3((F->n + ND_BLK - 1) / ND_BLK), dim3(ND_BLK), 0, s, F->n, base, Ic, J, val,
                        (const int *)F->pos.p, (const int *)F->node_of.p, nodes, (const int *)F->blist.p, F->P.p);
     for (size_t lv = 0; lv < F->plan.level.size(); lv++) {
         const NdLevel &L = F->plan.level[lv];

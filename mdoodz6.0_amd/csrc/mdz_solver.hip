@@ -32,6 +32,7 @@
  */
 #include <hip/hip_runtime.h>
 
+#include <limits.h>
 #include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -73,6 +74,21 @@ static int sv_err(int code, const char *fmt, ...) {
         hipError_t _e = (x);                                                                       \
         if (_e != hipSuccess) return sv_err(MDZ_EHIP, "%s: %s", #x, hipGetErrorString(_e));        \
     } while (0)
+/* A sparse matrix in slices of 64 rows: entry e of row i at base[i / 64] +
+ * 64 e + i % 64, so that a wave reads its rows' e-th entries side by side;
+ * a slice is as wide as its longest row, rounded up to eight, and a shorter
+ * row is padded with zeros at column i. */
+struct SliceView {
+    const int *base, *Ic, *J;
+    double *A;
+};
+struct SlicedRows {
+    int *base = nullptr, *Ic = nullptr, *J = nullptr;
+    double *A = nullptr;
+    int width = 0; /* of the widest slice */
+    SliceView view() const { return SliceView{base, Ic, J, A}; }
+};
+
 struct MdzSolver {
     hipStream_t s = nullptr;
     int n = 0, np = 0, kd = 0, nb = 0, nequ = 0;
@@ -80,9 +96,7 @@ struct MdzSolver {
     bool ordered = false;
     /* patterns of Jts = A - B Dpen C and Js = AJ - BJ Dpen C (unique sorted
      * columns per row), their values */
-    int *ts_Ic = nullptr, *ts_J = nullptr, *js_Ic = nullptr, *js_J = nullptr;
-    double *ts_val = nullptr, *js_val = nullptr;
-    int nnz_ts = 0, nnz_js = 0;
+    SlicedRows ts, js;
     /* pc_type 1: AJ's transpose (row i: the entries of AJ's column i, their rows) */
     int pc_type = 0;
     int *tr_Ic = nullptr, *tr_J = nullptr, *tr_src = nullptr;
@@ -96,9 +110,9 @@ struct MdzSolver {
     hipGraphExec_t pc_exec = nullptr;
     const void *pc_key[2] = {};
     unsigned long long pc_version = 0;
-    double *partial = nullptr; /* SV_RED * 32 */
-    double *dscal = nullptr;   /* device scalars: 0..31 dots, 32.. misc */
-    double *hscal = nullptr;   /* pinned host copy */
+    double *partial = nullptr; /* SV_RED * 32 slots, twice */
+    double *dscal = nullptr;   /* the orthogonalisation's dots of the last directions */
+    double *hscal = nullptr;   /* pinned: sums the host reads, written by the device */
 };
 
 /* ------------------------------------------------------------------ */
@@ -165,36 +179,61 @@ static CsrView view(const SolverCsr &c) { return CsrView{c.Ic, c.J, c.A}; }
  * Solvers.c:2404-2408, pscale = 1/2).  Jts and Js go through this one function: on a linear model
  * (AJ = A, BJ = B) they are the same numbers, and the factor of Jts is an
  * exact inverse of Js. */
-__global__ void __launch_bounds__(SV_BLK) k_schur_values(int n, const int *Ic, const int *J, CsrView P, double pscale,
-                                                         const int *TIc, const int *TJ, const int *Tsrc, CsrView B,
-                                                         CsrView C, const double *Dpen, double *val) {
-    const int i = blockIdx.x * SV_BLK + threadIdx.x;
-    if (i >= n) return;
-    const int e0 = Ic[i], e1 = Ic[i + 1];
-    auto at = [&](int j) {
-        int e = e0;
-        while (e < e1 - 1 && J[e] != j) e++;
-        return e;
-    };
-    for (int e = e0; e < e1; e++) val[e] = 0.0;
-    for (int eb = B.Ic[i]; eb < B.Ic[i + 1]; eb++) {
-        const int k = B.J[eb];
-        const double bk = B.A[eb], dk = Dpen[k];
-        for (int ec = C.Ic[k]; ec < C.Ic[k + 1]; ec++) {
-            const int e = at(C.J[ec]);
-            val[e] = val[e] + bk * (dk * C.A[ec]);
-        }
+template <bool LDS>
+__global__ void __launch_bounds__(64) k_schur_values(int n, SliceView M, CsrView P, double pscale, const int *TIc,
+                                                     const int *TJ, const int *Tsrc, CsrView B, CsrView C,
+                                                     const double *Dpen) {
+    extern __shared__ double sv_lds[];
+    const int l = threadIdx.x, i = blockIdx.x * 64 + l;
+    const int base = M.base[blockIdx.x], wide = (M.base[blockIdx.x + 1] - base) >> 6;
+    /* the slice's columns and sums in LDS (they are searched and summed some
+     * forty times a row); rows too wide for it work in place */
+    double *val = LDS ? sv_lds : M.A + base;
+    const int *col = M.J + base;
+    if (LDS) {
+        int *c = (int *)(sv_lds + wide * 64);
+        for (int e = 0; e < wide; e++) c[e * 64 + l] = col[e * 64 + l];
+        col = c;
     }
-    for (int ep = P.Ic[i]; ep < P.Ic[i + 1]; ep++) {
-        const int e = at(P.J[ep]);
-        val[e] = val[e] - pscale * P.A[ep];
-    }
-    if (TIc) /* pc_type 1: the transpose's half, P(j, i) for the entries of column i */
-        for (int et = TIc[i]; et < TIc[i + 1]; et++) {
-            const int e = at(TJ[et]);
-            val[e] = val[e] - pscale * P.A[Tsrc[et]];
+    for (int e = 0; e < wide; e++) val[e * 64 + l] = 0.0;
+    if (i < n) {
+        const int len = M.Ic[i + 1] - M.Ic[i];
+        auto at = [&](int j) { /* the row's columns increase */
+            int a = 0, b = len - 1;
+            while (a < b) {
+                const int m = (a + b) >> 1;
+                if (col[m * 64 + l] < j) a = m + 1;
+                else b = m;
+            }
+            return a * 64 + l;
+        };
+        for (int eb = B.Ic[i]; eb < B.Ic[i + 1]; eb++) {
+            const int k = B.J[eb];
+            const double bk = B.A[eb], dk = Dpen[k];
+            for (int ec = C.Ic[k]; ec < C.Ic[k + 1]; ec++) {
+                const int e = at(C.J[ec]);
+                val[e] = val[e] + bk * (dk * C.A[ec]);
+            }
         }
-    for (int e = e0; e < e1; e++) val[e] = -val[e];
+        for (int ep = P.Ic[i]; ep < P.Ic[i + 1]; ep++) {
+            const int e = at(P.J[ep]);
+            val[e] = val[e] - pscale * P.A[ep];
+        }
+        if (TIc) /* pc_type 1: the transpose's half, P(j, i) for the entries of column i */
+            for (int et = TIc[i]; et < TIc[i + 1]; et++) {
+                const int e = at(TJ[et]);
+                val[e] = val[e] - pscale * P.A[Tsrc[et]];
+            }
+    }
+    for (int e = 0; e < wide; e++) M.A[base + e * 64 + l] = -val[e * 64 + l];
+}
+
+/* columns of a sliced matrix from its CSR ones */
+__global__ void __launch_bounds__(64) k_slice_columns(int n, const int *base, const int *Ic, const int *J, int *out) {
+    const int l = threadIdx.x, i = blockIdx.x * 64 + l;
+    const int b = base[blockIdx.x], wide = (base[blockIdx.x + 1] - b) >> 6;
+    const int e0 = i < n ? Ic[i] : 0, len = i < n ? Ic[i + 1] - e0 : 0;
+    for (int e = 0; e < wide; e++) out[b + e * 64 + l] = e < len ? J[e0 + e] : min(i, n - 1);
 }
 
 /* ------------------------------------------------------------------ */
@@ -206,34 +245,66 @@ __device__ __forceinline__ double row_dot(const CsrView &M, int i, const double 
     return s;
 }
 
+/* the same of a sliced matrix */
+__device__ __forceinline__ double slice_dot(const SliceView &M, int i, const double *x) {
+    const int b = M.base[i >> 6], w = M.base[(i >> 6) + 1] - b;
+    const int *J = M.J + b + (i & 63);
+    const double *A = M.A + b + (i & 63);
+    double s = 0.0;
+    for (int e = 0; e < w; e += 512) { /* (widths are multiples of eight) */
+        double p[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) p[u] = A[e + 64 * u] * x[J[e + 64 * u]];
+#pragma unroll
+        for (int u = 0; u < 8; u++) s += p[u];
+    }
+    return s;
+}
+
+/* row i of M x by the 8 lanes of a group, the sum in every lane */
+__device__ __forceinline__ double group_dot(const CsrView &M, int i, int g, const double *x) {
+    double s = 0.0;
+    for (int e = M.Ic[i] + g; e < M.Ic[i + 1]; e += 8) s += M.A[e] * x[M.J[e]];
+    for (int o = 4; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    return s;
+}
+
 /* b - row i of M x with products and sums carried in two doubles (the error
  * of each is exact: Ogita, Rump and Oishi 2005, Dot2).  The penalty entries
  * make a residual the difference of terms about 1e5 times larger, whose
  * rounding the soft modes amplify: in plain doubles it is what bounds the
  * correction's accuracy.  The rows are read at memory speed either way. */
-__device__ __forceinline__ double row_residual(const CsrView &M, int i, const double *x, double b) {
-    double s = b, c = 0.0;
-    for (int e = M.Ic[i]; e < M.Ic[i + 1]; e++) {
-        const double a = -M.A[e], y = x[M.J[e]];
-        const double p = a * y, q = __builtin_fma(a, y, -p);
+struct TwoSum {
+    double s, c = 0.0;
+    __device__ __forceinline__ void sub(double a, double y) { /* s - a y */
+        const double p = -a * y, q = __builtin_fma(-a, y, -p);
         const double t = s + p, z = t - s;
         c += ((s - (t - z)) + (p - z)) + q;
         s = t;
     }
-    return s + c;
+};
+
+__device__ __forceinline__ double row_residual(const CsrView &M, int i, const double *x, double b) {
+    TwoSum r{b};
+    for (int e = M.Ic[i]; e < M.Ic[i + 1]; e++) r.sub(M.A[e], x[M.J[e]]);
+    return r.s + r.c;
 }
 
-/* out = M x */
-__global__ void __launch_bounds__(SV_BLK) k_csr_apply(int n, CsrView M, const double *x, double *out) {
-    const int i = blockIdx.x * SV_BLK + threadIdx.x;
-    if (i < n) out[i] = row_dot(M, i, x);
-}
-
-/* out = b - M x */
-__global__ void __launch_bounds__(SV_BLK) k_csr_residual(int n, CsrView M, const double *x, const double *b,
-                                                         double *out) {
-    const int i = blockIdx.x * SV_BLK + threadIdx.x;
-    if (i < n) out[i] = row_residual(M, i, x, b[i]);
+/* out = b - M x, slot 0: its sum of squares */
+__global__ void __launch_bounds__(SV_BLK) k_slice_residual(int n, SliceView M, const double *x, const double *b,
+                                                           double *out, double *partial) {
+    __shared__ double lds4[4];
+    double ss = 0.0;
+    for (int i = blockIdx.x * SV_BLK + threadIdx.x; i < n; i += SV_RED * SV_BLK) {
+        const int e0 = M.base[i >> 6], w = M.base[(i >> 6) + 1] - e0;
+        TwoSum r{b[i]};
+        for (int e = e0 + (i & 63); e < e0 + w; e += 64) r.sub(M.A[e], x[M.J[e]]);
+        const double f = r.s + r.c;
+        out[i] = f;
+        ss += f * f;
+    }
+    ss = block_sum(ss, lds4);
+    if (threadIdx.x == 0) partial[(size_t)blockIdx.x * 32] = ss;
 }
 
 /* udum = (bu - BJ (Dpen bp)) - BJ (incomp dp)  (Solvers.c:2510-2516) */
@@ -260,18 +331,21 @@ __global__ void __launch_bounds__(SV_BLK) k_ph_dp(int np, CsrView CJ, const doub
     dp[k] = Dpen[k] * pd + dp[k];
 }
 
-/* fu = (bu - AJ du) - BJ dp, with per-block maxima (slot 0) and the sums of
+/* fu = (bu - AJ du) - BJ dp (8 lanes a row), with per-block maxima (slot 0) and the sums of
  * squares over u and v equations (slots 1, 2) */
 __global__ void __launch_bounds__(SV_BLK) k_res_mom(int n, int nequ, CsrView AJ, CsrView BJ, const double *bu,
                                                     const double *du, const double *dp, double *fu, double *partial) {
     __shared__ double lds4[4];
     double mx = -INFINITY, su = 0.0, sv = 0.0;
-    for (int i = blockIdx.x * SV_BLK + threadIdx.x; i < n; i += SV_RED * SV_BLK) {
-        const double f = (bu[i] - row_dot(AJ, i, du)) - row_dot(BJ, i, dp);
-        fu[i] = f;
-        mx = fmax(mx, f);
-        if (i < nequ) su += f * f;
-        else sv += f * f;
+    const int g = threadIdx.x & 7;
+    for (int i = (blockIdx.x * SV_BLK + threadIdx.x) >> 3; i < n; i += SV_RED * SV_BLK / 8) {
+        const double f = (bu[i] - group_dot(AJ, i, g, du)) - group_dot(BJ, i, g, dp);
+        if (g == 0) {
+            fu[i] = f;
+            mx = fmax(mx, f);
+            if (i < nequ) su += f * f;
+            else sv += f * f;
+        }
     }
     mx = block_max(mx, lds4);
     su = block_sum(su, lds4);
@@ -303,24 +377,32 @@ __global__ void __launch_bounds__(SV_BLK) k_res_cont(int np, CsrView CJ, const d
     }
 }
 
-/* slot 0: sum of squares of f */
-__global__ void __launch_bounds__(SV_BLK) k_norm2(int n, const double *f, double *partial) {
-    __shared__ double lds4[4];
-    double s = 0.0;
-    for (int i = blockIdx.x * SV_BLK + threadIdx.x; i < n; i += SV_RED * SV_BLK) s += f[i] * f[i];
-    s = block_sum(s, lds4);
-    if (threadIdx.x == 0) partial[(size_t)blockIdx.x * 32] = s;
+/* sum of one row of SV_RED slots, by a wave (in every lane) */
+__device__ __forceinline__ double slots_sum(const double *row) {
+    double x = 0.0;
+#pragma unroll
+    for (int b = 0; b < SV_RED; b += 64) x += row[b + (threadIdx.x & 63)];
+    return wave_sum(x);
 }
 
-/* slots q < nq: v . VV[q] */
-__global__ void __launch_bounds__(SV_BLK) k_mdot(int n, const double *v, const double *VV, size_t ldv, int nq,
-                                                 double *partial) {
+/* A GCR direction after the preconditioner is three launches, each taking
+ * the sums that the one before left per block (every block adds them again,
+ * in the same order: a few KB from L2, less than a launch to do it once).
+ * At 257 x 129 cells these and the norm's take 27 us a direction, against 50
+ * for nine launches on CSR rows and a copy of the norm (the product alone 13
+ * for 16, at 513 x 257 cells 18 for 168: one lane a row of CSR reads lines
+ * of 64 rows for each entry).
+ *
+ * v = Js s; row q of dots: v . VV[q], q < nq */
+__global__ void __launch_bounds__(SV_BLK) k_gcr_product(int n, SliceView M, const double *s, const double *VV,
+                                                        size_t ldv, int nq, double *v, double *dots) {
     __shared__ double lds[SV_RESTART][4];
     double acc[SV_RESTART];
 #pragma unroll
     for (int q = 0; q < SV_RESTART; q++) acc[q] = 0.0;
     for (int i = blockIdx.x * SV_BLK + threadIdx.x; i < n; i += SV_RED * SV_BLK) {
-        const double vi = v[i];
+        const double vi = slice_dot(M, i, s);
+        v[i] = vi;
 #pragma unroll
         for (int q = 0; q < SV_RESTART; q++)
             if (q < nq) acc[q] += vi * VV[q * ldv + i];
@@ -336,55 +418,58 @@ __global__ void __launch_bounds__(SV_BLK) k_mdot(int n, const double *v, const d
     __syncthreads();
     if (threadIdx.x < nq) {
         const int q = threadIdx.x;
-        partial[(size_t)blockIdx.x * 32 + q] = (lds[q][0] + lds[q][1]) + (lds[q][2] + lds[q][3]);
+        dots[q * SV_RED + blockIdx.x] = (lds[q][0] + lds[q][1]) + (lds[q][2] + lds[q][3]);
     }
 }
 
-/* v -= sum_{q <= i1} val[q] VV[q] and s -= sum_{q <= i1} val[q] SS[q], one
- * term after the other (Solvers.c:164-168) */
-__global__ void __launch_bounds__(SV_BLK) k_orth(int n, int nq, const double *val, const double *VV,
-                                                 const double *SS, size_t ldv, double *v, double *s) {
-    const int i = blockIdx.x * SV_BLK + threadIdx.x;
-    if (i >= n) return;
-    double vi = v[i], si = s[i];
-    for (int q = 0; q < nq; q++) {
-        const double fact = -val[q];
-        vi = vi + fact * VV[q * ldv + i];
-        si = si + fact * SS[q * ldv + i];
+/* v -= sum_q val[q] VV[q] and s -= sum_q val[q] SS[q], one term after the
+ * other (Solvers.c:164-168): val[q] = v . VV[q] for q < i1, and from the
+ * second cycle on val[i1] of the cycle before; rows 0, 1 of fv: f . v, v . v */
+__global__ void __launch_bounds__(SV_BLK) k_gcr_orth(int n, int i1, int cycle, const double *dots, double *val,
+                                                     const double *VV, const double *SS, size_t ldv, const double *f,
+                                                     double *v, double *s, double *fv) {
+    __shared__ double sval[SV_RESTART], lds4[4];
+    const int w = threadIdx.x >> 6, nq = i1 + (cycle > 0);
+    for (int q = w; q < nq; q += 4) {
+        const double x = q < i1 ? slots_sum(dots + q * SV_RED) : val[q];
+        if ((threadIdx.x & 63) == 0) {
+            sval[q] = x;
+            if (blockIdx.x == 0 && q < i1) val[q] = x;
+        }
     }
-    v[i] = vi;
-    s[i] = si;
-}
-
-/* slots 0, 1: f . v and v . v */
-__global__ void __launch_bounds__(SV_BLK) k_dot2(int n, const double *f, const double *v, double *partial) {
-    __shared__ double lds4[4];
+    __syncthreads();
     double a = 0.0, b = 0.0;
     for (int i = blockIdx.x * SV_BLK + threadIdx.x; i < n; i += SV_RED * SV_BLK) {
-        a += f[i] * v[i];
-        b += v[i] * v[i];
+        double vi = v[i], si = s[i];
+        for (int q = 0; q < nq; q++) {
+            const double fact = -sval[q];
+            vi = vi + fact * VV[q * ldv + i];
+            si = si + fact * SS[q * ldv + i];
+        }
+        v[i] = vi;
+        s[i] = si;
+        a += f[i] * vi;
+        b += vi * vi;
     }
     a = block_sum(a, lds4);
     b = block_sum(b, lds4);
     if (threadIdx.x == 0) {
-        partial[(size_t)blockIdx.x * 32] = a;
-        partial[(size_t)blockIdx.x * 32 + 1] = b;
+        fv[blockIdx.x] = a;
+        fv[SV_RED + blockIdx.x] = b;
     }
 }
 
-/* Solvers.c:170-182: v, s scaled by 1 / |v|, x += (f.v / |v|) s,
- * f -= (f.v / |v|) v; v and s also stored as direction i1 (VVq, SSq);
- * slot 0: sum of squares of the new f */
-__global__ void __launch_bounds__(SV_BLK) k_gcr_update(int n, const double *fv_vv, double *v, double *s, double *x,
-                                                       double *f, double *VVq, double *SSq, double *partial) {
+/* Solvers.c:170-182: v, s scaled by 1 / |v| are direction i1 (VVq, SSq), x
+ * += (f.v / |v|) s, f -= (f.v / |v|) v; slot 0: sum of squares of the new f */
+__global__ void __launch_bounds__(SV_BLK) k_gcr_update(int n, const double *fv, const double *v, const double *s,
+                                                       double *x, double *f, double *VVq, double *SSq,
+                                                       double *partial) {
     __shared__ double lds4[4];
-    const double nrm = sqrt(fv_vv[1]);
-    const double rdv = fv_vv[0] / nrm, fact = 1.0 / nrm;
+    const double nrm = sqrt(slots_sum(fv + SV_RED));
+    const double rdv = slots_sum(fv) / nrm, fact = 1.0 / nrm;
     double ss = 0.0;
     for (int i = blockIdx.x * SV_BLK + threadIdx.x; i < n; i += SV_RED * SV_BLK) {
         const double vi = v[i] * fact, si = s[i] * fact;
-        v[i] = vi;
-        s[i] = si;
         VVq[i] = vi;
         SSq[i] = si;
         x[i] = x[i] + rdv * si;
@@ -437,7 +522,7 @@ int mdz_solver_create(MdzSolver **out, hipStream_t s) {
         delete S;
         return rc;
     }
-    hipError_t e = hipMalloc((void **)&S->partial, (size_t)SV_RED * 32 * sizeof(double));
+    hipError_t e = hipMalloc((void **)&S->partial, 2 * (size_t)SV_RED * 32 * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void **)&S->dscal, 128 * sizeof(double));
     if (e == hipSuccess) e = hipHostMalloc((void **)&S->hscal, 128 * sizeof(double), hipHostMallocDefault);
     if (e != hipSuccess) {
@@ -448,6 +533,11 @@ int mdz_solver_create(MdzSolver **out, hipStream_t s) {
     return MDZ_OK;
 }
 
+static void free_rows(SlicedRows &m) {
+    hipFree(m.base); hipFree(m.Ic); hipFree(m.J); hipFree(m.A);
+    m = SlicedRows();
+}
+
 void mdz_solver_destroy(MdzSolver *S) {
     if (!S) return;
     if (S->s) hipStreamSynchronize(S->s);
@@ -455,7 +545,8 @@ void mdz_solver_destroy(MdzSolver *S) {
     if (S->pc_graph) hipGraphDestroy(S->pc_graph);
     mdz_factor_destroy(S->fac);
     hipFree(S->work); hipFree(S->partial); hipFree(S->dscal);
-    hipFree(S->ts_Ic); hipFree(S->ts_J); hipFree(S->js_Ic); hipFree(S->js_J); hipFree(S->ts_val); hipFree(S->js_val);
+    free_rows(S->ts);
+    free_rows(S->js);
     hipFree(S->tr_Ic); hipFree(S->tr_J); hipFree(S->tr_src);
     if (S->hscal) hipHostFree(S->hscal);
     delete S;
@@ -544,6 +635,44 @@ static int upload_ints(int **d, const std::vector<int> &h) {
     return MDZ_OK;
 }
 
+/* slices of a CSR pattern, on the device */
+static int slice_rows(SlicedRows &m, int n, const std::vector<int> &Ic, const std::vector<int> &J, hipStream_t s) {
+    const int ns = mdz_div_up_sv(n, 64);
+    std::vector<int> base((size_t)ns + 1, 0);
+    long long at = 0;
+    m.width = 0;
+    for (int q = 0; q < ns; q++) {
+        int w = 0;
+        for (int i = 64 * q; i < std::min(n, 64 * q + 64); i++) w = std::max(w, Ic[(size_t)i + 1] - Ic[i]);
+        w = (w + 7) & ~7;
+        m.width = std::max(m.width, w);
+        at += 64LL * w;
+        if (at > INT_MAX) return sv_err(MDZ_EUNSUPPORTED, "solver: more than 2^31 matrix entries");
+        base[(size_t)q + 1] = (int)at;
+    }
+    int *csr = nullptr, rc;
+    hipFree(m.J); hipFree(m.A);
+    m.J = nullptr;
+    m.A = nullptr;
+    if ((rc = upload_ints(&m.base, base)) || (rc = upload_ints(&m.Ic, Ic)) || (rc = upload_ints(&csr, J))) {
+        hipFree(csr);
+        return rc;
+    }
+    const size_t len = std::max<size_t>((size_t)at, 1);
+    hipError_t e = hipMalloc((void **)&m.J, len * sizeof(int));
+    if (e == hipSuccess) e = hipMalloc((void **)&m.A, len * sizeof(double));
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_slice_columns, dim3(ns), dim3(64), 0, s, n, (const int *)m.base, (const int *)m.Ic,
+                           (const int *)csr, m.J);
+        e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+    }
+    hipFree(csr);
+    if (e != hipSuccess)
+        return sv_err(e == hipErrorOutOfMemory ? MDZ_ENOMEM : MDZ_EHIP, "solver rows: %s", hipGetErrorString(e));
+    return MDZ_OK;
+}
+
 static int check_pattern(const SolverPattern &p, int nrow, int ncol, const char *name) {
     if (!p.Ic || !p.J) return sv_err(MDZ_EINVAL, "solver ordering: pattern %s missing", name);
     if (p.Ic[0] != 0) return sv_err(MDZ_EINVAL, "solver ordering: row pointers of %s", name);
@@ -607,17 +736,11 @@ static int order_system(MdzSolver *S, int Nx, int Nz, int nu, int np, const int 
     if (nb <= 0) nb = SV_NB_DEFAULT;
     if (nb < 64 || nb % 64) return sv_err(MDZ_EINVAL, "solver block size %d (a multiple of 64)", nb);
     S->ordered = false;
-    if ((rc = mdz_factor_analyse(S->fac, Nx, Nz, nu, mom_node, tsI, tsJ)) || (rc = upload_ints(&S->ts_Ic, tsI)) ||
-        (rc = upload_ints(&S->ts_J, tsJ)) || (rc = upload_ints(&S->js_Ic, jsI)) || (rc = upload_ints(&S->js_J, jsJ)) ||
+    if ((rc = mdz_factor_analyse(S->fac, Nx, Nz, nu, mom_node, tsI, tsJ)) ||
+        (rc = slice_rows(S->ts, nu, tsI, tsJ, S->s)) || (rc = slice_rows(S->js, nu, jsI, jsJ, S->s)) ||
         (rc = upload_ints(&S->tr_Ic, trI)) || (rc = upload_ints(&S->tr_J, trJ)) || (rc = upload_ints(&S->tr_src, trS)))
         return rc;
     S->pc_type = pc_type;
-    hipFree(S->ts_val); hipFree(S->js_val);
-    S->ts_val = S->js_val = nullptr;
-    SVHIP(hipMalloc((void **)&S->ts_val, std::max(tsJ.size(), (size_t)1) * sizeof(double)));
-    SVHIP(hipMalloc((void **)&S->js_val, std::max(jsJ.size(), (size_t)1) * sizeof(double)));
-    S->nnz_ts = (int)tsJ.size();
-    S->nnz_js = (int)jsJ.size();
     S->n = nu;
     S->np = np;
     S->nequ = nequ;
@@ -654,29 +777,35 @@ static int ensure_buffers(MdzSolver *S) {
     return MDZ_OK;
 }
 
-/* device scalar slots */
-enum { SC_VAL = 0, SC_FV = 32, SC_NORM = 34, SC_RES = 40 };
+/* slots of the pinned scalars */
+enum { SC_NORM = 0, SC_RES = 8 };
 
-static int read_scalars(MdzSolver *S, int first, int count) {
-    SVHIP(hipMemcpyAsync(S->hscal + first, S->dscal + first, count * sizeof(double), hipMemcpyDeviceToHost, S->s));
+/* the scalars of the launches so far */
+static int wait_scalars(MdzSolver *S) {
+    SVHIP(hipGetLastError());
     SVHIP(hipStreamSynchronize(S->s));
     return MDZ_OK;
 }
 
+/* values of a sliced P - B Dpen C */
+static void schur_values(const SlicedRows &m, int n, const CsrView &P, double pscale, const int *TIc, const int *TJ,
+                         const int *Tsrc, const CsrView &B, const CsrView &C, const double *Dpen, hipStream_t s) {
+    const dim3 grid(mdz_div_up_sv(n, 64)), blk(64);
+    const size_t lds = (size_t)m.width * 64 * (sizeof(double) + sizeof(int));
+    if (lds <= 64 * 1024)
+        hipLaunchKernelGGL(k_schur_values<true>, grid, blk, lds, s, n, m.view(), P, pscale, TIc, TJ, Tsrc, B, C, Dpen);
+    else
+        hipLaunchKernelGGL(k_schur_values<false>, grid, blk, 0, s, n, m.view(), P, pscale, TIc, TJ, Tsrc, B, C, Dpen);
+}
+
 static int factorise(MdzSolver *S, const SolverInput &in) {
-    const int n = S->n;
-    hipStream_t s = S->s;
-    const dim3 gN(mdz_div_up_sv(n, SV_BLK)), blk(SV_BLK);
     const bool sym = S->pc_type == 1;
-    hipLaunchKernelGGL(k_schur_values, gN, blk, 0, s, n, (const int *)S->ts_Ic, (const int *)S->ts_J,
-                       view(sym ? in.AJ : in.A), sym ? 0.5 : 1.0, (const int *)(sym ? S->tr_Ic : nullptr),
-                       (const int *)S->tr_J, (const int *)S->tr_src, view(in.B), view(in.C), in.Dpen, S->ts_val);
-    hipLaunchKernelGGL(k_schur_values, gN, blk, 0, s, n, (const int *)S->js_Ic, (const int *)S->js_J, view(in.AJ), 1.0,
-                       (const int *)nullptr, (const int *)nullptr, (const int *)nullptr, view(in.BJ), view(in.C),
-                       in.Dpen, S->js_val);
+    schur_values(S->ts, S->n, view(sym ? in.AJ : in.A), sym ? 0.5 : 1.0, sym ? S->tr_Ic : nullptr, S->tr_J, S->tr_src,
+                 view(in.B), view(in.C), in.Dpen, S->s);
+    schur_values(S->js, S->n, view(in.AJ), 1.0, nullptr, nullptr, nullptr, view(in.BJ), view(in.C), in.Dpen, S->s);
     SVHIP(hipGetLastError());
     int bad = -1;
-    const int rc = mdz_factor_numeric(S->fac, S->ts_Ic, S->ts_J, S->ts_val, &bad);
+    const int rc = mdz_factor_numeric(S->fac, S->ts.base, S->ts.Ic, S->ts.J, S->ts.A, &bad);
     if (rc) return rc;
     if (bad >= 0)
         return sv_err(MDZ_ESOLVE, "Cholesky factor of Jts: the pivot of momentum equation %d is not positive", bad);
@@ -717,19 +846,9 @@ static int run_precondition(MdzSolver *S) {
     return MDZ_OK;
 }
 
-/* out = Js x, or b - Js x */
-static void apply_js(MdzSolver *S, const double *x, const double *b, double *out) {
-    const CsrView js{S->js_Ic, S->js_J, S->js_val};
-    const dim3 grid(mdz_div_up_sv(S->n, SV_BLK)), blk(SV_BLK);
-    if (b) hipLaunchKernelGGL(k_csr_residual, grid, blk, 0, S->s, S->n, js, x, b, out);
-    else hipLaunchKernelGGL(k_csr_apply, grid, blk, 0, S->s, S->n, js, x, out);
-}
-
-static int final_sum(MdzSolver *S, int nq, int max_mask, int slot) {
+static void final_sum(MdzSolver *S, int nq, int max_mask, int slot) {
     hipLaunchKernelGGL(k_final, dim3(nq), dim3(SV_BLK), 0, S->s, (const double *)S->partial, nq, max_mask,
-                       S->dscal + slot);
-    SVHIP(hipGetLastError());
-    return MDZ_OK;
+                       S->hscal + slot);
 }
 
 /* kspgcr (Solvers.c:100-227) on x with right-hand side b */
@@ -737,13 +856,12 @@ static int kspgcr(MdzSolver *S, const SolverInput &in, const double *b, double *
     const int noisy = in.noisy;
     const int n = S->n;
     hipStream_t s = S->s;
-    const dim3 gN(mdz_div_up_sv(n, SV_BLK)), gR(SV_RED), blk(SV_BLK);
+    const dim3 gR(SV_RED), blk(SV_BLK);
+    double *dots = S->partial + (size_t)SV_RED * 32, *fv = dots + (size_t)SV_RED * 30;
     int rc;
-    SVHIP(hipMemsetAsync(S->dscal + SC_VAL, 0, SV_RESTART * sizeof(double), s));
-    SVHIP(hipMemsetAsync(S->VV, 0, 2 * SV_RESTART * S->ldv * sizeof(double), s));
-    apply_js(S, x, b, S->f); /* f = b - M x */
-    hipLaunchKernelGGL(k_norm2, gR, blk, 0, s, n, (const double *)S->f, S->partial);
-    if ((rc = final_sum(S, 1, 0, SC_NORM)) || (rc = read_scalars(S, SC_NORM, 1))) return rc;
+    hipLaunchKernelGGL(k_slice_residual, gR, blk, 0, s, n, S->js.view(), (const double *)x, b, S->f, S->partial);
+    final_sum(S, 1, 0, SC_NORM);
+    if ((rc = wait_scalars(S))) return rc;
     double norm_r = sqrt(S->hscal[SC_NORM]);
     const double rnorm0 = norm_r;
     int its = 0, success = 0;
@@ -751,22 +869,19 @@ static int kspgcr(MdzSolver *S, const SolverInput &in, const double *b, double *
         *its_out = 0;
         return MDZ_OK;
     }
-    while (!success && its < SV_MAXIT) {
+    for (int cycle = 0; !success && its < SV_MAXIT; cycle++) {
         for (int i1 = 0; i1 < SV_RESTART; i1++) {
+            double *VVq = S->VV + (size_t)i1 * S->ldv, *SSq = S->SS + (size_t)i1 * S->ldv;
             if ((rc = run_precondition(S))) return rc;
-            apply_js(S, S->sv, nullptr, S->v);
-            if (i1 > 0) {
-                hipLaunchKernelGGL(k_mdot, gR, blk, 0, s, n, (const double *)S->v, (const double *)S->VV, S->ldv, i1,
-                                   S->partial);
-                if ((rc = final_sum(S, i1, 0, SC_VAL))) return rc;
-            }
-            hipLaunchKernelGGL(k_orth, gN, blk, 0, s, n, i1 + 1, (const double *)(S->dscal + SC_VAL),
-                               (const double *)S->VV, (const double *)S->SS, S->ldv, S->v, S->sv);
-            hipLaunchKernelGGL(k_dot2, gR, blk, 0, s, n, (const double *)S->f, (const double *)S->v, S->partial);
-            if ((rc = final_sum(S, 2, 0, SC_FV))) return rc;
-            hipLaunchKernelGGL(k_gcr_update, gR, blk, 0, s, n, (const double *)(S->dscal + SC_FV), S->v, S->sv, x, S->f,
-                               S->VV + (size_t)i1 * S->ldv, S->SS + (size_t)i1 * S->ldv, S->partial);
-            if ((rc = final_sum(S, 1, 0, SC_NORM)) || (rc = read_scalars(S, SC_NORM, 1))) return rc;
+            hipLaunchKernelGGL(k_gcr_product, gR, blk, 0, s, n, S->js.view(), (const double *)S->sv,
+                               (const double *)S->VV, S->ldv, i1, S->v, dots);
+            hipLaunchKernelGGL(k_gcr_orth, gR, blk, 0, s, n, i1, cycle, (const double *)dots, S->dscal,
+                               (const double *)S->VV, (const double *)S->SS, S->ldv, (const double *)S->f, S->v, S->sv,
+                               fv);
+            hipLaunchKernelGGL(k_gcr_update, gR, blk, 0, s, n, (const double *)fv, (const double *)S->v,
+                               (const double *)S->sv, x, S->f, VVq, SSq, S->partial);
+            final_sum(S, 1, 0, SC_NORM);
+            if ((rc = wait_scalars(S))) return rc;
             norm_r = sqrt(S->hscal[SC_NORM]);
             if (noisy > 1) {
                 printf("[%1.4d] %1.4d KSP GCR Residual %1.12e %1.12e\n", its / (SV_RESTART + 1), its, norm_r,
@@ -797,7 +912,8 @@ static int residuals(MdzSolver *S, const SolverInput &in, const double *du, cons
                            S->fp, S->partial);
     else
         return sv_err(MDZ_EINVAL, "solver: no continuity rows");
-    return final_sum(S, 5, (1 << 0) | (1 << 3), SC_RES);
+    final_sum(S, 5, (1 << 0) | (1 << 3), SC_RES);
+    return wait_scalars(S);
 }
 
 int mdz_solver_solve(MdzSolver *S, const SolverInput &in, double *du, double *dp, mdz_solve_info *info) {
@@ -819,7 +935,7 @@ int mdz_solver_solve(MdzSolver *S, const SolverInput &in, double *du, double *dp
     hipStream_t s = S->s;
     SVHIP(hipMemsetAsync(du, 0, (size_t)S->n * sizeof(double), s));
     SVHIP(hipMemsetAsync(dp, 0, (size_t)S->np * sizeof(double), s));
-    if ((rc = residuals(S, in, du, dp)) || (rc = read_scalars(S, SC_RES, 5))) return rc;
+    if ((rc = residuals(S, in, du, dp))) return rc;
     const double maxru0 = S->hscal[SC_RES];
     double maxdiv = 0.0, maxru = 0.0, maxdiv0 = 0.0;
     int k;
@@ -832,7 +948,7 @@ int mdz_solver_solve(MdzSolver *S, const SolverInput &in, double *du, double *dp
         inf.ksp_its_total += its;
         hipLaunchKernelGGL(k_ph_dp, dim3(mdz_div_up_sv(S->np, SV_BLK)), dim3(SV_BLK), 0, s, S->np, view(in.CJ), in.bp,
                            (const double *)du, in.D1, in.Dpen, dp);
-        if ((rc = residuals(S, in, du, dp)) || (rc = read_scalars(S, SC_RES, 5))) return rc;
+        if ((rc = residuals(S, in, du, dp))) return rc;
         maxru = S->hscal[SC_RES];
         maxdiv = S->hscal[SC_RES + 3];
         if (k == 0) maxdiv0 = maxdiv;
