@@ -523,53 +523,66 @@ __global__ void __launch_bounds__(ND_BLK) k_nd_invert(const NdTask *__restrict__
 /* ------------------------------------------------------------------ */
 /* solves                                                               */
 /* ------------------------------------------------------------------ */
+/* A level of a solve is bound by its chain of dependent reads (a few MB over
+ * the whole chip): the task holds all of its front, the children's update
+ * vectors are found by one map, and the first ND_PRE columns or rows of T of
+ * every thread are read while the vector is still being gathered (257 x 129
+ * cells: 52 directions in 7.7 ms, 8.1 before).  Taking the levels at the top
+ * into one front of a thousand unknowns saves launches and loses as much to
+ * its panels (and its explicit inverse, one launch, is not accurate enough). */
+#define ND_PRE 8
+
 /* the children's update-vector entries of row r of a front */
-__device__ __forceinline__ double nd_child_vec(const NdNode *__restrict__ nodes, const NdNode &N,
-                                               const int *__restrict__ inv, const double *g, int r) {
+__device__ __forceinline__ double nd_child_vec(const NdSolve &t, const int *__restrict__ at, const double *g, int r) {
     double v = 0.0;
-#pragma unroll
-    for (int q = 0; q < 2; q++)
-        if (N.child[q] >= 0) {
-            const int i = inv[N.inv[q] + r];
-            if (i >= 0) v += g[nodes[N.child[q]].boff + i];
-        }
+    if (t.ga >= 0) v += g[at[t.ga + r]];
+    if (t.gb >= 0) v += g[at[t.gb + r]];
     return v;
 }
 
-/* Forward solve of a level: task = (node, tile of RT rows); y = L11^-1 r on
+/* Forward solve of a level: one tile of RT rows of a front; y = L11^-1 r on
  * the own rows, g = (children's) - L21 L11^-1 r on the boundary rows, r =
  * f + children's.  RT rows x 256 / RT column groups per workgroup: a wave
  * reads RT contiguous rows of 64 / RT columns; the groups' sums are added in
  * a fixed order. */
 template <int RT>
-__global__ void __launch_bounds__(ND_BLK) k_nd_forward(const NdTask *__restrict__ task,
-                                                       const NdNode *__restrict__ nodes, const int *__restrict__ inv,
-                                                       const int *__restrict__ eq, const double *__restrict__ P,
-                                                       const double *__restrict__ Lb, const double *__restrict__ f,
-                                                       double *__restrict__ y,
+__global__ void __launch_bounds__(ND_BLK) k_nd_forward(const NdSolve *__restrict__ task,
+                                                       const int *__restrict__ at, const int *__restrict__ eq,
+                                                       const double *__restrict__ P, const double *__restrict__ Lb,
+                                                       const double *__restrict__ f, double *__restrict__ y,
                                                        double *g) {
     constexpr int CG = ND_BLK / RT;
     __shared__ double rs[ND_CH];
     __shared__ double red[CG][RT];
-    const NdTask t = task[blockIdx.x];
-    const NdNode N = nodes[t.node];
+    const NdSolve t = task[blockIdx.x];
     const int lr = threadIdx.x % RT, cg = threadIdx.x / RT;
-    const int m = N.s + N.b, row0 = t.a * RT, row = row0 + lr;
-    const double *Tr = (N.np > 1 ? P : Lb) + N.poff + (row < m ? row : 0);
+    const int m = t.s + t.b, row0 = t.tile * RT, row = row0 + lr;
+    const double *Tr = (t.panels > 1 ? P : Lb) + t.toff + (row < m ? row : 0);
     /* own rows end at the diagonal tile of the last row */
     const int last = min(row0 + RT, m) - 1;
-    const int cend = last < N.s ? min(N.s, (last / ND_T + 1) * ND_T) : N.s;
-    const int rend = row < N.s ? min(N.s, (row / ND_T + 1) * ND_T) : row < m ? N.s : 0;
+    const int cend = last < t.s ? min(t.s, (last / ND_T + 1) * ND_T) : t.s;
+    const int rend = row >= m ? 0 : row < t.s ? min(t.s, (row / ND_T + 1) * ND_T) : t.s;
+    double pre[ND_PRE];
+    if (t.s > 0)
+#pragma unroll
+        for (int u = 0; u < ND_PRE; u++) pre[u] = Tr[(long long)min(cg + u * CG, t.s - 1) * t.ld];
     double acc = 0.0;
     for (int cb = 0; cb < cend; cb += ND_CH) {
         const int ce = min(cend, cb + ND_CH);
         if (cb) __syncthreads();
-        for (int c = cb + threadIdx.x; c < ce; c += ND_BLK)
-            rs[c - cb] = f[eq[N.ooff + c]] + nd_child_vec(nodes, N, inv, g, c);
+        for (int c = cb + threadIdx.x; c < ce; c += ND_BLK) {
+            rs[c - cb] = f[eq[t.ooff + c]] + nd_child_vec(t, at, g, c);
+        }
         __syncthreads();
         const int re = min(rend, ce);
+        int c = cb + cg;
+        if (cb == 0) {
+#pragma unroll
+            for (int u = 0; u < ND_PRE; u++, c += CG)
+                if (c < re) acc += pre[u] * rs[c];
+        }
 #pragma unroll 8
-        for (int c = cb + cg; c < re; c += CG) acc += Tr[(long long)c * N.ld] * rs[c - cb];
+        for (; c < re; c += CG) acc += Tr[(long long)c * t.ld] * rs[c - cb];
     }
     red[cg][lr] = acc;
     __syncthreads();
@@ -577,45 +590,54 @@ __global__ void __launch_bounds__(ND_BLK) k_nd_forward(const NdTask *__restrict_
         double sum = 0.0;
 #pragma unroll
         for (int q = 0; q < CG; q++) sum += red[q][lr];
-        if (row < N.s) y[N.ooff + row] = sum;
-        else g[N.boff + row - N.s] = nd_child_vec(nodes, N, inv, g, row) - sum;
+        if (row < t.s) y[t.ooff + row] = sum;
+        else g[t.boff + row - t.s] = nd_child_vec(t, at, g, row) - sum;
     }
 }
 
-/* Backward solve of a level: task = (node, tile of CT columns); x = T^T (y,
- * -x of the boundary): 16 lanes per column (128 contiguous bytes a step) */
+/* Backward solve of a level: one tile of CT columns of a front (inside one
+ * 64-column tile); x = T^T (y, -x of the boundary): 16 lanes per column (128
+ * contiguous bytes a step) */
 template <int CT>
-__global__ void __launch_bounds__(ND_BLK) k_nd_backward(const NdTask *__restrict__ task,
-                                                        const NdNode *__restrict__ nodes,
+__global__ void __launch_bounds__(ND_BLK) k_nd_backward(const NdSolve *__restrict__ task,
                                                         const int *__restrict__ blist, const int *__restrict__ eq,
-                                                        const double *__restrict__ P,
-                                                        const double *__restrict__ Lb, const double *__restrict__ y,
-                                                        double *x, double *__restrict__ out) {
+                                                        const double *__restrict__ P, const double *__restrict__ Lb,
+                                                        const double *__restrict__ y, double *x,
+                                                        double *__restrict__ out) {
     constexpr int NC = CT / 16;
     __shared__ double vs[ND_CH];
-    const NdTask t = task[blockIdx.x];
-    const NdNode N = nodes[t.node];
+    const NdSolve t = task[blockIdx.x];
     const int l = threadIdx.x & 15, cl = threadIdx.x >> 4;
-    const int m = N.s + N.b, c0 = t.a * CT;
-    double acc[NC];
-#pragma unroll
-    for (int q = 0; q < NC; q++) acc[q] = 0.0;
+    const int m = t.s + t.b, c0 = t.tile * CT;
     const int rfirst = (c0 / ND_T) * ND_T; /* rows of the columns' diagonal tile and below */
+    const double *Tc = (t.panels > 1 ? P : Lb) + t.toff + (long long)min(c0 + cl, t.s - 1) * t.ld;
+    const long long step = 16LL * t.ld;
+    double acc[NC], pre[NC][ND_PRE];
+#pragma unroll
+    for (int q = 0; q < NC; q++) {
+        acc[q] = 0.0;
+        const double *p = c0 + cl + 16 * q < t.s ? Tc + q * step : Tc;
+#pragma unroll
+        for (int u = 0; u < ND_PRE; u++) pre[q][u] = p[min(rfirst + l + 16 * u, m - 1)];
+    }
     for (int rb = rfirst; rb < m; rb += ND_CH) {
         const int re = min(m, rb + ND_CH);
         if (rb > rfirst) __syncthreads();
         for (int r = rb + threadIdx.x; r < re; r += ND_BLK)
-            vs[r - rb] = r < N.s ? y[N.ooff + r] : -x[blist[N.boff + r - N.s]];
+            vs[r - rb] = r < t.s ? y[t.ooff + r] : -x[blist[t.boff + r - t.s]];
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < NC; q++) {
-            const int c = c0 + cl + 16 * q;
-            if (c < N.s) {
-                const double *Tc = (N.np > 1 ? P : Lb) + N.poff + (long long)c * N.ld;
-                const int rs = max(rb, (c / ND_T) * ND_T);
+            if (c0 + cl + 16 * q < t.s) {
                 double a = 0.0;
+                int r = rb + l;
+                if (rb == rfirst) {
+#pragma unroll
+                    for (int u = 0; u < ND_PRE; u++, r += 16)
+                        if (r < re) a += pre[q][u] * vs[r - rb];
+                }
 #pragma unroll 8
-                for (int r = rs + l; r < re; r += 16) a += Tc[r] * vs[r - rb];
+                for (; r < re; r += 16) a += Tc[q * step + r] * vs[r - rb];
                 acc[q] += a;
             }
         }
@@ -625,9 +647,9 @@ __global__ void __launch_bounds__(ND_BLK) k_nd_backward(const NdTask *__restrict
         double a = acc[q];
         for (int o = 8; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
         const int c = c0 + cl + 16 * q;
-        if (l == 0 && c < N.s) {
-            x[N.ooff + c] = a;
-            out[eq[N.ooff + c]] = a;
+        if (l == 0 && c < t.s) {
+            x[t.ooff + c] = a;
+            out[eq[t.ooff + c]] = a;
         }
     }
 }
@@ -648,7 +670,8 @@ struct MdzFactor {
     NdPlan plan; /* after the upload: level, invert, eq and the lengths */
     NdBuf<NdNode> nodes;
     NdBuf<NdTask> tasks;
-    NdBuf<int> pos, eq, node_of, blist, inv, bad;
+    NdBuf<NdSolve> solves;
+    NdBuf<int> at, pos, eq, node_of, blist, inv, bad;
     NdBuf<double> P, Lb, Linv, U[2], y, x, g;
 };
 
@@ -687,7 +710,7 @@ int mdz_factor_create(MdzFactor **out, hipStream_t s) {
 void mdz_factor_destroy(MdzFactor *F) {
     if (!F) return;
     if (F->s) hipStreamSynchronize(F->s);
-    nd_free(F->nodes); nd_free(F->tasks);
+    nd_free(F->nodes); nd_free(F->tasks); nd_free(F->solves); nd_free(F->at);
     nd_free(F->pos); nd_free(F->eq); nd_free(F->node_of); nd_free(F->blist); nd_free(F->inv); nd_free(F->bad);
     nd_free(F->P); nd_free(F->Lb); nd_free(F->Linv); nd_free(F->U[0]); nd_free(F->U[1]);
     nd_free(F->y); nd_free(F->x); nd_free(F->g);
@@ -704,14 +727,16 @@ int mdz_factor_analyse(MdzFactor *F, int Nx, int Nz, int n, const int *mom_node,
     NdPlan &p = F->plan;
     int rc = nd_plan(p, Nx, Nz, n, mom_node, Ic, J);
     if (rc) return rc;
-    if ((rc = nd_upload(F->nodes, p.node)) || (rc = nd_upload(F->tasks, p.task)) || (rc = nd_upload(F->pos, p.pos)) ||
+    if ((rc = nd_upload(F->nodes, p.node)) || (rc = nd_upload(F->tasks, p.task)) ||
+        (rc = nd_upload(F->solves, p.solve)) || (rc = nd_upload(F->at, p.at)) || (rc = nd_upload(F->pos, p.pos)) ||
         (rc = nd_upload(F->eq, p.eq)) || (rc = nd_upload(F->node_of, p.node_of)) ||
         (rc = nd_upload(F->blist, p.blist)) || (rc = nd_upload(F->inv, p.inv)) || (rc = nd_reserve(F->bad, 1)) ||
         (rc = nd_reserve(F->P, p.panel_len)) || (rc = nd_reserve(F->Lb, p.panel_len)) ||
         (rc = nd_reserve(F->Linv, p.nlin * ND_T * ND_T)) || (rc = nd_reserve(F->U[0], p.ulen[0])) ||
         (rc = nd_reserve(F->U[1], p.ulen[1])) || (rc = nd_reserve(F->y, (size_t)n)) ||
-        (rc = nd_reserve(F->x, (size_t)n)) || (rc = nd_reserve(F->g, p.blist.size())))
+        (rc = nd_reserve(F->x, (size_t)n)) || (rc = nd_reserve(F->g, p.blist.size() + 1)))
         return rc;
+    FCHK(hipMemsetAsync(F->g.p, 0, (p.blist.size() + 1) * sizeof(double), F->s));
     F->n = n;
     return MDZ_OK;
 }
@@ -752,27 +777,30 @@ int mdz_factor_numeric(MdzFactor *F, const int *base, const int *Ic, const int *
 
 void mdz_factor_apply(MdzFactor *F, const double *f, double *x) {
     hipStream_t s = F->s;
-    const NdNode *nodes = F->nodes.p;
-    for (const NdLevel &L : F->plan.level) {
+    const dim3 blk(ND_BLK);
+    const size_t nl = F->plan.level.size();
+    const double *P = F->P.p, *Lb = F->Lb.p;
+    for (size_t q = 0; q < nl; q++) {
+        const NdLevel &L = F->plan.level[q];
         if (!L.forward.count) continue;
-        const NdTask *t = F->tasks.p + L.forward.first;
-        const dim3 grid(L.forward.count), blk(ND_BLK);
-#define FWD(RT)                                                                                                   \
-    hipLaunchKernelGGL((k_nd_forward<RT>), grid, blk, 0, s, t, nodes, (const int *)F->inv.p, (const int *)F->eq.p, \
-                       (const double *)F->P.p, (const double *)F->Lb.p, f, F->y.p, F->g.p)
+        const NdSolve *t = F->solves.p + L.forward.first;
+        const dim3 grid(L.forward.count);
+#define FWD(RT)                                                                                                       \
+    hipLaunchKernelGGL((k_nd_forward<RT>), grid, blk, 0, s, t, (const int *)F->at.p, (const int *)F->eq.p, P, Lb, f, \
+                       F->y.p, F->g.p)
         if (L.rt == 64) FWD(64);
         else if (L.rt == 32) FWD(32);
         else FWD(16);
 #undef FWD
     }
-    for (size_t q = F->plan.level.size(); q-- > 0;) {
+    for (size_t q = nl; q-- > 0;) {
         const NdLevel &L = F->plan.level[q];
         if (!L.backward.count) continue;
-        const NdTask *t = F->tasks.p + L.backward.first;
-        const dim3 grid(L.backward.count), blk(ND_BLK);
-#define BWD(CT)                                                                                                      \
-    hipLaunchKernelGGL((k_nd_backward<CT>), grid, blk, 0, s, t, nodes, (const int *)F->blist.p, (const int *)F->eq.p, \
-                       (const double *)F->P.p, (const double *)F->Lb.p, (const double *)F->y.p, F->x.p, x)
+        const NdSolve *t = F->solves.p + L.backward.first;
+        const dim3 grid(L.backward.count);
+#define BWD(CT)                                                                                                     \
+    hipLaunchKernelGGL((k_nd_backward<CT>), grid, blk, 0, s, t, (const int *)F->blist.p, (const int *)F->eq.p, P, Lb, \
+                       (const double *)F->y.p, F->x.p, x)
         if (L.ct == 64) BWD(64);
         else if (L.ct == 32) BWD(32);
         else BWD(16);

@@ -30,7 +30,6 @@ int mdz_error(int code, const char *msg);
 #ifndef ND_LEAF
 #define ND_LEAF 64 /* most unknowns of a leaf */
 #endif
-
 /* One node of the elimination tree.  Rows of its front: s own unknowns
  * (positions ooff ..), then b boundary unknowns (positions blist[boff ..],
  * increasing).  Panel: (s + b) x s, column-major, at poff with leading
@@ -45,6 +44,15 @@ struct NdNode {
 };
 struct NdTask {
     int node, a, b;
+};
+
+/* One workgroup of a solve: its front, where the rows of T are, and its tile.
+ * Maps ga, gb: from a row of the front to the update vectors of its children,
+ * all levels' in one array (its last entry, always zero, where the child has
+ * no such row); -1: no such child. */
+struct NdSolve {
+    long long toff;
+    int s, b, ld, panels, ooff, boff, ga, gb, tile, pad;
 };
 
 struct NdRange {
@@ -62,6 +70,8 @@ struct NdPlan {
     std::vector<NdRange> invert;
     std::vector<NdNode> node;
     std::vector<NdTask> task;
+    std::vector<NdSolve> solve;
+    std::vector<int> at; /* inv with places in the array of update vectors */
     std::vector<int> pos, eq, node_of; /* position of an equation, and back; node of a position */
     std::vector<int> blist, inv;
     size_t panel_len = 0, ulen[2] = {0, 0}, nlin = 0;
@@ -306,7 +316,7 @@ static int nd_plan(NdPlan &plan, int Nx, int Nz, int n, const int *mom_node, con
             poff += (long long)k.ld * k.s;
             k.uoff = uoff;
             uoff += (long long)k.ldu * k.b;
-            if (boff + k.b > INT_MAX || lin + k.np > INT_MAX || ioff + 2LL * m > INT_MAX)
+            if (boff + k.b >= INT_MAX || lin + k.np > INT_MAX || ioff + 2LL * m > INT_MAX)
                 return mdz_error(MDZ_EUNSUPPORTED, "factor: too many unknowns");
             k.boff = (int)boff;
             boff += k.b;
@@ -320,8 +330,10 @@ static int nd_plan(NdPlan &plan, int Nx, int Nz, int n, const int *mom_node, con
         ulen[lv & 1] = std::max(ulen[lv & 1], (size_t)uoff);
     }
     std::vector<int> &blist = plan.blist, &inv = plan.inv;
+    std::vector<int> &at_g = plan.at;
     blist.resize((size_t)boff);
     inv.resize((size_t)ioff);
+    at_g.resize((size_t)ioff);
     bool nested = true;
     {
         std::mutex mu;
@@ -333,11 +345,13 @@ static int nd_plan(NdPlan &plan, int Nx, int Nz, int n, const int *mom_node, con
                 for (int c = 0; c < 2; c++) {
                     if (k.child[c] < 0) continue;
                     const std::vector<int> &kb = B[(size_t)k.child[c]];
-                    int *v = inv.data() + k.inv[c];
+                    const int first = N[(size_t)k.child[c]].boff;
+                    int *v = inv.data() + k.inv[c], *g = at_g.data() + k.inv[c];
                     size_t p = 0;
                     for (int r = 0; r < k.s + k.b; r++) {
                         const int at_r = r < k.s ? k.ooff + r : B[(size_t)q][r - k.s];
                         v[r] = p < kb.size() && kb[p] == at_r ? (int)p++ : -1;
+                        g[r] = v[r] < 0 ? (int)boff : first + v[r];
                     }
                     if (p != kb.size()) good = false;
                 }
@@ -350,6 +364,7 @@ static int nd_plan(NdPlan &plan, int Nx, int Nz, int n, const int *mom_node, con
     /* launches */
     std::vector<NdTask> &task = plan.task;
     task.clear();
+    plan.solve.clear();
     plan.level.assign(nl, NdLevel());
     plan.invert.clear();
     int npmax = 0;
@@ -387,14 +402,18 @@ static int nd_plan(NdPlan &plan, int Nx, int Nz, int n, const int *mom_node, con
         /* tiles of the solves: as tall as keeps two workgroups per CU busy */
         L.rt = rows >= 64 * 512 ? 64 : rows >= 32 * 512 ? 32 : 16;
         L.ct = cols >= 64 * 512 ? 64 : cols >= 32 * 512 ? 32 : 16;
-        first = begin();
+        auto solve = [&](const NdNode &k, int tile) {
+            return NdSolve{k.poff, k.s,    k.b,    k.ld, k.np, k.ooff, k.boff, k.child[0] < 0 ? -1 : k.inv[0],
+                           k.child[1] < 0 ? -1 : k.inv[1], tile, 0};
+        };
+        first = (int)plan.solve.size();
         for (int q = q0; q < q1; q++)
-            for (int r = 0; r < N[q].s + N[q].b; r += L.rt) task.push_back({q, r / L.rt, 0});
-        L.forward = end(first);
-        first = begin();
+            for (int r = 0; r < N[q].s + N[q].b; r += L.rt) plan.solve.push_back(solve(N[q], r / L.rt));
+        L.forward = {first, (int)plan.solve.size() - first};
+        first = (int)plan.solve.size();
         for (int q = q0; q < q1; q++)
-            for (int c = 0; c < N[q].s; c += L.ct) task.push_back({q, c / L.ct, 0});
-        L.backward = end(first);
+            for (int c = 0; c < N[q].s; c += L.ct) plan.solve.push_back(solve(N[q], c / L.ct));
+        L.backward = {first, (int)plan.solve.size() - first};
     }
     for (int p = 0; p < (npmax > 1 ? npmax : 0); p++) { /* (fronts of one panel need none) */
         const int first = (int)task.size();

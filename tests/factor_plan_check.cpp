@@ -66,9 +66,17 @@ static int check(int Nx, int Nz, int reach, bool periodic, double drop, int seed
             all(L.panel[j], [&](const NdNode &k, NdTask t) {
                 return j < std::max(1, k.np) && t.b >= std::min(j + 1, k.np) && t.a >= t.b && t.a < tiles(k);
             });
-        all(L.forward, [&](const NdNode &k, NdTask t) { return t.a * L.rt < k.s + k.b; });
-        all(L.backward, [&](const NdNode &k, NdTask t) { return t.a * L.ct < k.s; });
+        for (const NdRange *r : {&L.forward, &L.backward})
+            for (int q = r->first; q < r->first + r->count; q++) {
+                const NdSolve &t = p.solve[q];
+                ok = ok && t.tile * (r == &L.forward ? L.rt : L.ct) < t.s + (r == &L.forward ? t.b : 0) &&
+                     t.toff + (long long)t.ld * t.s <= (long long)p.panel_len && t.ooff + t.s <= n &&
+                     t.boff + t.b <= (int)p.blist.size();
+                for (int m : {t.ga, t.gb})
+                    ok = ok && (m < 0 || (size_t)m + t.s + t.b <= p.at.size());
+            }
     }
+    for (int a : p.at) ok = ok && a >= 0 && a <= (int)p.blist.size();
     for (const NdRange &r : p.invert)
         all(r, [&](const NdNode &k, NdTask t) { return t.a < k.np && t.b >= t.a && t.b < tiles(k); });
     /* the matrix, its fronts */
@@ -117,7 +125,8 @@ static int check(int Nx, int Nz, int reach, bool periodic, double drop, int seed
             for (int cc = 0; cc < m; cc++)
                 for (int r = cc; r < m; r++) {
                     const int ir = p.inv[k.inv[c] + r], ic = p.inv[k.inv[c] + cc];
-                    ok = ok && ir < K.b && ic < K.b && (ir < 0 || ic < 0 || ir >= ic);
+                    ok = ok && ir < K.b && ic < K.b && (ir < 0 || ic < 0 || ir >= ic) &&
+                         p.at[k.inv[c] + r] == (ir < 0 ? (int)p.blist.size() : K.boff + ir);
                     if (ir >= 0 && ic >= 0) M[(size_t)cc * m + r] += MK[(size_t)(K.s + ic) * (K.s + K.b) + K.s + ir];
                 }
         }
