@@ -21,6 +21,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "mdz_kernels.h"
@@ -45,7 +46,6 @@
 #define LDS_W3T (LDS_W2T + 64 * LS64)
 #define LDS_W4T (LDS_W3T + 64 * LS64)
 #define LDS_ALL (LDS_W4T + 64 * LS16)
-#define AS LS64 /* row stride of the staged activations [rows][64 samples] */
 
 /* z[mt] = W[16mt .. 16mt+15][:] * B (+ bias), NK K-steps of 16 inputs; W
  * row-major with leading dimension ldw (in LDS); NM output tiles. */
@@ -242,219 +242,304 @@ __device__ __forceinline__ int lds_index(int i) {
 }
 
 /* weights into LDS: the forward ones (nw = MLP_WP_W2T) or all (MLP_WP_TOTAL),
- * two entries per thread and step */
+ * eight entries per thread and step (rows are 16 or 64 long: the eight share
+ * one; padded rows start on 8 bytes) */
 __device__ __forceinline__ void load_weights(DevMLPW w, unsigned short *sW, float *sB, int nw) {
-    const unsigned *src = (const unsigned *)w.wp;
-    for (int i = threadIdx.x; i < nw / 2; i += blockDim.x) {
-        const unsigned v = src[i];
-        const int d = lds_index(2 * i); /* rows have even lengths: 2i and 2i+1 share a row */
-        *(unsigned *)(sW + d) = v;
+    const uint4 *src = (const uint4 *)w.wp;
+    for (int i = threadIdx.x; i < nw / 8; i += blockDim.x) {
+        const uint4 v = src[i];
+        uint2 *d = (uint2 *)(sW + lds_index(8 * i));
+        d[0] = uint2{v.x, v.y};
+        d[1] = uint2{v.z, v.w};
     }
     for (int i = threadIdx.x; i < MLP_BP_TOTAL; i += blockDim.x) sB[i] = w.bp[i];
 }
 
 /* ------------------------------------------------------------------ */
-/* training step: forward + backward of 64 samples per block            */
+/* training step                                                        */
 /* ------------------------------------------------------------------ */
 __device__ __forceinline__ long long sample_index(long long j, long long n, unsigned long long mul,
                                                   unsigned long long add) {
     return (long long)((((unsigned long long)j % (unsigned long long)n) * mul + add) % (unsigned long long)n);
 }
 
-/* partial[block][p]: this block's gradient of sum((y - t)^2) / (2 * batch);
- * loss[block]: this block's sum of squared errors */
-__global__ void __launch_bounds__(TBLK) k_mlp_train_step(const float *__restrict__ X, const float *__restrict__ Y,
-                                                         long long n, long long first, unsigned long long mul,
-                                                         unsigned long long add, float inv_batch, DevMLPW w,
-                                                         float *__restrict__ partial, float *__restrict__ loss) {
-    __shared__ __attribute__((aligned(16))) unsigned short sW[LDS_ALL];
-    __shared__ float sB[MLP_BP_TOTAL];
-    __shared__ __attribute__((aligned(16))) unsigned short Xs[16 * AS];
-    __shared__ __attribute__((aligned(16))) unsigned short H1s[64 * AS], H2s[64 * AS], H3s[64 * AS];
-    __shared__ __attribute__((aligned(16))) unsigned short D1s[64 * AS], D2s[64 * AS], D3s[64 * AS], D4s[16 * AS];
-    __shared__ float sLoss[4];
-    load_weights(w, sW, sB, MLP_WP_TOTAL);
-    const int l = threadIdx.x & 63, r = l & 15, q = l >> 4, wv = threadIdx.x >> 6;
-    const int s = 16 * wv + r; /* sample within the block */
-    const long long idx = sample_index(first + (long long)blockIdx.x * TSAMP + s, n, mul, add);
-    /* features and targets */
-    float f[MLP_IN];
-#pragma unroll
-    for (int k = 0; k < MLP_IN; k++) f[k] = X[idx * MLP_IN + k];
-    const bf16x4 x = lane_features(f);
-#pragma unroll
-    for (int j = 0; j < 4; j++) Xs[(4 * q + j) * AS + s] = (unsigned short)x[j];
-    float t0 = 0.0f, t1 = 0.0f;
-    if (q == 0) {
-        t0 = Y[idx * 2];
-        t1 = Y[idx * 2 + 1];
-    }
-    __syncthreads();
+#define TWAVES 4                 /* waves of a training block, each on its own 16 samples at a time */
+#define TBLOCKS 256              /* most training blocks: one per CU */
+#define TS16 20                  /* row stride of 16 staged samples */
+#define TWAVE_LDS (4 * 64 * TS16 + 2 * 16 * TS16) /* H1 H2 H3 D, X D4 */
 
-    /* forward */
-    f32x4 z1[4], z2[4], z3[4], y;
-    mlp_forward(sW, sB, x, z1, z2, z3, y);
+/* a hidden layer's activations and their derivative, the activations also
+ * staged [row][sample] for the weight gradient */
+__device__ __forceinline__ void train_act(f32x4 *z, bf16x4 *h, unsigned short *Hs) {
+    const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
 #pragma unroll
-    for (int mt = 0; mt < 4; mt++)
+    for (int t = 0; t < 4; t++) {
+        f32x4 v;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int row = 16 * mt + 4 * q + i;
-            H1s[row * AS + s] = f2bf(silu(z1[mt][i]));
-            H2s[row * AS + s] = f2bf(silu(z2[mt][i]));
-            H3s[row * AS + s] = f2bf(silu(z3[mt][i]));
+            const float s = sigmoidf_(z[t][i]);
+            v[i] = z[t][i] * s;
+            z[t][i] = s * (1.0f + z[t][i] * (1.0f - s));
         }
-    /* loss and output gradient (rows 0, 1 in lanes q == 0) */
-    f32x4 dz4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    float se = 0.0f;
-    if (q == 0) {
-        float e0 = y[0] - t0, e1 = y[1] - t1;
-        se = e0 * e0 + e1 * e1;
-        dz4[0] = e0 * inv_batch;
-        dz4[1] = e1 * inv_batch;
-    }
+        h[t] = pack4(v);
 #pragma unroll
-    for (int i = 0; i < 4; i++) D4s[(4 * q + i) * AS + s] = f2bf(dz4[i]);
+        for (int i = 0; i < 4; i++) Hs[(16 * t + 4 * q + i) * TS16 + r] = (unsigned short)h[t][i];
+    }
+}
+
+/* a hidden layer's output gradients d (times the activation's derivative),
+ * rounded and staged; the sum of row l over the samples is added to *bias */
+__device__ __forceinline__ void train_grad(const f32x4 *d, const f32x4 *dact, bf16x4 *bd, unsigned short *Ds,
+                                           float *bias) {
+    const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        bd[t] = pack4(d[t] * dact[t]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) Ds[(16 * t + 4 * q + i) * TS16 + r] = (unsigned short)bd[t][i];
+    }
+    __builtin_amdgcn_wave_barrier();
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; k += 4) {
+        const bf16x4 v = lds4(Ds + l * TS16 + k);
+#pragma unroll
+        for (int i = 0; i < 4; i++) sum += bf2f((unsigned short)v[i]);
+    }
+    *bias += sum;
+}
+
+/* Forward and backward pass of `tiles` tiles of 16 samples, one wave per
+ * tile; partial[block][p]: the block's gradient of sum((y - t)^2) / (2
+ * batch), loss[block]: its sum of squared errors.
+ *
+ * The matrix products of a tile are about 120 instructions; what bounds the
+ * kernel is the chain through the layers and what surrounds the samples.
+ * So the waves are independent (a tile's activations are transposed through
+ * the wave's own LDS, no barrier), four to a CU with one copy of the weights
+ * (eight halve the registers and spill: 3 % slower), and a wave keeps its weight gradients in 160 accumulators over
+ * all of its tiles: 256 partial gradients of 36 KB a step, whatever the
+ * batch.  The sums over the four waves rotate through the parameters' eight
+ * parts, in an order that depends on nothing.  Measured, batch 65 536: step
+ * TRAIN_US us with its reduction and Adam, against 105 for one block per 64
+ * samples that wrote 1024 partial gradients, a reduction of 37 MB and Adam. */
+__global__ void __launch_bounds__(TWAVES * 64, 1) k_mlp_train_step(
+    const float *__restrict__ X, const float *__restrict__ Y, long long n, long long first, unsigned long long mul,
+    unsigned long long add, long long stride, int tiles, float inv_batch, DevMLPW w, float *__restrict__ partial,
+    float *__restrict__ loss) {
+    __shared__ __attribute__((aligned(16))) unsigned short sW[LDS_ALL];
+    __shared__ float sB[MLP_BP_TOTAL];
+    __shared__ __attribute__((aligned(16))) unsigned short sA[TWAVES * TWAVE_LDS];
+    __shared__ float sLoss[TWAVES];
+    static_assert(TWAVES == 4 && sizeof(unsigned short) * TWAVES * TWAVE_LDS >= sizeof(float) * MLP_NPARAMS,
+                  "the gradients' sums");
+    load_weights(w, sW, sB, MLP_WP_TOTAL);
+    const int l = threadIdx.x & 63, r = l & 15, q = l >> 4, wv = threadIdx.x >> 6;
+    unsigned short *H1s = sA + wv * TWAVE_LDS, *H2s = H1s + 64 * TS16, *H3s = H2s + 64 * TS16, *Ds = H3s + 64 * TS16,
+                   *Xs = Ds + 64 * TS16, *D4s = Xs + 16 * TS16;
+    f32x4 g1[4] = {}, g2[4][4] = {}, g3[4][4] = {}, g4[4] = {};
+    float gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f, gb4 = 0.0f, se = 0.0f;
+    int tile = blockIdx.x * TWAVES + wv;
+    long long idx = sample_index(first + 16LL * tile + r, n, mul, add);
+    float f[4], tgt[2] = {0.0f, 0.0f};
+    auto fetch = [&] {
+#pragma unroll
+        for (int j = 0; j < 4; j++) f[j] = 4 * q + j < MLP_IN ? X[idx * MLP_IN + 4 * q + j] : 0.0f;
+        if (q == 0) {
+            tgt[0] = Y[idx * 2];
+            tgt[1] = Y[idx * 2 + 1];
+        }
+    };
+    if (tile < tiles) fetch();
+    __syncthreads();
+    for (; tile < tiles; tile += gridDim.x * TWAVES) {
+        bf16x4 x;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            x[j] = (short)f2bf(f[j]);
+            Xs[(4 * q + j) * TS16 + r] = (unsigned short)x[j];
+        }
+        const float t0 = tgt[0], t1 = tgt[1];
+        idx += stride; /* the wave's next tile, read ahead */
+        if (idx >= n) idx -= n;
+        if (tile + (int)gridDim.x * TWAVES < tiles) fetch();
+
+        /* forward; z1..z3 become the activations' derivatives */
+        f32x4 z1[4], z2[4], z3[4], y;
+        bf16x4 h[4];
+        dense<4, 1>(sW + LDS_W1, LS16, &x, sB, z1);
+        train_act(z1, h, H1s);
+        dense<4, 4>(sW + LDS_W2, LS64, h, sB + 64, z2);
+        train_act(z2, h, H2s);
+        dense<4, 4>(sW + LDS_W3, LS64, h, sB + 128, z3);
+        train_act(z3, h, H3s);
+        dense<1, 4>(sW + LDS_W4, LS64, h, sB + 192, &y);
+
+        /* loss and output gradient (rows 0, 1 in lanes q == 0) */
+        f32x4 d[4] = {};
+        bf16x4 bd[4];
+        if (q == 0) {
+            const float e0 = y[0] - t0, e1 = y[1] - t1;
+            se += e0 * e0 + e1 * e1;
+            d[0][0] = e0 * inv_batch;
+            d[0][1] = e1 * inv_batch;
+        }
+        bd[0] = pack4(d[0]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) D4s[(4 * q + i) * TS16 + r] = (unsigned short)bd[0][i];
+        __builtin_amdgcn_wave_barrier();
+        {
+            float sum = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 16; k += 4) {
+                const bf16x4 v = lds4(D4s + r * TS16 + k);
+#pragma unroll
+                for (int i = 0; i < 4; i++) sum += bf2f((unsigned short)v[i]);
+            }
+            gb4 += sum;
+            const bf16x4 a = lds4(D4s + r * TS16 + 4 * q);
+#pragma unroll
+            for (int nt = 0; nt < 4; nt++) g4[nt] = mfma(a, lds4(H3s + (16 * nt + r) * TS16 + 4 * q), g4[nt]);
+        }
+        /* backward through the hidden layers */
+        dense<4, 1, false>(sW + LDS_W4T, LS16, bd, nullptr, d);
+        train_grad(d, z3, bd, Ds, &gb3);
+#pragma unroll
+        for (int mt = 0; mt < 4; mt++) {
+            const bf16x4 a = lds4(Ds + (16 * mt + r) * TS16 + 4 * q);
+#pragma unroll
+            for (int nt = 0; nt < 4; nt++) g3[mt][nt] = mfma(a, lds4(H2s + (16 * nt + r) * TS16 + 4 * q), g3[mt][nt]);
+        }
+        dense<4, 4, false>(sW + LDS_W3T, LS64, bd, nullptr, d);
+        train_grad(d, z2, bd, Ds, &gb2);
+#pragma unroll
+        for (int mt = 0; mt < 4; mt++) {
+            const bf16x4 a = lds4(Ds + (16 * mt + r) * TS16 + 4 * q);
+#pragma unroll
+            for (int nt = 0; nt < 4; nt++) g2[mt][nt] = mfma(a, lds4(H1s + (16 * nt + r) * TS16 + 4 * q), g2[mt][nt]);
+        }
+        dense<4, 4, false>(sW + LDS_W2T, LS64, bd, nullptr, d);
+        train_grad(d, z1, bd, Ds, &gb1);
+        const bf16x4 xt = lds4(Xs + r * TS16 + 4 * q);
+#pragma unroll
+        for (int mt = 0; mt < 4; mt++) g1[mt] = mfma(lds4(Ds + (16 * mt + r) * TS16 + 4 * q), xt, g1[mt]);
+        __builtin_amdgcn_wave_barrier();
+    }
+
+    /* the block's gradient: wave wv adds part (2 wv + k) mod 8 in round k (the
+     * first two rounds are the first to touch a part) */
+    float *sum = (float *)sA;
+#pragma unroll 1
+    for (int k = 0; k < 8; k++) {
+        __syncthreads();
+        const int part = (2 * wv + k) & 7;
+        auto put = [&](int p, float v) { sum[p] = k > 1 ? sum[p] + v : v; };
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            if (part == c) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int row = 16 * c + 4 * q + i;
+                    if (r < MLP_IN) put(MLP_OFF_W1 + row * MLP_IN + r, g1[c][i]);
+#pragma unroll
+                    for (int nt = 0; nt < 4; nt++) put(MLP_OFF_W2 + row * 64 + 16 * nt + r, g2[c][nt][i]);
+                }
+            }
+            if (part == c + 4) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int row = 16 * c + 4 * q + i;
+#pragma unroll
+                    for (int nt = 0; nt < 4; nt++) put(MLP_OFF_W3 + row * 64 + 16 * nt + r, g3[c][nt][i]);
+                }
+                if (q == 0) {
+                    put(MLP_OFF_W4 + 16 * c + r, g4[c][0]);
+                    put(MLP_OFF_W4 + 64 + 16 * c + r, g4[c][1]);
+                }
+            }
+        }
+        if (part == 0) put(MLP_OFF_B1 + l, gb1);
+        if (part == 1) put(MLP_OFF_B2 + l, gb2);
+        if (part == 2) put(MLP_OFF_B3 + l, gb3);
+        if (part == 3 && l < MLP_OUT) put(MLP_OFF_B4 + l, gb4);
+    }
     for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o, 64);
     if (l == 0) sLoss[wv] = se;
-
-    /* backward through the hidden layers */
-    f32x4 d[4];
-    bf16x4 bd[4];
-    bd[0] = pack4(dz4);
-    dense<4, 1, false>(sW + LDS_W4T, LS16, bd, nullptr, d);
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) d[mt][i] *= dsilu(z3[mt][i]);
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++) {
-        bd[mt] = pack4(d[mt]);
-#pragma unroll
-        for (int i = 0; i < 4; i++) D3s[(16 * mt + 4 * q + i) * AS + s] = (unsigned short)bd[mt][i];
-    }
-    dense<4, 4, false>(sW + LDS_W3T, LS64, bd, nullptr, d);
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) d[mt][i] *= dsilu(z2[mt][i]);
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++) {
-        bd[mt] = pack4(d[mt]);
-#pragma unroll
-        for (int i = 0; i < 4; i++) D2s[(16 * mt + 4 * q + i) * AS + s] = (unsigned short)bd[mt][i];
-    }
-    dense<4, 4, false>(sW + LDS_W2T, LS64, bd, nullptr, d);
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) D1s[(16 * mt + 4 * q + i) * AS + s] = f2bf(d[mt][i] * dsilu(z1[mt][i]));
     __syncthreads();
-
-    /* weight gradients, K = the block's 64 samples; wave wv owns output rows
-     * 16 wv .. 16 wv + 15 of W1..W3 and input columns 16 wv .. of W4 */
     float *P = partial + (size_t)blockIdx.x * MLP_NPARAMS;
-    {
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++)
-            acc = mfma(lds4(D1s + (16 * wv + r) * AS + 16 * ks + 4 * q), lds4(Xs + r * AS + 16 * ks + 4 * q), acc);
-        if (r < MLP_IN)
-#pragma unroll
-            for (int i = 0; i < 4; i++) P[MLP_OFF_W1 + (16 * wv + 4 * q + i) * MLP_IN + r] = acc[i];
+    for (int p = threadIdx.x; p < MLP_NPARAMS; p += TWAVES * 64) P[p] = sum[p];
+    if (threadIdx.x == 0) {
+        float s = 0.0f;
+        for (int i = 0; i < TWAVES; i++) s += sLoss[i];
+        loss[blockIdx.x] = s;
     }
-#pragma unroll
-    for (int layer = 0; layer < 2; layer++) {
-        const unsigned short *Dz = layer == 0 ? D2s : D3s;
-        const unsigned short *Hin = layer == 0 ? H1s : H2s;
-        const int off = layer == 0 ? MLP_OFF_W2 : MLP_OFF_W3;
-#pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
-            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++)
-                acc = mfma(lds4(Dz + (16 * wv + r) * AS + 16 * ks + 4 * q),
-                           lds4(Hin + (16 * nt + r) * AS + 16 * ks + 4 * q), acc);
-#pragma unroll
-            for (int i = 0; i < 4; i++) P[off + (16 * wv + 4 * q + i) * 64 + 16 * nt + r] = acc[i];
-        }
-    }
-    {
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++)
-            acc = mfma(lds4(D4s + r * AS + 16 * ks + 4 * q), lds4(H3s + (16 * wv + r) * AS + 16 * ks + 4 * q), acc);
-        if (q == 0) {
-            P[MLP_OFF_W4 + 0 * 64 + 16 * wv + r] = acc[0];
-            P[MLP_OFF_W4 + 1 * 64 + 16 * wv + r] = acc[1];
-        }
-    }
-    /* bias gradients: row sums of the staged output gradients */
-    for (int o = threadIdx.x; o < 3 * 64 + MLP_OUT; o += TBLK) {
-        const unsigned short *row = o < 64 ? D1s + o * AS : o < 128 ? D2s + (o - 64) * AS
-                                  : o < 192 ? D3s + (o - 128) * AS : D4s + (o - 192) * AS;
-        float acc = 0.0f;
-        for (int j = 0; j < TSAMP; j++) acc += bf2f(row[j]);
-        const int dst = o < 64 ? MLP_OFF_B1 + o : o < 128 ? MLP_OFF_B2 + o - 64 : o < 192 ? MLP_OFF_B3 + o - 128
-                                                                                           : MLP_OFF_B4 + o - 192;
-        P[dst] = acc;
-    }
-    if (threadIdx.x == 0) loss[blockIdx.x] = sLoss[0] + sLoss[1] + sLoss[2] + sLoss[3];
 }
 
-/* g[p] = sum over blocks of partial[block][p]; loss_acc += sum of the
- * block losses.  A block reduces 64 parameters: its four waves take every
- * fourth partial (four independent accumulators each), then the slices are
- * added in a fixed order, so the result does not depend on scheduling. */
+/* Adam (Kingma & Ba 2015) on an FP32 master weight; refreshes the BF16
+ * kernel copies */
+struct AdamStep {
+    float *w, *m, *v;
+    float lr, b1, b2, eps, c1, c2;
+    unsigned short *wp;
+    float *bp;
+};
+__device__ __forceinline__ void adam_param(const AdamStep &a, int p, float gp) {
+    const float mp = a.b1 * a.m[p] + (1.0f - a.b1) * gp;
+    const float vp = a.b2 * a.v[p] + (1.0f - a.b2) * gp * gp;
+    a.m[p] = mp;
+    a.v[p] = vp;
+    const float wn = a.w[p] - a.lr * (mp / a.c1) / (sqrtf(vp / a.c2) + a.eps);
+    a.w[p] = wn;
+    pack_param(p, wn, a.wp, a.bp);
+}
+
+/* g[p] = sum over blocks of partial[block][p]; loss_acc += sum of the block
+ * losses; with ADAM the parameters take their step at once.  A block reduces
+ * 64 parameters: its eight waves take every eighth partial (four independent
+ * accumulators each), then the slices are added in a fixed order, so the
+ * result does not depend on scheduling. */
 #define RED_P 64
-__global__ void __launch_bounds__(256) k_mlp_reduce(const float *__restrict__ partial, int nblocks,
-                                                    float *__restrict__ g, const float *__restrict__ loss,
-                                                    double *loss_acc) {
-    __shared__ float sp[4][RED_P];
+#define RED_W 8
+template <bool ADAM>
+__global__ void __launch_bounds__(RED_P *RED_W) k_mlp_reduce(const float *__restrict__ partial, int nblocks,
+                                                             float *__restrict__ g, const float *__restrict__ loss,
+                                                             double *loss_acc, AdamStep adam) {
+    __shared__ float sp[RED_W][RED_P];
     const int pl = threadIdx.x & (RED_P - 1), sl = threadIdx.x >> 6;
     const int p = blockIdx.x * RED_P + pl;
-    float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (p < MLP_NPARAMS) {
         int b = sl;
-        for (; b + 12 < nblocks; b += 16) {
-            a0 += partial[(size_t)b * MLP_NPARAMS + p];
-            a1 += partial[(size_t)(b + 4) * MLP_NPARAMS + p];
-            a2 += partial[(size_t)(b + 8) * MLP_NPARAMS + p];
-            a3 += partial[(size_t)(b + 12) * MLP_NPARAMS + p];
+        for (; b + 7 * RED_W < nblocks; b += 8 * RED_W) {
+            float x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[u] = partial[(size_t)(b + u * RED_W) * MLP_NPARAMS + p];
+#pragma unroll
+            for (int u = 0; u < 8; u++) a[u & 3] += x[u];
         }
-        for (; b < nblocks; b += 4) a0 += partial[(size_t)b * MLP_NPARAMS + p];
+        for (; b < nblocks; b += RED_W) a[0] += partial[(size_t)b * MLP_NPARAMS + p];
     }
-    sp[sl][pl] = (a0 + a1) + (a2 + a3);
+    sp[sl][pl] = (a[0] + a[1]) + (a[2] + a[3]);
     __syncthreads();
-    if (sl == 0 && p < MLP_NPARAMS) g[p] = (sp[0][pl] + sp[1][pl]) + (sp[2][pl] + sp[3][pl]);
-    if (blockIdx.x == 0 && loss_acc) {
-        __shared__ double sl_[256];
+    if (sl == 0 && p < MLP_NPARAMS) {
+        float s = 0.0f;
+#pragma unroll
+        for (int k = 0; k < RED_W; k++) s += sp[k][pl];
+        g[p] = s;
+        if (ADAM) adam_param(adam, p, s);
+    }
+    if (blockIdx.x == 0 && sl == 1 && loss_acc) {
         double s = 0.0;
-        for (int b = threadIdx.x; b < nblocks; b += 256) s += loss[b];
-        sl_[threadIdx.x] = s;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double t = 0.0;
-            for (int i = 0; i < 256; i++) t += sl_[i];
-            *loss_acc += t;
-        }
+        for (int b = pl; b < nblocks; b += 64) s += loss[b];
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        if (pl == 0) *loss_acc += s;
     }
 }
 
-/* Adam (Kingma & Ba 2015) on the FP32 master weights; refreshes the BF16
- * kernel copies */
-__global__ void k_mlp_adam(float *__restrict__ w, float *__restrict__ m, float *__restrict__ v,
-                           const float *__restrict__ g, float lr, float b1, float b2, float eps, float c1, float c2,
-                           unsigned short *wp, float *bp) {
+__global__ void k_mlp_adam(AdamStep a, const float *__restrict__ g) {
     const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= MLP_NPARAMS) return;
-    const float gp = g[p];
-    const float mp = b1 * m[p] + (1.0f - b1) * gp;
-    const float vp = b2 * v[p] + (1.0f - b2) * gp * gp;
-    m[p] = mp;
-    v[p] = vp;
-    const float wn = w[p] - lr * (mp / c1) / (sqrtf(vp / c2) + eps);
-    w[p] = wn;
-    pack_param(p, wn, wp, bp);
+    if (p < MLP_NPARAMS) adam_param(a, p, g[p]);
 }
 
 /* forward pass over stored samples (outputs Y[n][2]) */
@@ -783,25 +868,44 @@ extern "C" int mdz_mlp_download_samples(mdz_mlp *n, long long first, long long c
     return MDZ_OK;
 }
 
-/* gradient of sum((y-t)^2) / (2 * count) over the stored samples [first, first + count) */
+/* the constants of the network's next Adam step */
+static AdamStep adam_step(mdz_mlp *n, float lr) {
+    n->t++;
+    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+    return AdamStep{n->w, n->m, n->v, lr, b1, b2, eps, 1.0f - powf(b1, (float)n->t), 1.0f - powf(b2, (float)n->t),
+                    n->wp, n->bp};
+}
+
+/* gradient of sum((y-t)^2) / (2 * count) over the stored samples [first,
+ * first + count), with an Adam step of rate *lr where lr is not null */
 static int mlp_gradient(mdz_mlp *n, long long first, int count, unsigned long long mul, unsigned long long add,
-                        double *loss_acc) {
+                        double *loss_acc, const float *lr) {
     if (count < TSAMP || count % TSAMP) return mdz_error(MDZ_EINVAL, "batch must be a multiple of 64");
-    const int nb = count / TSAMP;
+    const int tiles = count / 16, nb = std::min(TBLOCKS, mdz_div_up(tiles, TWAVES));
     if (nb > n->partial_blocks) {
         hipFree(n->partial);
         hipFree(n->loss);
         n->partial = nullptr;
         n->loss = nullptr;
+        n->partial_blocks = 0;
         MCHK(hipMalloc((void **)&n->partial, (size_t)nb * MLP_NPARAMS * 4));
         MCHK(hipMalloc((void **)&n->loss, (size_t)nb * 4));
         n->partial_blocks = nb;
     }
     DevMLPW w{n->wp, n->bp};
-    hipLaunchKernelGGL(k_mlp_train_step, dim3(nb), dim3(TBLK), 0, n->s, (const float *)n->X, (const float *)n->Y, n->n,
-                       first, mul, add, 1.0f / (float)count, w, n->partial, n->loss);
-    hipLaunchKernelGGL(k_mlp_reduce, dim3(mdz_div_up(MLP_NPARAMS, RED_P)), dim3(256), 0, n->s, (const float *)n->partial,
-                       nb, n->g, (const float *)n->loss, loss_acc);
+    /* from one tile of a wave to its next: 16 nb TWAVES samples on */
+    const unsigned long long un = (unsigned long long)n->n;
+    const long long stride = (long long)(((unsigned long long)(16LL * nb * TWAVES) % un) * (mul % un) % un);
+    hipLaunchKernelGGL(k_mlp_train_step, dim3(nb), dim3(TWAVES * 64), 0, n->s, (const float *)n->X, (const float *)n->Y,
+                       n->n, first, mul, add, stride, tiles, 1.0f / (float)count, w, n->partial, n->loss);
+    const dim3 grid(mdz_div_up(MLP_NPARAMS, RED_P)), blk(RED_P * RED_W);
+    const AdamStep as = lr ? adam_step(n, *lr) : AdamStep{};
+    if (lr)
+        hipLaunchKernelGGL(k_mlp_reduce<true>, grid, blk, 0, n->s, (const float *)n->partial, nb, n->g,
+                           (const float *)n->loss, loss_acc, as);
+    else
+        hipLaunchKernelGGL(k_mlp_reduce<false>, grid, blk, 0, n->s, (const float *)n->partial, nb, n->g,
+                           (const float *)n->loss, loss_acc, as);
     MCHK(hipGetLastError());
     return MDZ_OK;
 }
@@ -809,7 +913,7 @@ static int mlp_gradient(mdz_mlp *n, long long first, int count, unsigned long lo
 extern "C" int mdz_mlp_gradient(mdz_mlp *n, long long first, int count, float *grad, double *loss) {
     if (!n || first < 0 || first + count > n->n) return mdz_error(MDZ_EINVAL, "mdz_mlp_gradient: range");
     MCHK(hipMemsetAsync(n->loss_acc, 0, 8, n->s));
-    int rc = mlp_gradient(n, first, count, 1ULL, 0ULL, n->loss_acc);
+    int rc = mlp_gradient(n, first, count, 1ULL, 0ULL, n->loss_acc, nullptr);
     if (rc) return rc;
     if (grad) MCHK(hipMemcpyAsync(grad, n->g, MLP_NPARAMS * 4, hipMemcpyDeviceToHost, n->s));
     if (loss) MCHK(hipMemcpyAsync(loss, n->loss_acc, 8, hipMemcpyDeviceToHost, n->s));
@@ -817,22 +921,13 @@ extern "C" int mdz_mlp_gradient(mdz_mlp *n, long long first, int count, float *g
     return MDZ_OK;
 }
 
-static int mlp_adam(mdz_mlp *n, float lr) {
-    n->t++;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float c1 = 1.0f - powf(b1, (float)n->t), c2 = 1.0f - powf(b2, (float)n->t);
-    hipLaunchKernelGGL(k_mlp_adam, dim3(mdz_div_up(MLP_NPARAMS, 256)), dim3(256), 0, n->s, n->w, n->m, n->v,
-                       (const float *)n->g, lr, b1, b2, eps, c1, c2, n->wp, n->bp);
-    MCHK(hipGetLastError());
-    return MDZ_OK;
-}
-
 /* one Adam step with a caller-supplied gradient */
 extern "C" int mdz_mlp_adam_step(mdz_mlp *n, const float *grad, float lr) {
     if (!n || !grad) return mdz_error(MDZ_EINVAL, "mdz_mlp_adam_step");
     MCHK(hipMemcpyAsync(n->g, grad, MLP_NPARAMS * 4, hipMemcpyHostToDevice, n->s));
-    int rc = mlp_adam(n, lr);
-    if (rc) return rc;
+    hipLaunchKernelGGL(k_mlp_adam, dim3(mdz_div_up(MLP_NPARAMS, 256)), dim3(256), 0, n->s, adam_step(n, lr),
+                       (const float *)n->g);
+    MCHK(hipGetLastError());
     MCHK(hipStreamSynchronize(n->s));
     return MDZ_OK;
 }
@@ -859,9 +954,7 @@ extern "C" int mdz_mlp_train(mdz_mlp *n, int epochs, int batch, float lr, unsign
         const unsigned long long add = (st >> 7) % (unsigned long long)n->n;
         MCHK(hipMemsetAsync(n->loss_acc, 0, 8, n->s));
         for (long long k = 0; k < steps; k++) {
-            int rc = mlp_gradient(n, k * batch, batch, mul, add, n->loss_acc);
-            if (rc) return rc;
-            rc = mlp_adam(n, lr);
+            int rc = mlp_gradient(n, k * batch, batch, mul, add, n->loss_acc, &lr);
             if (rc) return rc;
         }
         double acc = 0.0;
