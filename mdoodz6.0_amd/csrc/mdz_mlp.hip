@@ -263,67 +263,118 @@ __device__ __forceinline__ long long sample_index(long long j, long long n, unsi
     return (long long)((((unsigned long long)j % (unsigned long long)n) * mul + add) % (unsigned long long)n);
 }
 
-#define TWAVES 4                 /* waves of a training block, each on its own 16 samples at a time */
+#define TWAVES 4                 /* waves of a training block, each on its own 32 samples at a time */
 #define TBLOCKS 256              /* most training blocks: one per CU */
-#define TS16 20                  /* row stride of 16 staged samples */
-#define TWAVE_LDS (4 * 64 * TS16 + 2 * 16 * TS16) /* H1 H2 H3 D, X D4 */
+#define TSW 36                   /* row stride of 32 staged samples */
+#define TWAVE_LDS (4 * 64 * TSW + 2 * 16 * TSW) /* H1 H2 H3 D, X D4 */
 
-/* a hidden layer's activations and their derivative, the activations also
- * staged [row][sample] for the weight gradient */
-__device__ __forceinline__ void train_act(f32x4 *z, bf16x4 *h, unsigned short *Hs) {
+/* dense() of two groups of 16 samples, the weights read once */
+template <int NM, int NK, bool BIAS>
+__device__ __forceinline__ void dense_x2(const unsigned short *W, int ldw, const bf16x4 (*b)[NK], const float *bias,
+                                         f32x4 (*z)[4]) {
     const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-        f32x4 v;
+    for (int mt = 0; mt < NM; mt++) {
+        f32x4 acc[2] = {};
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float s = sigmoidf_(z[t][i]);
-            v[i] = z[t][i] * s;
-            z[t][i] = s * (1.0f + z[t][i] * (1.0f - s));
+        for (int ks = 0; ks < NK; ks++) {
+            const bf16x4 a = lds4(W + (16 * mt + r) * ldw + 16 * ks + 4 * q);
+#pragma unroll
+            for (int g = 0; g < 2; g++) acc[g] = mfma(a, b[g][ks], acc[g]);
         }
-        h[t] = pack4(v);
 #pragma unroll
-        for (int i = 0; i < 4; i++) Hs[(16 * t + 4 * q + i) * TS16 + r] = (unsigned short)h[t][i];
+        for (int g = 0; g < 2; g++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) z[g][mt][i] = BIAS ? acc[g][i] + bias[16 * mt + 4 * q + i] : acc[g][i];
     }
 }
 
-/* a hidden layer's output gradients d (times the activation's derivative),
- * rounded and staged; the sum of row l over the samples is added to *bias */
-__device__ __forceinline__ void train_grad(const f32x4 *d, const f32x4 *dact, bf16x4 *bd, unsigned short *Ds,
-                                           float *bias) {
+/* 8 staged samples of a row: the lane's operand of a 16 x 16 x 32 product */
+__device__ __forceinline__ bf16x8 lds8(const unsigned short *p) {
+    const bf16x4 a = lds4(p), b = lds4(p + 4);
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+/* a hidden layer's activations and (in z) their derivative, the activations
+ * also staged [row][sample] for the weight gradient */
+__device__ __forceinline__ void train_act(f32x4 (*z)[4], bf16x4 (*h)[4], unsigned short *Hs) {
     const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-        bd[t] = pack4(d[t] * dact[t]);
+    for (int g = 0; g < 2; g++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) Ds[(16 * t + 4 * q + i) * TS16 + r] = (unsigned short)bd[t][i];
-    }
-    __builtin_amdgcn_wave_barrier();
+        for (int t = 0; t < 4; t++) {
+            f32x4 v;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float s = sigmoidf_(z[g][t][i]);
+                v[i] = z[g][t][i] * s;
+                z[g][t][i] = s * (1.0f + z[g][t][i] * (1.0f - s));
+            }
+            h[g][t] = pack4(v);
+#pragma unroll
+            for (int i = 0; i < 4; i++) Hs[(16 * t + 4 * q + i) * TSW + 16 * g + r] = (unsigned short)h[g][t][i];
+        }
+}
+
+/* sum of a staged row over its 32 samples */
+__device__ __forceinline__ float row_sum(const unsigned short *row) {
     float sum = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 16; k += 4) {
-        const bf16x4 v = lds4(Ds + l * TS16 + k);
+    for (int k = 0; k < 32; k += 4) {
+        const bf16x4 v = lds4(row + k);
 #pragma unroll
         for (int i = 0; i < 4; i++) sum += bf2f((unsigned short)v[i]);
     }
-    *bias += sum;
+    return sum;
 }
 
-/* Forward and backward pass of `tiles` tiles of 16 samples, one wave per
+/* a hidden layer's output gradients d (times the activation's derivative),
+ * rounded and staged */
+__device__ __forceinline__ void train_grad(const f32x4 (*d)[4], const f32x4 (*dact)[4], bf16x4 (*bd)[4],
+                                           unsigned short *Ds) {
+    const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            bd[g][t] = pack4(d[g][t] * dact[g][t]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) Ds[(16 * t + 4 * q + i) * TSW + 16 * g + r] = (unsigned short)bd[g][t][i];
+        }
+    __builtin_amdgcn_wave_barrier();
+}
+
+/* g[mt][nt] += D H^T over the 32 staged samples */
+__device__ __forceinline__ void weight_grad(const unsigned short *Ds, const unsigned short *Hs, f32x4 (*g)[4]) {
+    const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
+    bf16x8 h[4];
+#pragma unroll
+    for (int nt = 0; nt < 4; nt++) h[nt] = lds8(Hs + (16 * nt + r) * TSW + 8 * q);
+#pragma unroll
+    for (int mt = 0; mt < 4; mt++) {
+        const bf16x8 a = lds8(Ds + (16 * mt + r) * TSW + 8 * q);
+#pragma unroll
+        for (int nt = 0; nt < 4; nt++) g[mt][nt] = mfma32(a, h[nt], g[mt][nt]);
+    }
+}
+
+/* Forward and backward pass of `tiles` tiles of 32 samples, one wave per
  * tile; partial[block][p]: the block's gradient of sum((y - t)^2) / (2
  * batch), loss[block]: its sum of squared errors.
  *
- * The matrix products of a tile are about 120 instructions; what bounds the
+ * The matrix products of a tile are about 200 instructions; what bounds the
  * kernel is the chain through the layers and what surrounds the samples.
  * So the waves are independent (a tile's activations are transposed through
- * the wave's own LDS, no barrier), four to a CU with one copy of the weights
- * (eight halve the registers and spill: 3 % slower), and a wave keeps its weight gradients in 160 accumulators over
- * all of its tiles: 256 partial gradients of 36 KB a step, whatever the
- * batch.  The sums over the four waves rotate through the parameters' eight
- * parts, in an order that depends on nothing.  Measured, batch 65 536: step
- * TRAIN_US us with its reduction and Adam, against 105 for one block per 64
- * samples that wrote 1024 partial gradients, a reduction of 37 MB and Adam. */
+ * the wave's own LDS, no barrier), two groups of 16 samples run through the
+ * layers side by side, four waves to a CU share one copy of the weights
+ * (eight halve the registers and spill), and a wave keeps its weight
+ * gradients in 160 accumulators over all of its tiles: 256 partial gradients
+ * of 36 KB a step, whatever the batch.  The sums over the four waves rotate
+ * through the parameters' eight parts, in an order that depends on nothing.
+ * Measured, batch 65 536: a step 43 us with its reduction and Adam (47 with
+ * one group a wave), against 105 for one block per 64 samples that wrote
+ * 1024 partial gradients, a reduction of 37 MB and Adam. */
 __global__ void __launch_bounds__(TWAVES * 64, 1) k_mlp_train_step(
     const float *__restrict__ X, const float *__restrict__ Y, long long n, long long first, unsigned long long mul,
     unsigned long long add, long long stride, int tiles, float inv_batch, DevMLPW w, float *__restrict__ partial,
@@ -334,96 +385,114 @@ __global__ void __launch_bounds__(TWAVES * 64, 1) k_mlp_train_step(
     __shared__ float sLoss[TWAVES];
     static_assert(TWAVES == 4 && sizeof(unsigned short) * TWAVES * TWAVE_LDS >= sizeof(float) * MLP_NPARAMS,
                   "the gradients' sums");
-    load_weights(w, sW, sB, MLP_WP_TOTAL);
     const int l = threadIdx.x & 63, r = l & 15, q = l >> 4, wv = threadIdx.x >> 6;
-    unsigned short *H1s = sA + wv * TWAVE_LDS, *H2s = H1s + 64 * TS16, *H3s = H2s + 64 * TS16, *Ds = H3s + 64 * TS16,
-                   *Xs = Ds + 64 * TS16, *D4s = Xs + 16 * TS16;
+    /* (all reads of the weights and of the first samples in flight at once:
+     * one round trip instead of ten) */
+    constexpr int WL = (MLP_WP_TOTAL / 8 + TWAVES * 64 - 1) / (TWAVES * 64);
+    uint4 wl[WL];
+#pragma unroll
+    for (int k = 0; k < WL; k++)
+        wl[k] = ((const uint4 *)w.wp)[min((int)threadIdx.x + k * TWAVES * 64, MLP_WP_TOTAL / 8 - 1)];
+    const float bl = w.bp[min((int)threadIdx.x, MLP_BP_TOTAL - 1)];
+    unsigned short *H1s = sA + wv * TWAVE_LDS, *H2s = H1s + 64 * TSW, *H3s = H2s + 64 * TSW, *Ds = H3s + 64 * TSW,
+                   *Xs = Ds + 64 * TSW, *D4s = Xs + 16 * TSW;
     f32x4 g1[4] = {}, g2[4][4] = {}, g3[4][4] = {}, g4[4] = {};
     float gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f, gb4 = 0.0f, se = 0.0f;
     int tile = blockIdx.x * TWAVES + wv;
-    long long idx = sample_index(first + 16LL * tile + r, n, mul, add);
-    float f[4], tgt[2] = {0.0f, 0.0f};
+    long long idx[2];
+    float f[2][4], tgt[2][2] = {};
+#pragma unroll
+    for (int g = 0; g < 2; g++) idx[g] = sample_index(first + 32LL * tile + 16 * g + r, n, mul, add);
     auto fetch = [&] {
 #pragma unroll
-        for (int j = 0; j < 4; j++) f[j] = 4 * q + j < MLP_IN ? X[idx * MLP_IN + 4 * q + j] : 0.0f;
-        if (q == 0) {
-            tgt[0] = Y[idx * 2];
-            tgt[1] = Y[idx * 2 + 1];
+        for (int g = 0; g < 2; g++) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) f[g][j] = 4 * q + j < MLP_IN ? X[idx[g] * MLP_IN + 4 * q + j] : 0.0f;
+            if (q == 0) {
+                tgt[g][0] = Y[idx[g] * 2];
+                tgt[g][1] = Y[idx[g] * 2 + 1];
+            }
         }
     };
     if (tile < tiles) fetch();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < WL; k++) {
+        const int i = threadIdx.x + k * TWAVES * 64;
+        if (i < MLP_WP_TOTAL / 8) {
+            uint2 *o = (uint2 *)(sW + lds_index(8 * i));
+            o[0] = uint2{wl[k].x, wl[k].y};
+            o[1] = uint2{wl[k].z, wl[k].w};
+        }
+    }
+    static_assert(MLP_BP_TOTAL <= TWAVES * 64, "one bias a thread");
+    if (threadIdx.x < MLP_BP_TOTAL) sB[threadIdx.x] = bl;
     __syncthreads();
     for (; tile < tiles; tile += gridDim.x * TWAVES) {
-        bf16x4 x;
+        bf16x4 x[2][1];
+        float t[2][2];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            x[j] = (short)f2bf(f[j]);
-            Xs[(4 * q + j) * TS16 + r] = (unsigned short)x[j];
+        for (int g = 0; g < 2; g++) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                x[g][0][j] = (short)f2bf(f[g][j]);
+                Xs[(4 * q + j) * TSW + 16 * g + r] = (unsigned short)x[g][0][j];
+            }
+            t[g][0] = tgt[g][0];
+            t[g][1] = tgt[g][1];
+            idx[g] += stride; /* the wave's next tile, read ahead */
+            if (idx[g] >= n) idx[g] -= n;
         }
-        const float t0 = tgt[0], t1 = tgt[1];
-        idx += stride; /* the wave's next tile, read ahead */
-        if (idx >= n) idx -= n;
         if (tile + (int)gridDim.x * TWAVES < tiles) fetch();
 
         /* forward; z1..z3 become the activations' derivatives */
-        f32x4 z1[4], z2[4], z3[4], y;
-        bf16x4 h[4];
-        dense<4, 1>(sW + LDS_W1, LS16, &x, sB, z1);
+        f32x4 z1[2][4], z2[2][4], z3[2][4], d[2][4];
+        bf16x4 h[2][4];
+        dense_x2<4, 1, true>(sW + LDS_W1, LS16, x, sB, z1);
         train_act(z1, h, H1s);
-        dense<4, 4>(sW + LDS_W2, LS64, h, sB + 64, z2);
+        dense_x2<4, 4, true>(sW + LDS_W2, LS64, h, sB + 64, z2);
         train_act(z2, h, H2s);
-        dense<4, 4>(sW + LDS_W3, LS64, h, sB + 128, z3);
+        dense_x2<4, 4, true>(sW + LDS_W3, LS64, h, sB + 128, z3);
         train_act(z3, h, H3s);
-        dense<1, 4>(sW + LDS_W4, LS64, h, sB + 192, &y);
+        dense_x2<1, 4, true>(sW + LDS_W4, LS64, h, sB + 192, d);
 
         /* loss and output gradient (rows 0, 1 in lanes q == 0) */
-        f32x4 d[4] = {};
-        bf16x4 bd[4];
-        if (q == 0) {
-            const float e0 = y[0] - t0, e1 = y[1] - t1;
-            se += e0 * e0 + e1 * e1;
-            d[0][0] = e0 * inv_batch;
-            d[0][1] = e1 * inv_batch;
-        }
-        bd[0] = pack4(d[0]);
+        bf16x4 b4[2][1], bd[2][4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) D4s[(4 * q + i) * TS16 + r] = (unsigned short)bd[0][i];
-        __builtin_amdgcn_wave_barrier();
-        {
-            float sum = 0.0f;
-#pragma unroll
-            for (int k = 0; k < 16; k += 4) {
-                const bf16x4 v = lds4(D4s + r * TS16 + k);
-#pragma unroll
-                for (int i = 0; i < 4; i++) sum += bf2f((unsigned short)v[i]);
+        for (int g = 0; g < 2; g++) {
+            f32x4 e = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (q == 0) {
+                const float e0 = d[g][0][0] - t[g][0], e1 = d[g][0][1] - t[g][1];
+                se += e0 * e0 + e1 * e1;
+                e[0] = e0 * inv_batch;
+                e[1] = e1 * inv_batch;
             }
-            gb4 += sum;
-            const bf16x4 a = lds4(D4s + r * TS16 + 4 * q);
+            b4[g][0] = pack4(e);
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) g4[nt] = mfma(a, lds4(H3s + (16 * nt + r) * TS16 + 4 * q), g4[nt]);
+            for (int i = 0; i < 4; i++) D4s[(4 * q + i) * TSW + 16 * g + r] = (unsigned short)b4[g][0][i];
+        }
+        __builtin_amdgcn_wave_barrier();
+        gb4 += row_sum(D4s + r * TSW);
+        {
+            const bf16x8 a = lds8(D4s + r * TSW + 8 * q);
+#pragma unroll
+            for (int nt = 0; nt < 4; nt++) g4[nt] = mfma32(a, lds8(H3s + (16 * nt + r) * TSW + 8 * q), g4[nt]);
         }
         /* backward through the hidden layers */
-        dense<4, 1, false>(sW + LDS_W4T, LS16, bd, nullptr, d);
-        train_grad(d, z3, bd, Ds, &gb3);
+        dense_x2<4, 1, false>(sW + LDS_W4T, LS16, b4, nullptr, d);
+        train_grad(d, z3, bd, Ds);
+        gb3 += row_sum(Ds + l * TSW);
+        weight_grad(Ds, H2s, g3);
+        dense_x2<4, 4, false>(sW + LDS_W3T, LS64, bd, nullptr, d);
+        train_grad(d, z2, bd, Ds);
+        gb2 += row_sum(Ds + l * TSW);
+        weight_grad(Ds, H1s, g2);
+        dense_x2<4, 4, false>(sW + LDS_W2T, LS64, bd, nullptr, d);
+        train_grad(d, z1, bd, Ds);
+        gb1 += row_sum(Ds + l * TSW);
+        const bf16x8 xt = lds8(Xs + r * TSW + 8 * q);
 #pragma unroll
-        for (int mt = 0; mt < 4; mt++) {
-            const bf16x4 a = lds4(Ds + (16 * mt + r) * TS16 + 4 * q);
-#pragma unroll
-            for (int nt = 0; nt < 4; nt++) g3[mt][nt] = mfma(a, lds4(H2s + (16 * nt + r) * TS16 + 4 * q), g3[mt][nt]);
-        }
-        dense<4, 4, false>(sW + LDS_W3T, LS64, bd, nullptr, d);
-        train_grad(d, z2, bd, Ds, &gb2);
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++) {
-            const bf16x4 a = lds4(Ds + (16 * mt + r) * TS16 + 4 * q);
-#pragma unroll
-            for (int nt = 0; nt < 4; nt++) g2[mt][nt] = mfma(a, lds4(H1s + (16 * nt + r) * TS16 + 4 * q), g2[mt][nt]);
-        }
-        dense<4, 4, false>(sW + LDS_W2T, LS64, bd, nullptr, d);
-        train_grad(d, z1, bd, Ds, &gb1);
-        const bf16x4 xt = lds4(Xs + r * TS16 + 4 * q);
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++) g1[mt] = mfma(lds4(Ds + (16 * mt + r) * TS16 + 4 * q), xt, g1[mt]);
+        for (int mt = 0; mt < 4; mt++) g1[mt] = mfma32(lds8(Ds + (16 * mt + r) * TSW + 8 * q), xt, g1[mt]);
         __builtin_amdgcn_wave_barrier();
     }
 
@@ -881,7 +950,7 @@ static AdamStep adam_step(mdz_mlp *n, float lr) {
 static int mlp_gradient(mdz_mlp *n, long long first, int count, unsigned long long mul, unsigned long long add,
                         double *loss_acc, const float *lr) {
     if (count < TSAMP || count % TSAMP) return mdz_error(MDZ_EINVAL, "batch must be a multiple of 64");
-    const int tiles = count / 16, nb = std::min(TBLOCKS, mdz_div_up(tiles, TWAVES));
+    const int tiles = count / 32, nb = std::min(TBLOCKS, mdz_div_up(tiles, TWAVES));
     if (nb > n->partial_blocks) {
         hipFree(n->partial);
         hipFree(n->loss);
@@ -893,9 +962,9 @@ static int mlp_gradient(mdz_mlp *n, long long first, int count, unsigned long lo
         n->partial_blocks = nb;
     }
     DevMLPW w{n->wp, n->bp};
-    /* from one tile of a wave to its next: 16 nb TWAVES samples on */
+    /* from one tile of a wave to its next: 32 nb TWAVES samples on */
     const unsigned long long un = (unsigned long long)n->n;
-    const long long stride = (long long)(((unsigned long long)(16LL * nb * TWAVES) % un) * (mul % un) % un);
+    const long long stride = (long long)(((unsigned long long)(32LL * nb * TWAVES) % un) * (mul % un) % un);
     hipLaunchKernelGGL(k_mlp_train_step, dim3(nb), dim3(TWAVES * 64), 0, n->s, (const float *)n->X, (const float *)n->Y,
                        n->n, first, mul, add, stride, tiles, 1.0f / (float)count, w, n->partial, n->loss);
     const dim3 grid(mdz_div_up(MLP_NPARAMS, RED_P)), blk(RED_P * RED_W);
