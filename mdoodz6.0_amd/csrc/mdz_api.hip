@@ -1533,15 +1533,28 @@ extern "C" int mdz_ctx_markers_to_grid(mdz_ctx *c, grid *mesh, const markers *m,
     NodeAxes ac, av;
     if (!rc) rc = mdz_mstore_axes(c->ms, 0, mesh, nullptr, nullptr, periodic, c->stream, &ac);
     if (!rc) rc = mdz_mstore_axes(c->ms, 1, mesh, nullptr, nullptr, periodic, c->stream, &av);
-    if (!rc) rc = mdz_mstore_bin(c->ms, 0, ac, c->stream);
-    if (!rc) rc = mdz_mstore_bin(c->ms, 1, av, c->stream);
     if (rc) return rc;
     const int np = c->model.Nb_phases < c->nph ? c->model.Nb_phases : c->nph;
     const int itp = c->model.itp_stencil == 9 ? 9 : 1;
-    const MarkerDev &md = mdz_mstore_dev(c->ms);
-    mdz_launch_p2mastah(md, 0, ac, 1, itp, P2GArgs{0, 0, np, nullptr, nullptr, c->g.BCp, nullptr, c->g.phase_n}, c->stream);
-    mdz_launch_p2mastah(md, 1, av, 1, itp, P2GArgs{0, 0, np, nullptr, nullptr, c->g.BCg, nullptr, c->g.phase_s}, c->stream);
-    if ((rc = cfd_on_ctx(c, mesh, &c->materials, &c->model))) return rc;
+    /* the 1-node stencil takes one binning by quarter cell for both families
+     * where the centroids lie between the vertices, as on any grid of the
+     * reference */
+    const double sx = (mesh->xc_coord[0] - mesh->xg_coord[0]) / mesh->dx;
+    const double sz = (mesh->zc_coord[0] - mesh->zg_coord[0]) / mesh->dz;
+    if (itp == 1 && sx > 0.25 && sx < 0.75 && sz > 0.25 && sz < 0.75) {
+        const SoftK sk = mdz_soft_constants(&c->materials, np);
+        if ((rc = mdz_mstore_step(c->ms, ac, av, sk, c->g.phase_n, c->g.phase_s, c->g.BCp, c->g.BCg, c->g.fric_n,
+                                  c->g.dil_n, c->g.C_n, c->g.fric_s, c->g.dil_s, c->g.C_s, c->stream)))
+            return rc;
+    } else {
+        if ((rc = mdz_mstore_bin(c->ms, 0, ac, c->stream)) || (rc = mdz_mstore_bin(c->ms, 1, av, c->stream))) return rc;
+        const MarkerDev &md = mdz_mstore_dev(c->ms);
+        mdz_launch_p2mastah(md, 0, ac, 1, itp, P2GArgs{0, 0, np, nullptr, nullptr, c->g.BCp, nullptr, c->g.phase_n},
+                            c->stream);
+        mdz_launch_p2mastah(md, 1, av, 1, itp, P2GArgs{0, 0, np, nullptr, nullptr, c->g.BCg, nullptr, c->g.phase_s},
+                            c->stream);
+        if ((rc = cfd_on_ctx(c, mesh, &c->materials, &c->model))) return rc;
+    }
     HIPCHK(hipGetLastError());
     if (download) {
         const size_t nc = fam_len(MDZ_FAM_C, c->Nx, c->Nz), nv = fam_len(MDZ_FAM_V, c->Nx, c->Nz);

@@ -144,23 +144,27 @@ struct MarkerRec {
 
 /* Markers on the device and their bins by nearest node, per node family
  * (slot 0 centroids, 1 vertices, 2 Vx nodes, 3 Vz nodes, 4 the axes a
- * caller of Interp_P2N passes): rec[f] holds the marker records bin by bin,
- * increasing marker index within a bin (a stable sort); start[f][b] ..
+ * caller of Interp_P2N passes, 5 the quarter cells): rec[f] holds the marker records bin by bin,
+ * increasing marker index within a bin; start[f][b] ..
  * start[f][b + 1] is bin b. */
-#define MDZ_MARKER_FAMS 5
+#define MDZ_MARKER_FAMS 6
+#define MDZ_FAM_QUARTER 5
 struct MarkerDev {
     int n, cap;
     double *x, *z;
     int *phase;
     double *val;                   /* per-marker values of the current interpolation */
-    int *key, *key_out;            /* sort keys (bin of each marker) */
-    MarkerRec *rec_in;             /* sort input */
+    int *key, *key_out;            /* rank of each marker in its bin, or sort keys */
+    MarkerRec *rec_in;             /* records bin by bin in any order, or the sort's input */
     MarkerRec *rec[MDZ_MARKER_FAMS];
     int *start[MDZ_MARKER_FAMS];
     size_t start_cap[MDZ_MARKER_FAMS];
     int binned[MDZ_MARKER_FAMS];   /* node count of the last binning, 0 = none */
     void *tmp;
     size_t tmp_bytes;
+    int *scan;                     /* scratch of the bins' scan, then the flag of a long bin */
+    size_t scan_len;
+    int *long_bin;                 /* pinned copy of the flag */
     __host__ __device__ MarkerSet set() const { return MarkerSet{n, x, z, phase}; }
 };
 
@@ -184,9 +188,10 @@ struct SoftK {
     int phi_soft[MDZ_MAX_PHASES], psi_soft[MDZ_MAX_PHASES], coh_soft[MDZ_MAX_PHASES];
 };
 
-/* bins of family slot fam on axes a (needs start_cap[fam] >= nodes + 1 and
- * tmp_bytes >= mdz_markers_sort_bytes) */
-int mdz_markers_bin(MarkerDev &md, int fam, const NodeAxes &a, hipStream_t s);
+/* bins of family slot fam on axes a, or (fam = MDZ_FAM_QUARTER) of the
+ * quarter cells of centroid axes a and vertex axes *v (needs start_cap[fam]
+ * >= bins + 1 and tmp_bytes >= mdz_markers_sort_bytes); synchronises */
+int mdz_markers_bin(MarkerDev &md, int fam, const NodeAxes &a, const NodeAxes *v, hipStream_t s);
 size_t mdz_markers_sort_bytes(int n, int nodes);
 void mdz_launch_p2mastah(const MarkerDev &md, int fam, const NodeAxes &a, int prop, int itp_stencil,
                          const P2GArgs &g, hipStream_t s);
@@ -206,6 +211,11 @@ int mdz_mstore_axes(MarkerStore *s, int fam, const grid *mesh, const double *Xh,
 int mdz_mstore_upload(MarkerStore *s, const markers *m, const double *mval, int nph, hipStream_t st);
 int mdz_mstore_values(MarkerStore *s, const double *mval, hipStream_t st);
 int mdz_mstore_bin(MarkerStore *s, int fam, const NodeAxes &a, hipStream_t st);
+/* phase fractions and strength parameters of centroids and vertices, 1-node
+ * stencil, from the quarter cells' bins */
+int mdz_mstore_step(MarkerStore *s, const NodeAxes &ac, const NodeAxes &av, const SoftK &sk, double *perc_n,
+                    double *perc_s, const int8_t *BCp, const int8_t *BCg, double *fric_n, double *dil_n, double *C_n,
+                    double *fric_s, double *dil_s, double *C_s, hipStream_t st);
 void mdz_mstore_rebin(MarkerStore *s); /* the next binning of every family sorts again */
 MarkerDev &mdz_mstore_dev(MarkerStore *s);
 double *mdz_mstore_node_field(MarkerStore *s);
