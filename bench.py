@@ -39,29 +39,30 @@ def stage_kernels(shape, learned=False, fused=True, net_in_rheology=True):
     rh, pic, jac = shape
 
     def values(kind, rows, capa, capb):
-        # 64-row blocks: the split pass (tag-free waves, then the listed general waves)
+        # 64-row blocks: the split pass (the listed general waves, then the tag-free ones)
         if rows == 64:
-            return ["k_values_split<%d, %d, %d, false>" % (kind, capa, capb),
-                    "k_values_split<%d, %d, %d, true>" % (kind, capa, capb)]
+            return ["k_values_split<%d, %d, %d>" % (kind, capa, capb)]
         if rows:
             return ["k_values_mom<%d, %d, %d, %d>" % (kind, rows, capa, capb)]
         return ["k_values_mom_direct<%d>" % kind, "k_values_cont"]
 
     separate = learned and not net_in_rheology
     prep = ["k_mlp_guess", "k_guess_vertices"] if separate else []
-    d0 = [] if fused else ["k_dtensor_cells<0>", "k_dtensor_vertices<0>"]
-    d1 = ["k_dtensor_cells<2>", "k_dtensor_vertices<2>"] if fused else ["k_dtensor_cells<1>", "k_dtensor_vertices<1>"]
+    # timed by stage, the right-hand sides and the D tensor are launches of
+    # their own; a unit runs them as one (k_rhs_dtensor<2, true>)
+    d0 = [] if fused else ["k_rhs_dtensor<0, false>"]
+    d1 = ["k_rhs_dtensor<2, false>"] if fused else ["k_rhs_dtensor<1, false>"]
     net = "true" if learned and net_in_rheology else "false"
     return {"strain_rates": ["k_strain_tile<true>"],
             "interp_guess": prep,
-            "rheology": ["k_rheo_cells_fast<%d, true, %s>" % (rh, net), "k_rheo_vertices_fast<%d, true, %s>" % (rh, net)],
-            "rhs": ["k_rhs_u", "k_rhs_v", "k_rhs_p"],
+            "rheology": ["k_rheo_fast<%d, true, %s, %d>" % (rh, net, part) for part in ((1, 2) if net == "true" else (0,))],
+            "rhs": ["k_rhs_dtensor<-1, true>"],
             "dtensor_picard": d0,
             "picard_values": values(0, pic, 9, 2),
             "dtensor_jacobian": d1,
             "jacobian_values": values(1, jac, 21, 6),
             "dtensor_picard_2": d0,
-            "residual": ["k_residual_tile<true>", "k_residual_mom<0, false, true>", "k_norms_final_slots"]}
+            "residual": ["k_residual_tile<true>", "k_norms_final_slots"]}
 
 
 # The strain rates and the vertex interpolation of div_u, T, P, d and phi

@@ -762,8 +762,7 @@ extern "C" void UpdateNonLinearity(grid *mesh, markers *particles, markers *topo
     dropin_check(up_list(c, mesh, {DT_IN}));
     mdz_launch_strain_interp5(c->g, c->prm, c->stream);
     dropin_check(rheology_pass(c, 0, c->stream, true));
-    mdz_launch_rhs(c->g, c->prm, c->xg, c->zvx, c->xvz, c->zg, c->stream);
-    mdz_launch_dtensor(c->g, c->prm, 0, c->status, c->stream);
+    mdz_launch_rhs_dtensor(c->g, c->prm, 0, c->xg, c->zvx, c->xvz, c->zg, c->status, c->stream);
     dropin_check(down_list(c, mesh, {STRAIN_OUT}));
     dropin_check(down_list(c, mesh, {RHEO_OUT}));
     dropin_check(down_list(c, mesh, {RHS_OUT}));
@@ -1301,17 +1300,16 @@ static int enqueue_unit(mdz_ctx *c, hipStream_t s) {
     mdz_launch_strain_interp5(c->g, c->prm, s);
     int rc = rheology_pass(c, c->prm.rheo_mode == MDZ_RHEO_LEARNED, s, true);
     if (rc) return rc;
-    mdz_launch_rhs(c->g, c->prm, c->xg, c->zvx, c->xvz, c->zg, s);
     const int kind = c->model.aniso == 1 ? 1 : 0;
     if (fused_dtensor(c)) {
-        mdz_launch_dtensor(c->g, c->prm, 2, c->status, s, c->dpic_n, c->dpic_s);
+        mdz_launch_rhs_dtensor(c->g, c->prm, 2, c->xg, c->zvx, c->xvz, c->zg, c->status, s, c->dpic_n, c->dpic_s);
         mdz_launch_values(0, ap, &c->blk[0], &c->blk[1], &c->blk[2], &c->blk[3], c->shape.pic, s);
         if ((rc = residual_norms(c, 0, ap, s))) return rc;
         mdz_launch_values(1, a, &c->blk[4], &c->blk[5], &c->blk[6], &c->blk[7], c->shape.jac, s);
         c->d_jac = 1;
         return MDZ_OK;
     }
-    mdz_launch_dtensor(c->g, c->prm, 0, c->status, s);
+    mdz_launch_rhs_dtensor(c->g, c->prm, 0, c->xg, c->zvx, c->xvz, c->zg, c->status, s);
     mdz_launch_values(0, a, &c->blk[0], &c->blk[1], &c->blk[2], &c->blk[3], c->shape.pic, s);
     mdz_launch_dtensor(c->g, c->prm, 1, c->status, s);
     mdz_launch_values(1, a, &c->blk[4], &c->blk[5], &c->blk[6], &c->blk[7], c->shape.jac, s);
@@ -1915,14 +1913,11 @@ static int enqueue_trial(mdz_ctx *c, const LsBufs &lb, int k, hipStream_t s) {
     mdz_launch_strain_interp5(c->g, c->prm, s);
     int rc = rheology_pass(c, c->prm.rheo_mode == MDZ_RHEO_LEARNED, s, true);
     if (rc) return rc;
-    mdz_launch_rhs(c->g, c->prm, c->xg, c->zvx, c->xvz, c->zg, s);
     int kind = c->model.aniso == 1 ? 1 : 0;
-    if (fused_dtensor(c)) {
-        a = picard_asm(c);
-        mdz_launch_dtensor(c->g, c->prm, 3, c->status, s, c->dpic_n, c->dpic_s);
-    } else {
-        mdz_launch_dtensor(c->g, c->prm, 0, c->status, s);
-    }
+    const bool fused = fused_dtensor(c);
+    if (fused) a = picard_asm(c);
+    mdz_launch_rhs_dtensor(c->g, c->prm, fused ? 3 : 0, c->xg, c->zvx, c->xvz, c->zg, c->status, s,
+                           fused ? c->dpic_n : nullptr, fused ? c->dpic_s : nullptr);
     if ((rc = residual_norms(c, kind, a, s))) return rc;
     hipLaunchKernelGGL(k_copy6, dim3(1), dim3(64), 0, s, (const double *)c->norm_out, lb.res + 6 * k);
     return MDZ_OK;

@@ -1158,26 +1158,19 @@ __global__ void __launch_bounds__(VBLK) k_values_mom(DevAsm a, DevBlock A, DevBl
     for (int i = threadIdx.x; i < nb; i += VBLK) __builtin_nontemporal_store(sB[i], B.A + b0 + i);
 }
 
-/* The staged value pass split in two launches of 64-row blocks (one wave
- * each), for patterns whose free-row flags and list of general waves are
- * built: GEN = false takes every wave whose rows are all free with the
- * tag-free row code only (fewer registers, so more waves in flight; a wave
- * with a row that is not free returns at once), and the continuity rows in
- * its tail blocks; GEN = true takes only the listed general waves
- * (A.gen_waves, A.n_gen of them) with the general row code.  Same row code
- * and staging as k_values_mom, so the same values bit for bit. */
-template <int KIND, int CAPA, int CAPB, bool GEN>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(GEN ? 1 : (KIND == 1 ? 3 : 6))))
-k_values_split(DevAsm a, DevBlock A, DevBlock B, DevBlock C, DevBlock D, int nbm) {
-    __shared__ double sA[64 * CAPA];
-    __shared__ double sB[64 * CAPB];
-    __shared__ double sDump[64];
-    if (!GEN && (int)blockIdx.x >= nbm) {
-        const int eqn = ((int)blockIdx.x - nbm) * 64 + threadIdx.x;
-        if (eqn < a.e.neq_cont) values_cont_row(a, C, D, eqn, sDump + threadIdx.x);
-        return;
-    }
-    const int wv = GEN ? A.gen_waves[blockIdx.x] : xcd_tile_of(blockIdx.x, nbm);
+/* The staged value pass over 64-row blocks (one wave each), for patterns
+ * whose free-row flags and list of general waves are built: blocks [0, ngen)
+ * take the listed general waves (A.gen_waves) with the general row code, the
+ * next nbm blocks every wave whose rows are all free with the tag-free row
+ * code (a general wave returns at once there), the blocks after them the
+ * continuity rows.  A general wave is one long chain of dependent tag and
+ * field loads: first in the grid, it runs beside the tag-free waves
+ * instead of in a launch of its own after them (Jacobian, 1001 x 501 nodes:
+ * 92 us against 77 + 24; 2049 x 1025: 389 either way, the stores bound it).
+ * Same row code and staging as k_values_mom, so the same values bit for bit. */
+template <bool GEN, int KIND, int CAPA, int CAPB>
+__device__ __forceinline__ void values_wave(const DevAsm &a, DevBlock &A, DevBlock &B, int wv, double *sA, double *sB,
+                                            double *sDump) {
     const int r0 = wv * 64;
     const int r1 = min(r0 + 64, a.e.neq_mom);
     const int eqn = r0 + threadIdx.x;
@@ -1186,7 +1179,7 @@ k_values_split(DevAsm a, DevBlock A, DevBlock B, DevBlock C, DevBlock D, int nbm
      * rows' nodes and its row ranges */
     if (!GEN) {
         const int *pos = A.gen_waves + mdz_div_up(a.e.neq_mom, 64) + 1; /* scanned general-wave flags */
-        if (pos[wv + 1] != pos[wv]) return; /* a general wave: the GEN launch takes it */
+        if (pos[wv + 1] != pos[wv]) return; /* a general wave: listed, taken above */
     }
     const int a0 = A.Ic[r0], b0 = B.Ic[r0], a1 = A.Ic[r1], b1 = B.Ic[r1];
     const int n0 = a.e.mom_node[r0], nl = a.e.mom_node[r1 - 1];
@@ -1220,6 +1213,20 @@ k_values_split(DevAsm a, DevBlock A, DevBlock B, DevBlock C, DevBlock D, int nbm
     const int na = a1 - a0, nb = b1 - b0;
     for (int i = threadIdx.x; i < na; i += 64) __builtin_nontemporal_store(sA[i], A.A + a0 + i);
     for (int i = threadIdx.x; i < nb; i += 64) __builtin_nontemporal_store(sB[i], B.A + b0 + i);
+}
+
+template <int KIND, int CAPA, int CAPB, int WAVES>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES)))
+k_values_split(DevAsm a, DevBlock A, DevBlock B, DevBlock C, DevBlock D, int ngen, int nbm) {
+    __shared__ double sA[64 * CAPA];
+    __shared__ double sB[64 * CAPB];
+    __shared__ double sDump[64];
+    int b = blockIdx.x;
+    if (b < ngen) { values_wave<true, KIND, CAPA, CAPB>(a, A, B, A.gen_waves[b], sA, sB, sDump); return; }
+    b -= ngen;
+    if (b < nbm) { values_wave<false, KIND, CAPA, CAPB>(a, A, B, xcd_tile_of(b, nbm), sA, sB, sDump); return; }
+    const int eqn = (b - nbm) * 64 + threadIdx.x;
+    if (eqn < a.e.neq_cont) values_cont_row(a, C, D, eqn, sDump + threadIdx.x);
 }
 
 /* the same without staging, for patterns with longer rows */
@@ -1270,7 +1277,6 @@ struct NormSlots {
     int nsm, nsc;
     int slot0;        /* first momentum slot of this launch */
     const int *waves; /* general momentum launch: its waves, one per block */
-    int skip_free;    /* general launch: leave the free rows (done by k_residual_tile) */
 };
 
 /* NQ per-thread values summed over the block in a fixed order (waves by
@@ -1314,7 +1320,6 @@ __global__ void __launch_bounds__(BLK) k_residual_mom(DevAsm a, DevBlock A, Norm
     const int frow = A.free_row ? A.free_row[er] : 1;
     if (A.free_row) {
         if ((__all(run ? frow : 1) != 0) != FREE) run = false;
-        if (!FREE && ns.skip_free && frow) run = false;
     } else if (FREE) {
         run = false;
     }
@@ -1345,11 +1350,39 @@ __global__ void __launch_bounds__(BLK) k_residual_mom(DevAsm a, DevBlock A, Norm
     }
 }
 
+/* The general Picard rows (kind 0, Assemble = 0, with the norm work) of
+ * listed wave `slot`, in one wave; its sums go to slot ns.slot0 + slot. */
+__device__ __forceinline__ void residual_general_wave(const DevAsm &a, const DevBlock &A, const NormSlots &ns, int slot) {
+    const int lane = threadIdx.x & 63;
+    const int eqn = ns.waves[slot] * 64 + lane;
+    const bool in = eqn < a.e.neq_mom;
+    const int er = in ? eqn : a.e.neq_mom - 1;
+    const int node = a.e.mom_node[er];
+    const double bbc_in = A.bbc[er], F0 = A.F[er], dr = A.d[er];
+    const bool run = in && !A.free_row[er];
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    if (run) {
+        Sink<SINK_COUNT> ra{0, nullptr, nullptr, 0.0}, rb{0, nullptr, nullptr, 0.0};
+        double b = mom_rhs(a, node), F = F0;
+        momentum_row<false, SINK_COUNT>(0, a, make_tags(a.g), eqn, node, ra, rb, b, bbc_in, F);
+        A.b[eqn] = b;
+        const int nu = a.g.Nx * a.g.nzvx;
+        if (node < nu) { a.g.ru[node] = F; v[0] = F * F; v[1] = 1.0; }
+        else { a.g.rv[node - nu] = F; v[2] = F * F; v[3] = 1.0; }
+        A.F[eqn] = F * dr;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const double t = wave_sum(v[q]);
+        if (lane == 0) ns.partial[q * ns.nsm + ns.slot0 + slot] = t;
+    }
+}
+
 /* The residual pass (Picard, kind 0) with its norm work over tiles of
  * RT_TX x RT_TZ grid positions: lane (i, j) takes the x-momentum row of
  * u-node (i, j) and the z-momentum row of v-node (i, j) when their rows
  * are free (every tag they read is -1: free_node, from the pattern build;
- * the other momentum rows are left to the general launch over the listed
+ * the other momentum rows are left to the blocks of the listed
  * waves), and the continuity row of centroid (i, j).  The block stages
  * u, v, p_corr, the J = 0 D11 (= D22) at the centroids and D33 at the
  * vertices, and the u, v tags, of its tile with a one-node halo in LDS
@@ -1358,7 +1391,11 @@ __global__ void __launch_bounds__(BLK) k_residual_mom(DevAsm a, DevBlock A, Norm
  * that of the tag-free instance of xmom_inner / zmom_inner / continuity_row
  * (same expressions and summation order), so the values are bit for bit
  * those of k_residual_mom<0, true, .> and k_residual_cont.  Per-block sums
- * of F^2 and of the rows go to slot blockIdx.x of each family. */
+ * of F^2 and of the rows go to slot `tile` of each family.  The first ngb
+ * blocks take the listed general waves, one per wave.  The tiles stream from
+ * HBM and want eight waves per SIMD; the general rows then spill, which their
+ * few waves hide behind the tiles (2049 x 1025 nodes: 111 us, 129 without the
+ * bound, 110 + 15 in two launches; 1001 x 501: 37 against 33 + 12). */
 #define RT_TX 64
 #define RT_TZ 4
 struct ResTile {
@@ -1395,14 +1432,21 @@ __device__ __forceinline__ void tile_load(double (&dst)[H][W], signed char (*tds
 }
 
 template <bool NORM>
-__global__ void __launch_bounds__(RT_TX * RT_TZ) k_residual_tile(DevAsm a, DevBlock A, DevBlock C, DevBlock D,
-                                                                 const unsigned char *__restrict__ free_node,
-                                                                 int scaled, int ntx, NormSlots ns) {
+__global__ void __launch_bounds__(RT_TX * RT_TZ) __attribute__((amdgpu_waves_per_eu(8)))
+k_residual_tile(DevAsm a, DevBlock A, DevBlock C, DevBlock D, const unsigned char *__restrict__ free_node, int scaled,
+                int ntx, int ngb, NormSlots ns) {
     __shared__ ResTile T;
     const DevGrid &g = a.g;
     const int Nx = g.Nx, Nz = g.Nz, ncx = g.ncx, ncz = g.ncz, nxvz = g.nxvz, nzvx = g.nzvx;
     const int nu = Nx * nzvx;
-    const int tile = blockIdx.x;
+    /* the listed general waves first, one per wave of the block: their long
+     * load chains run beside the tiles */
+    if (NORM && (int)blockIdx.x < ngb) {
+        const int slot = blockIdx.x * (RT_TX * RT_TZ / 64) + ((int)threadIdx.x >> 6);
+        if (slot < A.n_gen) residual_general_wave(a, A, ns, slot);
+        return;
+    }
+    const int tile = blockIdx.x - ngb;
     const int i0 = (tile % ntx) * RT_TX, j0 = (tile / ntx) * RT_TZ;
     const int tx = threadIdx.x % RT_TX, ty = threadIdx.x / RT_TX;
     const int i = i0 + tx, j = j0 + ty;
@@ -1515,9 +1559,9 @@ __global__ void __launch_bounds__(RT_TX * RT_TZ) k_residual_tile(DevAsm a, DevBl
         block_sums<6>(vsum);
         if (threadIdx.x == 0) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) ns.partial[q * ns.nsm + blockIdx.x] = vsum[q];
-            ns.partial[4 * ns.nsm + blockIdx.x] = vsum[4];
-            ns.partial[4 * ns.nsm + ns.nsc + blockIdx.x] = vsum[5];
+            for (int q = 0; q < 4; q++) ns.partial[q * ns.nsm + tile] = vsum[q];
+            ns.partial[4 * ns.nsm + tile] = vsum[4];
+            ns.partial[4 * ns.nsm + ns.nsc + tile] = vsum[5];
         }
     }
 }
@@ -1787,14 +1831,23 @@ static void launch_staged(const DevAsm &a, DevBlock *A, DevBlock *B, DevBlock *C
                        nbm);
 }
 
+/* WAVES per SIMD of the launch: the Jacobian's general row code takes 207
+ * registers and spills at three waves per SIMD, where the tag-free code runs
+ * best; a grid that two waves per SIMD hold at once (1024 SIMDs) has nothing
+ * to gain from a third (41 x 41 nodes: 17.4 us against 23.0) */
+#define SPLIT_ROUND2 2048
+
 template <int KIND, int CAPA, int CAPB>
 static void launch_split(const DevAsm &a, DevBlock *A, DevBlock *B, DevBlock *C, DevBlock *D, hipStream_t s) {
     const int nbm = mdz_div_up(a.e.neq_mom, 64), nbc = mdz_div_up(a.e.neq_cont, 64);
-    hipLaunchKernelGGL((k_values_split<KIND, CAPA, CAPB, false>), dim3(nbm + nbc), dim3(64), 0, s, a, *A, *B, *C, *D,
-                       nbm);
-    if (A->n_gen > 0)
-        hipLaunchKernelGGL((k_values_split<KIND, CAPA, CAPB, true>), dim3(A->n_gen), dim3(64), 0, s, a, *A, *B, *C,
-                           *D, nbm);
+    const int grid = A->n_gen + nbm + nbc;
+    constexpr int MOST = KIND == 1 ? 3 : 6;
+    if (KIND == 1 && grid <= SPLIT_ROUND2)
+        hipLaunchKernelGGL((k_values_split<KIND, CAPA, CAPB, 2>), dim3(grid), dim3(64), 0, s, a, *A, *B, *C, *D,
+                           A->n_gen, nbm);
+    else
+        hipLaunchKernelGGL((k_values_split<KIND, CAPA, CAPB, MOST>), dim3(grid), dim3(64), 0, s, a, *A, *B, *C, *D,
+                           A->n_gen, nbm);
 }
 
 __global__ void __launch_bounds__(BLK) k_fill_bytes(unsigned char *p, int n) {
@@ -1948,14 +2001,10 @@ int mdz_launch_residual_norms(int kind, const DevAsm &a, DevBlock *A, DevBlock *
         const int ntx = mdz_div_up(a.g.Nx + 1, RT_TX), ntz = mdz_div_up(a.g.Nz + 1, RT_TZ), nt = ntx * ntz;
         const int ngen = A->n_gen;
         if ((size_t)(4 * (nt + ngen) + 2 * nt) <= partial_len) {
-            NormSlots ns{partial, nt + ngen, nt, 0, A->gen_waves, 0};
-            hipLaunchKernelGGL(k_residual_tile<true>, dim3(nt), dim3(RT_TX * RT_TZ), 0, s, a, *A, *C, *D,
-                               (const unsigned char *)A->free_node, d_scaled, ntx, ns);
-            if (ngen > 0) {
-                ns.slot0 = nt;
-                ns.skip_free = 1;
-                hipLaunchKernelGGL((k_residual_mom<0, false, true>), dim3(ngen), dim3(64), 0, s, a, *A, ns);
-            }
+            NormSlots ns{partial, nt + ngen, nt, nt, A->gen_waves};
+            const int ngb = mdz_div_up(ngen, RT_TX * RT_TZ / 64);
+            hipLaunchKernelGGL(k_residual_tile<true>, dim3(ngb + nt), dim3(RT_TX * RT_TZ), 0, s, a, *A, *C, *D,
+                               (const unsigned char *)A->free_node, d_scaled, ntx, ngb, ns);
             hipLaunchKernelGGL(k_norms_final_slots, dim3(3), dim3(1024), 0, s, (const double *)partial, nt + ngen, nt,
                                out6);
             return MDZ_OK;

@@ -43,6 +43,10 @@ void mdz_launch_dtensor(const DevGrid &g, const DevParams &prm, int mode, int *s
                         double *dp_n = nullptr, double *dp_s = nullptr);
 void mdz_launch_rhs(const DevGrid &g, const DevParams &prm, const double *xg, const double *zvx,
                     const double *xvz, const double *zg, hipStream_t s);
+/* both in one launch (neither reads what the other writes) */
+void mdz_launch_rhs_dtensor(const DevGrid &g, const DevParams &prm, int mode, const double *xg, const double *zvx,
+                            const double *xvz, const double *zg, int *status, hipStream_t s, double *dp_n = nullptr,
+                            double *dp_s = nullptr);
 
 /* assembly half (mdz_assembly.hip) */
 struct DevAsm {

@@ -744,19 +744,14 @@ __device__ __forceinline__ void rheo_node(const DevGrid &g, const DevParams &prm
     }
 }
 
-/* Two waves per SIMD: every variant fits 256 registers without scratch;
- * one wave per SIMD left the FP64 latency exposed.  Dynamic LDS: the
- * stash, (StashSlots::nd + max(Nb_phases, 4)) * NT doubles. */
+/* centroid `c0` of the lane (c0 >= nc: no node) */
 template <int NT, bool DIAG, bool NET>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
-k_rheo_cells_fast(DevGrid g, DevParams prm, FastConst fc, const PhaseK *__restrict__ pk, double R,
-                  const float *__restrict__ guess, DevMLPI w, SpreadConst sc, unsigned long long *hist) {
-    __shared__ unsigned int lh[3 * MDZ_HIST_BINS];
-    extern __shared__ double stash[];
+__device__ __forceinline__ void rheo_cell_fast(const DevGrid &g, const DevParams &prm, const FastConst &fc,
+                                               const PhaseK *__restrict__ pk, double R,
+                                               const float *__restrict__ guess, const DevMLPI &w,
+                                               const SpreadConst &sc, const BlockHist &bh, double *stash, int c0) {
     constexpr int ND = StashSlots<true, DIAG>::nd;
-    const BlockHist bh = hist_begin(lh, hist);
     const int nc = g.ncx * g.ncz;
-    const int c0 = blockIdx.x * NT + threadIdx.x;
     const int c = c0 < nc ? c0 : nc - 1;
     double *sl = stash + threadIdx.x;
     NodeLoad v;
@@ -776,19 +771,16 @@ k_rheo_cells_fast(DevGrid g, DevParams prm, FastConst fc, const PhaseK *__restri
     if constexpr (NET)
         gi = net_prologue<NT>(g, prm, w, pk, sc, c0 < nc && v.tag != 30 && v.tag != 31, c0, nc, v, sl + ND * NT);
     if (c0 < nc) rheo_node<NT, true, DIAG>(g, prm, pk, fc, R, gi, bh, c0, nc, v, sl);
-    hist_flush(bh, hist);
 }
 
+/* vertex `c1` of the lane (c1 >= nv: no node) */
 template <int NT, bool DIAG, bool NET>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
-k_rheo_vertices_fast(DevGrid g, DevParams prm, FastConst fc, const PhaseK *__restrict__ pk, double R,
-                     const float *__restrict__ guess, DevMLPI w, SpreadConst sc, unsigned long long *hist) {
-    __shared__ unsigned int lh[3 * MDZ_HIST_BINS];
-    extern __shared__ double stash[];
+__device__ __forceinline__ void rheo_vertex_fast(const DevGrid &g, const DevParams &prm, const FastConst &fc,
+                                                 const PhaseK *__restrict__ pk, double R,
+                                                 const float *__restrict__ guess, const DevMLPI &w,
+                                                 const BlockHist &bh, double *stash, int c1) {
     constexpr int ND = StashSlots<false, DIAG>::nd;
-    const BlockHist bh = hist_begin(lh, hist);
     const int nv = g.Nx * g.Nz;
-    const int c1 = blockIdx.x * NT + threadIdx.x;
     const int c = c1 < nv ? c1 : nv - 1;
     double *sl = stash + threadIdx.x;
     NodeLoad v;
@@ -824,6 +816,31 @@ k_rheo_vertices_fast(DevGrid g, DevParams prm, FastConst fc, const PhaseK *__res
         gi = GuessIn{nullptr, ph, guess_factor(ph, y0), guess_gdot(ph, y1)};
     }
     if (c1 < nv) rheo_node<NT, false, DIAG>(g, prm, pk, fc, R, gi, bh, c1, nv, v, sl);
+}
+
+enum { RHEO_BOTH, RHEO_CELLS, RHEO_VERTICES };
+
+/* The local iterations at the centroids, then at the vertices, as block
+ * ranges of one launch: the two are independent, so the last centroid waves
+ * and the first vertex waves share the chip (41 x 41 nodes: 13 us against
+ * 13 + 10, 1001 x 501: 119 against 79 + 62).  With the network's guess in the
+ * pass (NET) a vertex reads the network outputs of its centroids, which the
+ * centroid blocks write: then each has its own launch.  Two waves per SIMD: every variant fits 256 registers without
+ * scratch; one wave per SIMD left the FP64 latency exposed.  Dynamic LDS:
+ * the stash, (StashSlots::nd + max(Nb_phases, 4)) * NT doubles. */
+template <int NT, bool DIAG, bool NET, int PART>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
+k_rheo_fast(DevGrid g, DevParams prm, FastConst fc, const PhaseK *__restrict__ pk, double R,
+            const float *__restrict__ guess_n, const float *__restrict__ guess_s, DevMLPI w, SpreadConst sc,
+            unsigned long long *hist) {
+    __shared__ unsigned int lh[3 * MDZ_HIST_BINS];
+    extern __shared__ double stash[];
+    const BlockHist bh = hist_begin(lh, hist);
+    const int b = blockIdx.x, nbc = PART == RHEO_VERTICES ? 0 : mdz_div_up(g.ncx * g.ncz, NT);
+    if (PART != RHEO_VERTICES && b < nbc)
+        rheo_cell_fast<NT, DIAG, NET>(g, prm, fc, pk, R, guess_n, w, sc, bh, stash, b * NT + (int)threadIdx.x);
+    if (PART != RHEO_CELLS && b >= nbc)
+        rheo_vertex_fast<NT, DIAG, NET>(g, prm, fc, pk, R, guess_s, w, bh, stash, (b - nbc) * NT + (int)threadIdx.x);
     hist_flush(bh, hist);
 }
 
@@ -857,10 +874,16 @@ static void launch_fast(const DevGrid &g, const DevParams &prm, const PhaseK *pk
     const int nph = prm.Nb_phases > 4 ? prm.Nb_phases : 4; /* stash_fractions writes at least four slots */
     const size_t lds_c = (size_t)(StashSlots<true, DIAG>::nd + nph) * NT * sizeof(double);
     const size_t lds_v = (size_t)(StashSlots<false, DIAG>::nd + nph) * NT * sizeof(double);
-    hipLaunchKernelGGL((k_rheo_cells_fast<NT, DIAG, NET>), dim3(mdz_div_up(nc, NT)), dim3(NT), lds_c, s, g, prm, fc,
-                       pk, R, guess_n, w, sc, hist);
-    hipLaunchKernelGGL((k_rheo_vertices_fast<NT, DIAG, NET>), dim3(mdz_div_up(nv, NT)), dim3(NT), lds_v, s, g, prm,
-                       fc, pk, R, guess_s, w, sc, hist);
+    const int nbc = mdz_div_up(nc, NT), nbv = mdz_div_up(nv, NT);
+    if constexpr (NET) {
+        hipLaunchKernelGGL((k_rheo_fast<NT, DIAG, NET, RHEO_CELLS>), dim3(nbc), dim3(NT), lds_c, s, g, prm, fc, pk, R,
+                           guess_n, guess_s, w, sc, hist);
+        hipLaunchKernelGGL((k_rheo_fast<NT, DIAG, NET, RHEO_VERTICES>), dim3(nbv), dim3(NT), lds_v, s, g, prm, fc, pk,
+                           R, guess_n, guess_s, w, sc, hist);
+    } else {
+        hipLaunchKernelGGL((k_rheo_fast<NT, DIAG, NET, RHEO_BOTH>), dim3(nbc + nbv), dim3(NT),
+                           lds_c > lds_v ? lds_c : lds_v, s, g, prm, fc, pk, R, guess_n, guess_s, w, sc, hist);
+    }
 }
 
 template <int NT, bool DIAG>

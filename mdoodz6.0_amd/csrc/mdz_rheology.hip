@@ -549,9 +549,8 @@ __device__ __forceinline__ void aniso_factors(const DevParams &prm, double nx, d
  * in one batch before its tag test (the anisotropy fields and the
  * compressibility only where the model uses them, after that batch). */
 template <int MODE>
-__global__ void __launch_bounds__(BLK) k_dtensor_cells(DevGrid g, DevParams prm, double *__restrict__ dp) {
+__device__ __forceinline__ void dtensor_cell(const DevGrid &g, const DevParams &prm, double *__restrict__ dp, int k) {
     constexpr bool JAC = MODE == 1 || MODE == 2, PIC = MODE >= 2;
-    int k = xcd_tile() * BLK + threadIdx.x;
     if (k >= g.ncx * g.ncz) return;
     const int t = g.BCp[k];
     const double eta = g.eta_n[k];
@@ -604,9 +603,9 @@ __global__ void __launch_bounds__(BLK) k_dtensor_cells(DevGrid g, DevParams prm,
 }
 
 template <int MODE>
-__global__ void __launch_bounds__(BLK) k_dtensor_vertices(DevGrid g, DevParams prm, int *status, double *__restrict__ dp) {
+__device__ __forceinline__ void dtensor_vertex(const DevGrid &g, const DevParams &prm, int *status,
+                                               double *__restrict__ dp, int k) {
     constexpr bool JAC = MODE == 1 || MODE == 2, PIC = MODE >= 2;
-    int k = xcd_tile() * BLK + threadIdx.x;
     if (k >= g.Nx * g.Nz) return;
     const int t = g.BCg[k];
     const double eta = g.eta_s[k];
@@ -657,9 +656,8 @@ __global__ void __launch_bounds__(BLK) k_dtensor_vertices(DevGrid g, DevParams p
  * decide which of them are used, so that a wave waits for memory once. */
 __device__ __forceinline__ int clampi(int i, int n) { return i < 0 ? 0 : (i >= n ? n - 1 : i); }
 
-__global__ void __launch_bounds__(BLK) k_rhs_u(DevGrid g, DevParams prm, const double *__restrict__ xg,
-                                               const double *__restrict__ zvx) {
-    int c = xcd_tile() * BLK + threadIdx.x;
+__device__ __forceinline__ void rhs_u(const DevGrid &g, const DevParams &prm, const double *__restrict__ xg,
+                                      const double *__restrict__ zvx, int c) {
     int Nx = g.Nx, NzVx = g.nzvx, Ncx = g.ncx;
     if (c >= Nx * NzVx) return;
     int k = c % Nx, l = c / Nx;
@@ -710,16 +708,15 @@ __global__ void __launch_bounds__(BLK) k_rhs_u(DevGrid g, DevParams prm, const d
     g.roger_x[c] = -r;
 }
 
-__global__ void __launch_bounds__(BLK) k_rhs_v(DevGrid g, DevParams prm, const double *__restrict__ xvz,
-                                               const double *__restrict__ zg) {
-    int c = xcd_tile() * BLK + threadIdx.x;
+__device__ __forceinline__ void rhs_v(const DevGrid &g, const DevParams &prm, const double *__restrict__ xvz,
+                                      const double *__restrict__ zg, int c) {
     int Nx = g.Nx, NxVz = g.nxvz, Nz = g.Nz, Ncx = g.ncx;
     if (c >= NxVz * Nz) return;
     int k = c % NxVz, l = c / NxVz;
     int c1 = k + l * Nx - 1, c2 = k - 1 + (l - 1) * Ncx;
     const int nc = Ncx * g.ncz, nv = Nx * Nz, nw = NxVz * Nz;
     int iPrS = c2, iPrN = c2 + Ncx, ixyE = c1 + 1, ixyW = c1, iVyW = c - 1, iVyE = c + 1;
-    /* every input in one batch (clamped indices), as in k_rhs_u */
+    /* every input in one batch (clamped indices), as in rhs_u */
     const int tv = g.BCv[c];
     const int jS = clampi(iPrS, nc), jN = clampi(iPrN, nc), vW = clampi(ixyW, nv), vE = clampi(ixyE, nv);
     const int wW = clampi(iVyW, nw), wE = clampi(iVyE, nw);
@@ -745,7 +742,7 @@ __global__ void __launch_bounds__(BLK) k_rhs_v(DevGrid g, DevParams prm, const d
         r = -gz * rhoVz;
         if (prm.iselastic == 1 && l > 0 && l < Nz - 1) {
             double dx = g.dx, dz = g.dz, dt = prm.dt;
-            /* every term formed, applied by its flag (as in k_rhs_u) */
+            /* every term formed, applied by its flag (as in rhs_u) */
             const double tN = 1.0 / dz * (eN / (mN * dt) * (sN));
             const double tS = 1.0 / dz * (-eS / (mS * dt) * (sS));
             const double tE = 1.0 / dx * (eE / (mE * dt) * sE);
@@ -759,8 +756,7 @@ __global__ void __launch_bounds__(BLK) k_rhs_v(DevGrid g, DevParams prm, const d
     g.roger_z[c] = -r;
 }
 
-__global__ void __launch_bounds__(BLK) k_rhs_p(DevGrid g, DevParams prm) {
-    int c = xcd_tile() * BLK + threadIdx.x;
+__device__ __forceinline__ void rhs_p(const DevGrid &g, const DevParams &prm, int c) {
     if (c >= g.ncx * g.ncz) return;
     int t = g.BCp[c];
     if (t != 30 && t != 31) {
@@ -774,6 +770,36 @@ __global__ void __launch_bounds__(BLK) k_rhs_p(DevGrid g, DevParams prm) {
         }
         g.rhs_p[c] = r;
     }
+}
+
+/* The right-hand sides (RHS) and the D tensor (MODE 0..3 as above, -1 none)
+ * in one launch: both read only what the rheology wrote, so that their five
+ * passes -- u rows, v rows, cells, vertices, p rows -- are block ranges of
+ * one grid and run side by side: 4 us against 17 in five launches at 41 x 41
+ * nodes, 50 against 64 at 1001 x 501, 198 against 213 at 2049 x 1025 (HBM).
+ * Five waves per SIMD hold the u rows' 96 registers; four or six, with spills,
+ * are slower (50.1, 53.2 us). */
+template <int MODE, bool RHS>
+__global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(5)))
+k_rhs_dtensor(DevGrid g, DevParams prm, const double *__restrict__ xg, const double *__restrict__ zvx,
+              const double *__restrict__ xvz, const double *__restrict__ zg, int *status, double *__restrict__ dp_n,
+              double *__restrict__ dp_s) {
+    int b = blockIdx.x;
+    const int nbc = mdz_div_up(g.ncx * g.ncz, BLK), nbs = mdz_div_up(g.Nx * g.Nz, BLK);
+    if (RHS) {
+        const int nbu = mdz_div_up(g.Nx * g.nzvx, BLK), nbv = mdz_div_up(g.nxvz * g.Nz, BLK);
+        if (b < nbu) { rhs_u(g, prm, xg, zvx, xcd_tile_of(b, nbu) * BLK + threadIdx.x); return; }
+        b -= nbu;
+        if (b < nbv) { rhs_v(g, prm, xvz, zg, xcd_tile_of(b, nbv) * BLK + threadIdx.x); return; }
+        b -= nbv;
+    }
+    if constexpr (MODE >= 0) {
+        if (b < nbc) { dtensor_cell<MODE>(g, prm, dp_n, xcd_tile_of(b, nbc) * BLK + threadIdx.x); return; }
+        b -= nbc;
+        if (b < nbs) { dtensor_vertex<MODE>(g, prm, status, dp_s, xcd_tile_of(b, nbs) * BLK + threadIdx.x); return; }
+        b -= nbs;
+    }
+    if (RHS) rhs_p(g, prm, xcd_tile_of(b, nbc) * BLK + threadIdx.x);
 }
 
 /* ---------------------------------------------------------------- */
@@ -810,34 +836,41 @@ void mdz_launch_rheology(const DevGrid &g, const DevParams &prm, const mat_prop 
     hipLaunchKernelGGL(k_rheo_vertices, dim3(mdz_div_up(nv, BLK)), dim3(BLK), 0, s, g, prm, mt, guess_s, hist);
 }
 
+/* mode: 0..3 (mdz_launch_dtensor) or -1; rhs: with the right-hand sides */
+static void launch_rhs_dtensor(const DevGrid &g, const DevParams &prm, int mode, bool rhs, const double *xg,
+                               const double *zvx, const double *xvz, const double *zg, int *status, double *dp_n,
+                               double *dp_s, hipStream_t s) {
+    const int nc = mdz_div_up(g.ncx * g.ncz, BLK);
+    int nb = 0;
+    if (rhs) nb += mdz_div_up(g.Nx * g.nzvx, BLK) + mdz_div_up(g.nxvz * g.Nz, BLK) + nc;
+    if (mode >= 0) nb += nc + mdz_div_up(g.Nx * g.Nz, BLK);
+#define MDZ_RD(M, R)                                                                                               \
+    hipLaunchKernelGGL((k_rhs_dtensor<M, R>), dim3(nb), dim3(BLK), 0, s, g, prm, xg, zvx, xvz, zg, status, dp_n, dp_s)
+    switch (mode * 2 + (rhs ? 1 : 0)) {
+    case -1: MDZ_RD(-1, true); break;
+    case 0: MDZ_RD(0, false); break;
+    case 1: MDZ_RD(0, true); break;
+    case 2: MDZ_RD(1, false); break;
+    case 4: MDZ_RD(2, false); break;
+    case 5: MDZ_RD(2, true); break;
+    case 6: MDZ_RD(3, false); break;
+    default: MDZ_RD(3, true); break;
+    }
+#undef MDZ_RD
+}
+
 void mdz_launch_dtensor(const DevGrid &g, const DevParams &prm, int mode, int *status, hipStream_t s, double *dp_n,
                         double *dp_s) {
-    int nc = g.ncx * g.ncz, nv = g.Nx * g.Nz;
-    dim3 gc(mdz_div_up(nc, BLK)), gv(mdz_div_up(nv, BLK)), b(BLK);
-    switch (mode) {
-    case 0:
-        hipLaunchKernelGGL(k_dtensor_cells<0>, gc, b, 0, s, g, prm, dp_n);
-        hipLaunchKernelGGL(k_dtensor_vertices<0>, gv, b, 0, s, g, prm, status, dp_s);
-        break;
-    case 1:
-        hipLaunchKernelGGL(k_dtensor_cells<1>, gc, b, 0, s, g, prm, dp_n);
-        hipLaunchKernelGGL(k_dtensor_vertices<1>, gv, b, 0, s, g, prm, status, dp_s);
-        break;
-    case 2:
-        hipLaunchKernelGGL(k_dtensor_cells<2>, gc, b, 0, s, g, prm, dp_n);
-        hipLaunchKernelGGL(k_dtensor_vertices<2>, gv, b, 0, s, g, prm, status, dp_s);
-        break;
-    default:
-        hipLaunchKernelGGL(k_dtensor_cells<3>, gc, b, 0, s, g, prm, dp_n);
-        hipLaunchKernelGGL(k_dtensor_vertices<3>, gv, b, 0, s, g, prm, status, dp_s);
-        break;
-    }
+    launch_rhs_dtensor(g, prm, mode, false, nullptr, nullptr, nullptr, nullptr, status, dp_n, dp_s, s);
 }
 
 void mdz_launch_rhs(const DevGrid &g, const DevParams &prm, const double *xg, const double *zvx,
                     const double *xvz, const double *zg, hipStream_t s) {
-    int nu = g.Nx * g.nzvx, nw = g.nxvz * g.Nz, nc = g.ncx * g.ncz;
-    hipLaunchKernelGGL(k_rhs_u, dim3(mdz_div_up(nu, BLK)), dim3(BLK), 0, s, g, prm, xg, zvx);
-    hipLaunchKernelGGL(k_rhs_v, dim3(mdz_div_up(nw, BLK)), dim3(BLK), 0, s, g, prm, xvz, zg);
-    hipLaunchKernelGGL(k_rhs_p, dim3(mdz_div_up(nc, BLK)), dim3(BLK), 0, s, g, prm);
+    launch_rhs_dtensor(g, prm, -1, true, xg, zvx, xvz, zg, nullptr, nullptr, nullptr, s);
+}
+
+void mdz_launch_rhs_dtensor(const DevGrid &g, const DevParams &prm, int mode, const double *xg, const double *zvx,
+                            const double *xvz, const double *zg, int *status, hipStream_t s, double *dp_n,
+                            double *dp_s) {
+    launch_rhs_dtensor(g, prm, mode, true, xg, zvx, xvz, zg, status, dp_n, dp_s, s);
 }
