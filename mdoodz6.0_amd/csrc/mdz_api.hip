@@ -120,6 +120,7 @@ struct mdz_ctx {
     int *scratch;
     size_t scratch_len;
     double *norm_partial, *norm_out;
+    double *norm_host; /* pinned: the six sums of the last eager unit */
     size_t norm_partial_len;
     int *status;
     unsigned long long *hist;
@@ -309,6 +310,8 @@ static int ctx_alloc(mdz_ctx **out, int Nx, int Nz, int nph) {
     c->norm_partial_len = np;
     if (hipMalloc((void **)&c->norm_partial, np * sizeof(double) + 256) != hipSuccess) return set_err(MDZ_ENOMEM, "norms");
     if (hipMalloc((void **)&c->norm_out, 8 * sizeof(double)) != hipSuccess) return set_err(MDZ_ENOMEM, "norms");
+    if (hipHostMalloc((void **)&c->norm_host, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess)
+        return set_err(MDZ_ENOMEM, "norms");
     if (hipMalloc((void **)&c->status, 4 * sizeof(int)) != hipSuccess) return set_err(MDZ_ENOMEM, "status");
     if (hipMalloc((void **)&c->hist, 3 * MDZ_HIST_BINS * sizeof(unsigned long long)) != hipSuccess) return set_err(MDZ_ENOMEM, "hist");
     if (hipMalloc((void **)&c->d_mat, sizeof(mat_prop)) != hipSuccess) return set_err(MDZ_ENOMEM, "materials");
@@ -325,6 +328,7 @@ static void ctx_release(mdz_ctx *c) {
     hipStreamSynchronize(c->stream);
     ctx_free_blocks(c);
     hipFree(c->slab); hipFree(c->scratch); hipFree(c->norm_partial); hipFree(c->norm_out);
+    if (c->norm_host) hipHostFree(c->norm_host);
     hipFree(c->status); hipFree(c->hist); hipFree(c->d_mat); hipFree(c->d_pk); hipFree(c->guess_n); hipFree(c->guess_s);
     hipFree(c->cellnet);
     hipFree(c->d_net); hipFree(c->net_wp); hipFree(c->net_bp);
@@ -1285,17 +1289,19 @@ extern "C" int mdz_ctx_set_rheology_mode(mdz_ctx *c, int mode) {
     return MDZ_OK;
 }
 
-/* residual rows of block family `kind` and their norms into c->norm_out */
-static int residual_norms(mdz_ctx *c, int kind, const DevAsm &a, hipStream_t s) {
+/* residual rows of block family `kind` and their norms into c->norm_out
+ * (and host6, see mdz_launch_residual_norms) */
+static int residual_norms(mdz_ctx *c, int kind, const DevAsm &a, hipStream_t s, double *host6 = nullptr) {
     int rc = mdz_launch_residual_norms(kind, a, &c->blk[4 * kind], &c->blk[4 * kind + 2], &c->blk[4 * kind + 3],
-                                       c->norm_partial, c->norm_partial_len, c->norm_out, s, c->d_scaled[kind]);
+                                       c->norm_partial, c->norm_partial_len, c->norm_out, s, c->d_scaled[kind], host6);
     return rc ? set_err(rc, "residual norms") : MDZ_OK;
 }
 
 /* One Newton-iteration unit of a context, enqueued on stream s with no
  * allocation, memset, host synchronisation or copy: safe to capture into a
- * graph.  The norms stay in c->norm_out (six doubles). */
-static int enqueue_unit(mdz_ctx *c, hipStream_t s) {
+ * graph.  The norms stay in c->norm_out (six doubles); host6 (optional,
+ * pinned) receives them too. */
+static int enqueue_unit(mdz_ctx *c, hipStream_t s, double *host6 = nullptr) {
     DevAsm a = make_asm(c), ap = picard_asm(c);
     mdz_launch_strain_interp5(c->g, c->prm, s);
     int rc = rheology_pass(c, c->prm.rheo_mode == MDZ_RHEO_LEARNED, s, true);
@@ -1303,9 +1309,10 @@ static int enqueue_unit(mdz_ctx *c, hipStream_t s) {
     const int kind = c->model.aniso == 1 ? 1 : 0;
     if (fused_dtensor(c)) {
         mdz_launch_rhs_dtensor(c->g, c->prm, 2, c->xg, c->zvx, c->xvz, c->zg, c->status, s, c->dpic_n, c->dpic_s);
-        mdz_launch_values(0, ap, &c->blk[0], &c->blk[1], &c->blk[2], &c->blk[3], c->shape.pic, s);
-        if ((rc = residual_norms(c, 0, ap, s))) return rc;
-        mdz_launch_values(1, a, &c->blk[4], &c->blk[5], &c->blk[6], &c->blk[7], c->shape.jac, s);
+        const bool pair = mdz_launch_values_pair(ap, &c->blk[0], &c->blk[4], c->shape.pic, c->shape.jac, s);
+        if (!pair) mdz_launch_values(0, ap, &c->blk[0], &c->blk[1], &c->blk[2], &c->blk[3], c->shape.pic, s);
+        if ((rc = residual_norms(c, 0, ap, s, host6))) return rc;
+        if (!pair) mdz_launch_values(1, a, &c->blk[4], &c->blk[5], &c->blk[6], &c->blk[7], c->shape.jac, s);
         c->d_jac = 1;
         return MDZ_OK;
     }
@@ -1314,7 +1321,7 @@ static int enqueue_unit(mdz_ctx *c, hipStream_t s) {
     mdz_launch_dtensor(c->g, c->prm, 1, c->status, s);
     mdz_launch_values(1, a, &c->blk[4], &c->blk[5], &c->blk[6], &c->blk[7], c->shape.jac, s);
     mdz_launch_dtensor(c->g, c->prm, 0, c->status, s);
-    return residual_norms(c, kind, a, s);
+    return residual_norms(c, kind, a, s, host6);
 }
 
 /* resx, resz, resp from the six sums of the norm kernels */
@@ -1329,13 +1336,11 @@ static int norms_to_res(const double *out6, double *res3) {
 extern "C" int mdz_ctx_newton_unit(mdz_ctx *c, double *res3) {
     if (!c) return set_err(MDZ_EINVAL, "NULL context");
     g_status = 0;
-    int rc = enqueue_unit(c, c->stream);
+    int rc = enqueue_unit(c, c->stream, res3 ? c->norm_host : nullptr);
     if (rc) return rc;
     if (res3) {
-        double out6[6];
-        HIPCHK(hipMemcpyAsync(out6, c->norm_out, 6 * 8, hipMemcpyDeviceToHost, c->stream));
         if ((rc = sync(c))) return rc;
-        if ((rc = norms_to_res(out6, res3))) return rc;
+        if ((rc = norms_to_res(c->norm_host, res3))) return rc;
     }
     HIPCHK(hipGetLastError());
     return MDZ_OK;

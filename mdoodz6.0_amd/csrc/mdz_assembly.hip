@@ -1229,6 +1229,40 @@ k_values_split(DevAsm a, DevBlock A, DevBlock B, DevBlock C, DevBlock D, int nge
     if (eqn < a.e.neq_cont) values_cont_row(a, C, D, eqn, sDump + threadIdx.x);
 }
 
+/* The value passes of the Picard (P) and Jacobian (J) families in one launch
+ * of 64-row blocks: their general waves, tag-free waves and continuity rows
+ * in turn.  Picard rows read the J = 0 components of `a`, Jacobian rows the
+ * tensor of the grid, so the two need no order. */
+struct ValuesPair {
+    DevBlock A[2], B[2], C[2], D[2]; /* 0 Picard, 1 Jacobian */
+};
+
+template <int CAPA0, int CAPB0, int CAPA1, int CAPB1>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+k_values_pair(DevAsm a, ValuesPair p, int nbm, int nbc) {
+    __shared__ double sA[64 * CAPA1];
+    __shared__ double sB[64 * CAPB1];
+    __shared__ double sDump[64];
+    int b = blockIdx.x;
+    if (b < p.A[1].n_gen) {
+        values_wave<true, 1, CAPA1, CAPB1>(a, p.A[1], p.B[1], p.A[1].gen_waves[b], sA, sB, sDump);
+        return;
+    }
+    b -= p.A[1].n_gen;
+    if (b < p.A[0].n_gen) {
+        values_wave<true, 0, CAPA0, CAPB0>(a, p.A[0], p.B[0], p.A[0].gen_waves[b], sA, sB, sDump);
+        return;
+    }
+    b -= p.A[0].n_gen;
+    if (b < nbm) { values_wave<false, 1, CAPA1, CAPB1>(a, p.A[1], p.B[1], xcd_tile_of(b, nbm), sA, sB, sDump); return; }
+    b -= nbm;
+    if (b < nbm) { values_wave<false, 0, CAPA0, CAPB0>(a, p.A[0], p.B[0], xcd_tile_of(b, nbm), sA, sB, sDump); return; }
+    b -= nbm;
+    const int k = b < nbc ? 0 : 1;
+    const int eqn = (b - k * nbc) * 64 + threadIdx.x;
+    if (eqn < a.e.neq_cont) values_cont_row(a, p.C[k], p.D[k], eqn, sDump + threadIdx.x);
+}
+
 /* the same without staging, for patterns with longer rows */
 template <int KIND>
 __global__ void __launch_bounds__(BLK) k_values_mom_direct(DevAsm a, DevBlock A, DevBlock B) {
@@ -1841,13 +1875,32 @@ template <int KIND, int CAPA, int CAPB>
 static void launch_split(const DevAsm &a, DevBlock *A, DevBlock *B, DevBlock *C, DevBlock *D, hipStream_t s) {
     const int nbm = mdz_div_up(a.e.neq_mom, 64), nbc = mdz_div_up(a.e.neq_cont, 64);
     const int grid = A->n_gen + nbm + nbc;
-    constexpr int MOST = KIND == 1 ? 3 : 6;
-    if (KIND == 1 && grid <= SPLIT_ROUND2)
-        hipLaunchKernelGGL((k_values_split<KIND, CAPA, CAPB, 2>), dim3(grid), dim3(64), 0, s, a, *A, *B, *C, *D,
-                           A->n_gen, nbm);
-    else
-        hipLaunchKernelGGL((k_values_split<KIND, CAPA, CAPB, MOST>), dim3(grid), dim3(64), 0, s, a, *A, *B, *C, *D,
-                           A->n_gen, nbm);
+    if constexpr (KIND == 1)
+        if (grid <= SPLIT_ROUND2) {
+            hipLaunchKernelGGL((k_values_split<KIND, CAPA, CAPB, 2>), dim3(grid), dim3(64), 0, s, a, *A, *B, *C, *D,
+                               A->n_gen, nbm);
+            return;
+        }
+    hipLaunchKernelGGL((k_values_split<KIND, CAPA, CAPB, KIND == 1 ? 3 : 6>), dim3(grid), dim3(64), 0, s, a, *A, *B,
+                       *C, *D, A->n_gen, nbm);
+}
+
+/* One launch up to the size where two waves per SIMD hold both passes at
+ * once: there each pass is the latency of its general waves (18 and 9 us at
+ * 41 x 41 nodes), which overlap.  Beyond it the Picard pass would lose the six
+ * waves per SIMD that it has on its own. */
+bool mdz_launch_values_pair(const DevAsm &a, DevBlock *P, DevBlock *J, int vblk_p, int vblk_j, hipStream_t s) {
+    const bool split = P->free_row && P->gen_waves && J->free_row && J->gen_waves;
+    const bool fits = P[0].maxrow <= PIC_CAPA && P[1].maxrow <= PIC_CAPB && J[0].maxrow <= JAC_CAPA &&
+                      J[1].maxrow <= JAC_CAPB;
+    if (a.e.neq_mom <= 0 || vblk_p == 0 || vblk_j != 64 || !split || !fits) return false;
+    const int nbm = mdz_div_up(a.e.neq_mom, 64), nbc = mdz_div_up(a.e.neq_cont, 64);
+    const int grid = P->n_gen + J->n_gen + 2 * (nbm + nbc);
+    if (grid > SPLIT_ROUND2) return false;
+    const ValuesPair p{{P[0], J[0]}, {P[1], J[1]}, {P[2], J[2]}, {P[3], J[3]}};
+    hipLaunchKernelGGL((k_values_pair<PIC_CAPA, PIC_CAPB, JAC_CAPA, JAC_CAPB>), dim3(grid), dim3(64), 0, s, a, p, nbm,
+                       nbc);
+    return true;
 }
 
 __global__ void __launch_bounds__(BLK) k_fill_bytes(unsigned char *p, int n) {
@@ -1967,8 +2020,11 @@ size_t mdz_residual_norm_partials(int nm, int n_gen, int ncnt) {
     return 4 * ((size_t)mdz_div_up(nm, BLK) + (size_t)n_gen) + 2 * (size_t)mdz_div_up(ncnt, BLK);
 }
 
-/* one block per family: the slots of its sums and counts, in slot order */
-__global__ void __launch_bounds__(1024) k_norms_final_slots(const double *partial, int nsm, int nsc, double *out6) {
+/* one block per family: the slots of its sums and counts, in slot order;
+ * host6 (optional): pinned host memory that receives them as well, so that a
+ * caller needs no copy after the launch */
+__global__ void __launch_bounds__(1024) k_norms_final_slots(const double *partial, int nsm, int nsc, double *out6,
+                                                            double *host6) {
     const int f = blockIdx.x;
     const double *ps = f == 2 ? partial + 4 * (size_t)nsm : partial + 2 * f * (size_t)nsm;
     const int n = f == 2 ? nsc : nsm;
@@ -1988,11 +2044,15 @@ __global__ void __launch_bounds__(1024) k_norms_final_slots(const double *partia
         for (int q = 0; q < 1024 / 64; q++) { ts += ws[q][0]; tc += ws[q][1]; }
         out6[f] = ts;
         out6[3 + f] = tc;
+        if (host6) {
+            host6[f] = ts;
+            host6[3 + f] = tc;
+        }
     }
 }
 
 int mdz_launch_residual_norms(int kind, const DevAsm &a, DevBlock *A, DevBlock *C, DevBlock *D, double *partial,
-                              size_t partial_len, double *out6, hipStream_t s, int d_scaled) {
+                              size_t partial_len, double *out6, hipStream_t s, int d_scaled, double *host6) {
     const int nm = a.e.neq_mom, ncnt = a.e.neq_cont;
     if (nm > 0 && (!A->free_row || !A->gen_waves)) return MDZ_EINVAL;
     if (kind == 0 && nm > 0 && A->free_node && a.d11p == a.d22p) {
@@ -2006,7 +2066,7 @@ int mdz_launch_residual_norms(int kind, const DevAsm &a, DevBlock *A, DevBlock *
             hipLaunchKernelGGL(k_residual_tile<true>, dim3(ngb + nt), dim3(RT_TX * RT_TZ), 0, s, a, *A, *C, *D,
                                (const unsigned char *)A->free_node, d_scaled, ntx, ngb, ns);
             hipLaunchKernelGGL(k_norms_final_slots, dim3(3), dim3(1024), 0, s, (const double *)partial, nt + ngen, nt,
-                               out6);
+                               out6, host6);
             return MDZ_OK;
         }
     }
@@ -2023,7 +2083,8 @@ int mdz_launch_residual_norms(int kind, const DevAsm &a, DevBlock *A, DevBlock *
         }
     }
     if (ncnt > 0) hipLaunchKernelGGL(k_residual_cont<true>, dim3(nbc), dim3(BLK), 0, s, kind, a, *C, *D, ns);
-    hipLaunchKernelGGL(k_norms_final_slots, dim3(3), dim3(1024), 0, s, (const double *)partial, nbf + ngen, nbc, out6);
+    hipLaunchKernelGGL(k_norms_final_slots, dim3(3), dim3(1024), 0, s, (const double *)partial, nbf + ngen, nbc, out6,
+                       host6);
     return MDZ_OK;
 }
 

@@ -97,6 +97,10 @@ void mdz_launch_residual(int kind, const DevAsm &a, DevBlock *A, DevBlock *C, De
  * (sum_x, sum_z, sum_p, ndof_x, ndof_z, ndof_p) */
 size_t mdz_norm_partials(const DevGrid &g);
 void mdz_launch_norms(const DevAsm &a, DevBlock *A, DevBlock *D, double *partial, double *out6, hipStream_t s);
+/* the value passes of both families (P Picard, J Jacobian) in one launch;
+ * false, with nothing enqueued, where they are better apart or one of them
+ * cannot take the split pass */
+bool mdz_launch_values_pair(const DevAsm &a, DevBlock *P, DevBlock *J, int vblk_p, int vblk_j, hipStream_t s);
 /* the waves of A that are not all free rows, into A->gen_waves / A->n_gen
  * (after the free-row flags; A->gen_waves holds 2 * (neq_mom / 64 + 2)
  * ints: the list, then the flags and their scan; synchronises s to read
@@ -107,12 +111,14 @@ int mdz_build_general_waves(DevBlock *A, int neq_mom, int *scratch, size_t scrat
  * mdz_launch_norms.  partial: at least mdz_residual_norm_partials(...)
  * doubles (MDZ_ENOMEM when partial_len is smaller).  For kind 0 with the
  * free-node flags built, the free momentum rows and the continuity rows
- * run in LDS tiles (k_residual_tile) and the general launch takes only the
- * other rows of the listed waves.  d_scaled = 0: every d is 1 (F *= d is
- * skipped, with the same result). */
+ * run in LDS tiles (k_residual_tile), whose first blocks take the other rows
+ * of the listed waves.  d_scaled = 0: every d is 1 (F *= d is skipped, with
+ * the same result).  host6 (optional, pinned host memory): the six sums
+ * again, readable once the stream has been synchronised. */
 size_t mdz_residual_norm_partials(int neq_mom, int n_gen, int neq_cont);
 int mdz_launch_residual_norms(int kind, const DevAsm &a, DevBlock *A, DevBlock *C, DevBlock *D, double *partial,
-                              size_t partial_len, double *out6, hipStream_t s, int d_scaled = 1);
+                              size_t partial_len, double *out6, hipStream_t s, int d_scaled = 1,
+                              double *host6 = nullptr);
 
 /* diagonal scaling: d from the diagonals of A and D (ExtractDiagonalScale),
  * then A_ij d_i d_j with b, F scaled by d (ScaleMatrix) */

@@ -1,9 +1,11 @@
-"""GPU test of the 64-row value pass, whose one launch takes the listed general
-waves, the tag-free waves and the continuity rows as block ranges, against the
-pass with one lane per row and no staging: CSR values and right-hand sides are
-the same bit for bit.  The grids lie on both sides of the 2048 blocks up to
-which the Jacobian pass runs at two waves per SIMD (300 x 200 cells: 2800
-blocks), down to grids without a tag-free wave, with ragged last waves."""
+"""GPU test of the 64-row value passes, whose one launch takes the listed general
+waves, the tag-free waves and the continuity rows as block ranges -- of one
+block family, or of both -- against the pass with one lane per row and no
+staging: CSR values and right-hand sides are the same bit for bit.  The grids
+lie on both sides of the 2048 blocks up to which both families share a launch
+(180 x 120 cells: 2018 and the general waves) and up to which the Jacobian
+pass runs at two waves per SIMD (300 x 200 cells: 2800 blocks), down to grids
+without a tag-free wave, with ragged last waves."""
 import ctypes as C
 
 import numpy as np
@@ -22,7 +24,7 @@ def _values(mdz, hot, ctx, which):
     return A, b, bbc
 
 
-@pytest.mark.parametrize("cells", [(5, 4), (33, 16), (161, 97), (300, 200)], ids=lambda c: "%dx%d" % c)
+@pytest.mark.parametrize("cells", [(5, 4), (33, 16), (140, 90), (180, 120), (300, 200)], ids=lambda c: "%dx%d" % c)
 def test_one_launch_of_the_value_pass_equals_the_direct_pass(mdz, hot, cells):
     m = mdz.Model.lithosphere(cells[0], cells[1], 6)
     c = C.c_void_p()
