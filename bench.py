@@ -39,9 +39,10 @@ def stage_kernels(shape, learned=False, fused=True, net_in_rheology=True):
     rh, pic, jac = shape
 
     def values(kind, rows, capa, capb):
-        # 64-row blocks: the split pass (the listed general waves, then the tag-free ones)
+        # 64-row blocks: the split pass (the listed general waves, then the
+        # tag-free ones; its instance for grids above 2048 blocks)
         if rows == 64:
-            return ["k_values_split<%d, %d, %d>" % (kind, capa, capb)]
+            return ["k_values_split<%d, %d, %d, %d>" % (kind, capa, capb, (6, 3)[kind])]
         if rows:
             return ["k_values_mom<%d, %d, %d, %d>" % (kind, rows, capa, capb)]
         return ["k_values_mom_direct<%d>" % kind, "k_values_cont"]

@@ -1290,18 +1290,18 @@ extern "C" int mdz_ctx_set_rheology_mode(mdz_ctx *c, int mode) {
 }
 
 /* residual rows of block family `kind` and their norms into c->norm_out
- * (and host6, see mdz_launch_residual_norms) */
-static int residual_norms(mdz_ctx *c, int kind, const DevAsm &a, hipStream_t s, double *host6 = nullptr) {
+ * (and copy6, see mdz_launch_residual_norms) */
+static int residual_norms(mdz_ctx *c, int kind, const DevAsm &a, hipStream_t s, double *copy6 = nullptr) {
     int rc = mdz_launch_residual_norms(kind, a, &c->blk[4 * kind], &c->blk[4 * kind + 2], &c->blk[4 * kind + 3],
-                                       c->norm_partial, c->norm_partial_len, c->norm_out, s, c->d_scaled[kind], host6);
+                                       c->norm_partial, c->norm_partial_len, c->norm_out, s, c->d_scaled[kind], copy6);
     return rc ? set_err(rc, "residual norms") : MDZ_OK;
 }
 
 /* One Newton-iteration unit of a context, enqueued on stream s with no
  * allocation, memset, host synchronisation or copy: safe to capture into a
- * graph.  The norms stay in c->norm_out (six doubles); host6 (optional,
+ * graph.  The norms stay in c->norm_out (six doubles); copy6 (optional,
  * pinned) receives them too. */
-static int enqueue_unit(mdz_ctx *c, hipStream_t s, double *host6 = nullptr) {
+static int enqueue_unit(mdz_ctx *c, hipStream_t s, double *copy6 = nullptr) {
     DevAsm a = make_asm(c), ap = picard_asm(c);
     mdz_launch_strain_interp5(c->g, c->prm, s);
     int rc = rheology_pass(c, c->prm.rheo_mode == MDZ_RHEO_LEARNED, s, true);
@@ -1311,7 +1311,7 @@ static int enqueue_unit(mdz_ctx *c, hipStream_t s, double *host6 = nullptr) {
         mdz_launch_rhs_dtensor(c->g, c->prm, 2, c->xg, c->zvx, c->xvz, c->zg, c->status, s, c->dpic_n, c->dpic_s);
         const bool pair = mdz_launch_values_pair(ap, &c->blk[0], &c->blk[4], c->shape.pic, c->shape.jac, s);
         if (!pair) mdz_launch_values(0, ap, &c->blk[0], &c->blk[1], &c->blk[2], &c->blk[3], c->shape.pic, s);
-        if ((rc = residual_norms(c, 0, ap, s, host6))) return rc;
+        if ((rc = residual_norms(c, 0, ap, s, copy6))) return rc;
         if (!pair) mdz_launch_values(1, a, &c->blk[4], &c->blk[5], &c->blk[6], &c->blk[7], c->shape.jac, s);
         c->d_jac = 1;
         return MDZ_OK;
@@ -1321,7 +1321,7 @@ static int enqueue_unit(mdz_ctx *c, hipStream_t s, double *host6 = nullptr) {
     mdz_launch_dtensor(c->g, c->prm, 1, c->status, s);
     mdz_launch_values(1, a, &c->blk[4], &c->blk[5], &c->blk[6], &c->blk[7], c->shape.jac, s);
     mdz_launch_dtensor(c->g, c->prm, 0, c->status, s);
-    return residual_norms(c, kind, a, s, host6);
+    return residual_norms(c, kind, a, s, copy6);
 }
 
 /* resx, resz, resp from the six sums of the norm kernels */
@@ -1890,10 +1890,6 @@ __global__ void __launch_bounds__(1024) k_apply_bc(DevGrid g) {
         if (tu[j * nx + nx - 1] == -12) u[j * nx + nx - 1] = u[j * nx];
 }
 
-__global__ void k_copy6(const double *__restrict__ src, double *__restrict__ dst) {
-    if (threadIdx.x < 6) dst[threadIdx.x] = src[threadIdx.x];
-}
-
 /* Device buffers of a line search: the saved iterate (u, v, p), the
  * correction by equation number, the step lengths and six norm sums per
  * trial. */
@@ -1923,9 +1919,7 @@ static int enqueue_trial(mdz_ctx *c, const LsBufs &lb, int k, hipStream_t s) {
     if (fused) a = picard_asm(c);
     mdz_launch_rhs_dtensor(c->g, c->prm, fused ? 3 : 0, c->xg, c->zvx, c->xvz, c->zg, c->status, s,
                            fused ? c->dpic_n : nullptr, fused ? c->dpic_s : nullptr);
-    if ((rc = residual_norms(c, kind, a, s))) return rc;
-    hipLaunchKernelGGL(k_copy6, dim3(1), dim3(64), 0, s, (const double *)c->norm_out, lb.res + 6 * k);
-    return MDZ_OK;
+    return residual_norms(c, kind, a, s, lb.res + 6 * k);
 }
 
 extern "C" int mdz_ctx_line_search(mdz_ctx *c, const double *dx, int ntry, const double *alpha, double *res3n) {

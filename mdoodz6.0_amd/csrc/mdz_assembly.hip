@@ -2021,10 +2021,10 @@ size_t mdz_residual_norm_partials(int nm, int n_gen, int ncnt) {
 }
 
 /* one block per family: the slots of its sums and counts, in slot order;
- * host6 (optional): pinned host memory that receives them as well, so that a
- * caller needs no copy after the launch */
+ * copy6 (optional): a second place for them, in device or pinned host
+ * memory, so that a caller needs no copy after the launch (5 us) */
 __global__ void __launch_bounds__(1024) k_norms_final_slots(const double *partial, int nsm, int nsc, double *out6,
-                                                            double *host6) {
+                                                            double *copy6) {
     const int f = blockIdx.x;
     const double *ps = f == 2 ? partial + 4 * (size_t)nsm : partial + 2 * f * (size_t)nsm;
     const int n = f == 2 ? nsc : nsm;
@@ -2044,15 +2044,15 @@ __global__ void __launch_bounds__(1024) k_norms_final_slots(const double *partia
         for (int q = 0; q < 1024 / 64; q++) { ts += ws[q][0]; tc += ws[q][1]; }
         out6[f] = ts;
         out6[3 + f] = tc;
-        if (host6) {
-            host6[f] = ts;
-            host6[3 + f] = tc;
+        if (copy6) {
+            copy6[f] = ts;
+            copy6[3 + f] = tc;
         }
     }
 }
 
 int mdz_launch_residual_norms(int kind, const DevAsm &a, DevBlock *A, DevBlock *C, DevBlock *D, double *partial,
-                              size_t partial_len, double *out6, hipStream_t s, int d_scaled, double *host6) {
+                              size_t partial_len, double *out6, hipStream_t s, int d_scaled, double *copy6) {
     const int nm = a.e.neq_mom, ncnt = a.e.neq_cont;
     if (nm > 0 && (!A->free_row || !A->gen_waves)) return MDZ_EINVAL;
     if (kind == 0 && nm > 0 && A->free_node && a.d11p == a.d22p) {
@@ -2066,7 +2066,7 @@ int mdz_launch_residual_norms(int kind, const DevAsm &a, DevBlock *A, DevBlock *
             hipLaunchKernelGGL(k_residual_tile<true>, dim3(ngb + nt), dim3(RT_TX * RT_TZ), 0, s, a, *A, *C, *D,
                                (const unsigned char *)A->free_node, d_scaled, ntx, ngb, ns);
             hipLaunchKernelGGL(k_norms_final_slots, dim3(3), dim3(1024), 0, s, (const double *)partial, nt + ngen, nt,
-                               out6, host6);
+                               out6, copy6);
             return MDZ_OK;
         }
     }
@@ -2084,7 +2084,7 @@ int mdz_launch_residual_norms(int kind, const DevAsm &a, DevBlock *A, DevBlock *
     }
     if (ncnt > 0) hipLaunchKernelGGL(k_residual_cont<true>, dim3(nbc), dim3(BLK), 0, s, kind, a, *C, *D, ns);
     hipLaunchKernelGGL(k_norms_final_slots, dim3(3), dim3(1024), 0, s, (const double *)partial, nbf + ngen, nbc, out6,
-                       host6);
+                       copy6);
     return MDZ_OK;
 }
 

@@ -113,12 +113,13 @@ int mdz_build_general_waves(DevBlock *A, int neq_mom, int *scratch, size_t scrat
  * free-node flags built, the free momentum rows and the continuity rows
  * run in LDS tiles (k_residual_tile), whose first blocks take the other rows
  * of the listed waves.  d_scaled = 0: every d is 1 (F *= d is skipped, with
- * the same result).  host6 (optional, pinned host memory): the six sums
- * again, readable once the stream has been synchronised. */
+ * the same result).  copy6 (optional, device or pinned host memory): the
+ * six sums again; on the host readable once the stream has been
+ * synchronised. */
 size_t mdz_residual_norm_partials(int neq_mom, int n_gen, int neq_cont);
 int mdz_launch_residual_norms(int kind, const DevAsm &a, DevBlock *A, DevBlock *C, DevBlock *D, double *partial,
                               size_t partial_len, double *out6, hipStream_t s, int d_scaled = 1,
-                              double *host6 = nullptr);
+                              double *copy6 = nullptr);
 
 /* diagonal scaling: d from the diagonals of A and D (ExtractDiagonalScale),
  * then A_ij d_i d_j with b, F scaled by d (ScaleMatrix) */

@@ -825,9 +825,10 @@ enum { RHEO_BOTH, RHEO_CELLS, RHEO_VERTICES };
  * and the first vertex waves share the chip (41 x 41 nodes: 13 us against
  * 13 + 10, 1001 x 501: 119 against 79 + 62).  With the network's guess in the
  * pass (NET) a vertex reads the network outputs of its centroids, which the
- * centroid blocks write: then each has its own launch.  Two waves per SIMD: every variant fits 256 registers without
- * scratch; one wave per SIMD left the FP64 latency exposed.  Dynamic LDS:
- * the stash, (StashSlots::nd + max(Nb_phases, 4)) * NT doubles. */
+ * centroid blocks write: then each has its own launch.  Two waves per SIMD:
+ * every variant fits 256 registers (with both ranges and every output, 36
+ * bytes of scratch); one wave per SIMD left the FP64 latency exposed.
+ * Dynamic LDS: the stash, (StashSlots::nd + max(Nb_phases, 4)) * NT doubles. */
 template <int NT, bool DIAG, bool NET, int PART>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
 k_rheo_fast(DevGrid g, DevParams prm, FastConst fc, const PhaseK *__restrict__ pk, double R,
