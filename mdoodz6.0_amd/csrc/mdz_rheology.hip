@@ -8,8 +8,8 @@
  *   k_strain_tile                                   RheologyDensity.c:1902-1982 (+ GridRoutines.c:106)
  *   k_interp_c2v                                    GridRoutines.c:106-196
  *   k_rheo_cells / k_rheo_vertices                  RheologyDensity.c:961-1415
- *   k_dtensor_cells / k_dtensor_vertices            RheologyDensity.c:713-954
- *   k_rhs_u / k_rhs_v / k_rhs_p                     StokesRoutines.c:922-1128
+ *   dtensor_cell / dtensor_vertex (k_rhs_dtensor)   RheologyDensity.c:713-954
+ *   rhs_u / rhs_v / rhs_p (k_rhs_dtensor)           StokesRoutines.c:922-1128
  *
  * All HBM-bound except the rheology, which is FP64-VALU bound
  * (transcendentals of the local iterations).
