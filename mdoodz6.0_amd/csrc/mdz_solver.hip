@@ -424,12 +424,14 @@ __global__ void __launch_bounds__(SV_BLK) k_gcr_product(int n, SliceView M, cons
 
 /* v -= sum_q val[q] VV[q] and s -= sum_q val[q] SS[q], one term after the
  * other (Solvers.c:164-168): val[q] = v . VV[q] for q < i1, and from the
- * second cycle on val[i1] of the cycle before; rows 0, 1 of fv: f . v, v . v */
+ * second cycle on val[i1] of the cycle before -- but for the last direction
+ * of a cycle, whose val is set in none (0 in the reference, never written
+ * here); rows 0, 1 of fv: f . v, v . v */
 __global__ void __launch_bounds__(SV_BLK) k_gcr_orth(int n, int i1, int cycle, const double *dots, double *val,
                                                      const double *VV, const double *SS, size_t ldv, const double *f,
                                                      double *v, double *s, double *fv) {
     __shared__ double sval[SV_RESTART], lds4[4];
-    const int w = threadIdx.x >> 6, nq = i1 + (cycle > 0);
+    const int w = threadIdx.x >> 6, nq = i1 + (cycle > 0 && i1 < SV_RESTART - 1);
     for (int q = w; q < nq; q += 4) {
         const double x = q < i1 ? slots_sum(dots + q * SV_RED) : val[q];
         if ((threadIdx.x & 63) == 0) {

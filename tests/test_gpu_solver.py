@@ -311,3 +311,53 @@ def test_device_solve_matches_oracle_513x257(mdz, orc, hot):
         if gpu:
             gpu.close()
         m.free()
+
+
+def _fill_freed_memory(hot, byte=0xFF):
+    """Device memory for the next small and large allocations to find: buffers
+    filled with `byte` (0xFF: NaN), every other one freed -- the others, returned, keep
+    the freed ones from going back to the system."""
+    kept = []
+    for size, count in ((1 << 10, 4096), (1 << 18, 64), (1 << 22, 32)):
+        ptrs = [C.c_void_p() for _ in range(count)]
+        for q in ptrs:
+            assert hot.hipMalloc(C.byref(q), C.c_size_t(size)) == 0
+            assert hot.hipMemset(q, C.c_int(byte), C.c_size_t(size)) == 0
+        assert hot.hipDeviceSynchronize() == 0
+        for q in ptrs[::2]:
+            assert hot.hipFree(q) == 0
+        kept += ptrs[1::2]
+    return kept
+
+
+def test_restarted_gcr_in_used_memory(mdz, orc, hot):
+    """One GCR call of three cycles (77 directions), the solver's buffers in
+    memory that held NaN before: the oracle's counts.  kspgcr subtracts
+    val[i1] of the cycle before, which is never set for the last direction
+    of a cycle: 0 there, whatever the buffer held."""
+    print("case pwl, rel_tol_KSP 3e-7", flush=True)
+    m = mdz.Model.pwl_inclusion(60, 60)
+    m.m.model.penalty = 1e5
+    m.m.model.rel_tol_KSP = 3e-7
+    gpu, kept = None, []
+    try:
+        it = nd.Iterate(mdz, orc, m)
+        gpu = nd.GpuAssembler(mdz, hot, m, it)
+        gpu()
+        sysm = System(mdz, hot, gpu.ctx, it, m)
+        du, dp, oi = orc_solver.killer_solver(sysm.A, sysm.B, sysm.C, sysm.AJ, sysm.BJ, sysm.CJ, sysm.Dpen, sysm.D1,
+                                              sysm.inc, sysm.bu, sysm.bp, rel_tol_KSP=3e-7)
+        assert max(oi["ksp_its"]) > 2 * orc_solver.RESTART
+        kept = _fill_freed_memory(hot)
+        dx, info = _solve(mdz, hot, gpu.ctx, it.neq_mom + it.neq_cont, 0)
+        ksp = list(info.ksp_its[:info.ph_its])
+        ddu = np.linalg.norm(dx[:it.neq_mom] - du) / np.linalg.norm(du)
+        print("ksp", ksp, oi["ksp_its"], "du %.2e" % ddu)
+        assert ksp == oi["ksp_its"]
+        assert ddu < 1e-5
+    finally:
+        for q in kept:
+            hot.hipFree(q)
+        if gpu:
+            gpu.close()
+        m.free()
