@@ -547,9 +547,11 @@ int  mdz_ctx_solve(mdz_ctx *ctx, int nb, double *dx, mdz_solve_info *info);
  * reference): threads per block of the rheology kernels (64, 128, 256),
  * rows per block of the LDS-staged Picard (0 = unstaged, 64, 128, 256) and
  * Jacobian (0, 64, 128) value kernels; 64 rows take the split pass (the
- * tag-free row code over every wave, then the general row code over the
- * waves that hold a boundary row).  Default 64, 128, 64.  Results do not
- * depend on them. */
+ * general row code over the waves that hold a boundary row beside the
+ * tag-free row code over the others).  Default 64, 128, 64.  A unit on a
+ * small grid takes both value passes in one launch of 64-row blocks, unless
+ * a shape other than 64, 64 has been set for them here.  Results do not
+ * depend on any of it. */
 int  mdz_ctx_set_launch_shape(mdz_ctx *ctx, int rheo, int pic, int jac);
 int  mdz_ctx_get_launch_shape(mdz_ctx *ctx, int *shape3);
 

@@ -1309,7 +1309,7 @@ static int enqueue_unit(mdz_ctx *c, hipStream_t s, double *copy6 = nullptr) {
     const int kind = c->model.aniso == 1 ? 1 : 0;
     if (fused_dtensor(c)) {
         mdz_launch_rhs_dtensor(c->g, c->prm, 2, c->xg, c->zvx, c->xvz, c->zg, c->status, s, c->dpic_n, c->dpic_s);
-        const bool pair = mdz_launch_values_pair(ap, &c->blk[0], &c->blk[4], c->shape.pic, c->shape.jac, s);
+        const bool pair = mdz_launch_values_pair(ap, &c->blk[0], &c->blk[4], c->shape, s);
         if (!pair) mdz_launch_values(0, ap, &c->blk[0], &c->blk[1], &c->blk[2], &c->blk[3], c->shape.pic, s);
         if ((rc = residual_norms(c, 0, ap, s, copy6))) return rc;
         if (!pair) mdz_launch_values(1, a, &c->blk[4], &c->blk[5], &c->blk[6], &c->blk[7], c->shape.jac, s);
@@ -2288,7 +2288,7 @@ extern "C" void KillerSolver(SparseMat *matA, SparseMat *matB, SparseMat *matC, 
 
 extern "C" int mdz_ctx_set_launch_shape(mdz_ctx *c, int rheo, int pic, int jac) {
     if (!c) return set_err(MDZ_EINVAL, "NULL context");
-    LaunchShape sh{rheo, pic, jac};
+    LaunchShape sh{rheo, pic, jac, true};
     if (!mdz_shape_valid(sh))
         return set_err(MDZ_EINVAL, "launch shape (%d, %d, %d): rheology 64/128/256, Picard 0/64/128/256, Jacobian 0/64/128",
                        rheo, pic, jac);
@@ -2589,6 +2589,7 @@ extern "C" int mdz_ensemble_autotune(mdz_ensemble *e, int reps, int *report, int
         }
         mdz_ctx *c = e->ctx[rep];
         LaunchShape best = c->shape;
+        best.asked = false;
         for (int stage = 0; stage < 3 && !rc; stage++) {
             /* two rounds over the candidates, the second in reverse order,
              * and each candidate's faster round: a candidate timed while the

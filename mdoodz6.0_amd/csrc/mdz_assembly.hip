@@ -1889,11 +1889,12 @@ static void launch_split(const DevAsm &a, DevBlock *A, DevBlock *B, DevBlock *C,
  * once: there each pass is the latency of its general waves (18 and 9 us at
  * 41 x 41 nodes), which overlap.  Beyond it the Picard pass would lose the six
  * waves per SIMD that it has on its own. */
-bool mdz_launch_values_pair(const DevAsm &a, DevBlock *P, DevBlock *J, int vblk_p, int vblk_j, hipStream_t s) {
+bool mdz_launch_values_pair(const DevAsm &a, DevBlock *P, DevBlock *J, const LaunchShape &shape, hipStream_t s) {
     const bool split = P->free_row && P->gen_waves && J->free_row && J->gen_waves;
     const bool fits = P[0].maxrow <= PIC_CAPA && P[1].maxrow <= PIC_CAPB && J[0].maxrow <= JAC_CAPA &&
                       J[1].maxrow <= JAC_CAPB;
-    if (a.e.neq_mom <= 0 || vblk_p == 0 || vblk_j != 64 || !split || !fits) return false;
+    const bool rows64 = shape.jac == 64 && (shape.asked ? shape.pic == 64 : shape.pic != 0);
+    if (a.e.neq_mom <= 0 || !rows64 || !split || !fits) return false;
     const int nbm = mdz_div_up(a.e.neq_mom, 64), nbc = mdz_div_up(a.e.neq_cont, 64);
     const int grid = P->n_gen + J->n_gen + 2 * (nbm + nbc);
     if (grid > SPLIT_ROUND2) return false;

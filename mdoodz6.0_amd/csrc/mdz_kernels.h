@@ -76,6 +76,7 @@ void mdz_fill_pattern(int kind, const DevAsm &a, DevBlock *A, DevBlock *B, DevBl
  * same values bit for bit: the per-row arithmetic does not depend on it. */
 struct LaunchShape {
     int rheo, pic, jac;
+    bool asked = false; /* by a caller, who gets this shape and no other */
 };
 /* the shape the autotuner picks at 2049 x 1025 (64-row value blocks take
  * the split pass: tag-free waves, then the listed general waves) */
@@ -98,9 +99,9 @@ void mdz_launch_residual(int kind, const DevAsm &a, DevBlock *A, DevBlock *C, De
 size_t mdz_norm_partials(const DevGrid &g);
 void mdz_launch_norms(const DevAsm &a, DevBlock *A, DevBlock *D, double *partial, double *out6, hipStream_t s);
 /* the value passes of both families (P Picard, J Jacobian) in one launch;
- * false, with nothing enqueued, where they are better apart or one of them
- * cannot take the split pass */
-bool mdz_launch_values_pair(const DevAsm &a, DevBlock *P, DevBlock *J, int vblk_p, int vblk_j, hipStream_t s);
+ * false, with nothing enqueued, where they are better apart, one of them
+ * cannot take the split pass, or a caller asked for another shape */
+bool mdz_launch_values_pair(const DevAsm &a, DevBlock *P, DevBlock *J, const LaunchShape &shape, hipStream_t s);
 /* the waves of A that are not all free rows, into A->gen_waves / A->n_gen
  * (after the free-row flags; A->gen_waves holds 2 * (neq_mom / 64 + 2)
  * ints: the list, then the flags and their scan; synchronises s to read
