@@ -316,6 +316,15 @@ __device__ __forceinline__ void train_act(f32x4 (*z)[4], bf16x4 (*h)[4], unsigne
         }
 }
 
+/* LDS ordering between the lanes of one wave.  DS instructions of a wave run
+ * in the order they are issued, so that nothing has to be waited for; the
+ * fence (no instruction at this scope) keeps the compiler from moving an
+ * access across. */
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 /* sum of a staged row over its 32 samples */
 __device__ __forceinline__ float row_sum(const unsigned short *row) {
     float sum = 0.0f;
@@ -333,7 +342,7 @@ __device__ __forceinline__ float row_sum(const unsigned short *row) {
 __device__ __forceinline__ void train_grad(const f32x4 (*d)[4], const f32x4 (*dact)[4], bf16x4 (*bd)[4],
                                            unsigned short *Ds) {
     const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_order();
 #pragma unroll
     for (int g = 0; g < 2; g++)
 #pragma unroll
@@ -342,7 +351,7 @@ __device__ __forceinline__ void train_grad(const f32x4 (*d)[4], const f32x4 (*da
 #pragma unroll
             for (int i = 0; i < 4; i++) Ds[(16 * t + 4 * q + i) * TSW + 16 * g + r] = (unsigned short)bd[g][t][i];
         }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_order();
 }
 
 /* g[mt][nt] += D H^T over the 32 staged samples */
@@ -471,7 +480,7 @@ __global__ void __launch_bounds__(TWAVES * 64, 1) k_mlp_train_step(
 #pragma unroll
             for (int i = 0; i < 4; i++) D4s[(4 * q + i) * TSW + 16 * g + r] = (unsigned short)b4[g][0][i];
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
         gb4 += row_sum(D4s + r * TSW);
         {
             const bf16x8 a = lds8(D4s + r * TSW + 8 * q);
@@ -493,7 +502,7 @@ __global__ void __launch_bounds__(TWAVES * 64, 1) k_mlp_train_step(
         const bf16x8 xt = lds8(Xs + r * TSW + 8 * q);
 #pragma unroll
         for (int mt = 0; mt < 4; mt++) g1[mt] = mfma32(lds8(Ds + (16 * mt + r) * TSW + 8 * q), xt, g1[mt]);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
     }
 
     /* the block's gradient: wave wv adds part (2 wv + k) mod 8 in round k (the
