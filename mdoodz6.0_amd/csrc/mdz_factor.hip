@@ -110,7 +110,8 @@ __device__ __forceinline__ double nd_rsqrt(double p) {
 __device__ __forceinline__ void nd_potrf(double *S, int w, double *__restrict__ out, double *T, int ldt, int pos0,
                                          int *bad) {
     double *V = S + ND_DIAG, *buf = V + ND_T * ND_T;
-    double *piv = buf; /* 64 pivots; then two buffers of four columns and four reciprocal pivots */
+    double *piv = buf; /* 64 pivots; then two buffers of four columns, each with 32 doubles more for the
+                        * owner's reads past its sixteen */
     const int r = threadIdx.x & 63, q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nb = (w + 15) >> 4, W = nb << 4;
     double a[16];
@@ -737,6 +738,7 @@ int mdz_factor_analyse(MdzFactor *F, int Nx, int Nz, int n, const int *mom_node,
         (rc = nd_reserve(F->x, (size_t)n)) || (rc = nd_reserve(F->g, p.blist.size() + 1)))
         return rc;
     FCHK(hipMemsetAsync(F->g.p, 0, (p.blist.size() + 1) * sizeof(double), F->s));
+    p.release_uploaded();
     F->n = n;
     return MDZ_OK;
 }

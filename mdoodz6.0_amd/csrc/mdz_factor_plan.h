@@ -75,6 +75,15 @@ struct NdPlan {
     std::vector<int> pos, eq, node_of; /* position of an equation, and back; node of a position */
     std::vector<int> blist, inv;
     size_t panel_len = 0, ulen[2] = {0, 0}, nlin = 0;
+
+    /* gives back what only the device reads, once it is there: level, invert, eq and the
+     * lengths remain */
+    void release_uploaded() {
+        std::vector<NdNode>().swap(node);
+        std::vector<NdTask>().swap(task);
+        std::vector<NdSolve>().swap(solve);
+        for (std::vector<int> *v : {&at, &pos, &node_of, &blist, &inv}) std::vector<int>().swap(*v);
+    }
 };
 
 namespace {

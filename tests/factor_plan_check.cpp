@@ -160,6 +160,17 @@ static int check(int Nx, int Nz, int reach, bool periodic, double drop, int seed
         den += b[i] * b[i];
     }
     const double err = sqrt(num / den);
+    /* what the device holds is given back; the next analysis makes the same plan */
+    const std::vector<int> pos = p.pos, at_kept = p.at, blist = p.blist, inv = p.inv, node_of = p.node_of;
+    const size_t counts[3] = {p.node.size(), p.task.size(), p.solve.size()};
+    p.release_uploaded();
+    ok = ok && p.node.capacity() + p.task.capacity() + p.solve.capacity() + p.at.capacity() + p.pos.capacity() +
+                       p.node_of.capacity() + p.blist.capacity() + p.inv.capacity() ==
+                   0;
+    ok = ok && !p.level.empty() && (int)p.eq.size() == n;
+    if (nd_plan(p, Nx, Nz, n, mom.data(), Ic, J)) return 1;
+    ok = ok && p.pos == pos && p.at == at_kept && p.blist == blist && p.inv == inv && p.node_of == node_of &&
+         p.node.size() == counts[0] && p.task.size() == counts[1] && p.solve.size() == counts[2];
     printf("%d x %d reach %d periodic %d drop %.1f: %d unknowns, %zu fronts, %zu levels, residual %.1e\n", Nx, Nz, reach,
            (int)periodic, drop, n, F.size(), p.level.size(), err);
     return !(ok && err < 1e-12);
