@@ -1465,7 +1465,6 @@ __device__ __forceinline__ void tile_load(double (&dst)[H][W], signed char (*tds
     }
 }
 
-template <bool NORM>
 __global__ void __launch_bounds__(RT_TX * RT_TZ) __attribute__((amdgpu_waves_per_eu(8)))
 k_residual_tile(DevAsm a, DevBlock A, DevBlock C, DevBlock D, const unsigned char *__restrict__ free_node, int scaled,
                 int ntx, int ngb, NormSlots ns) {
@@ -1475,7 +1474,7 @@ k_residual_tile(DevAsm a, DevBlock A, DevBlock C, DevBlock D, const unsigned cha
     const int nu = Nx * nzvx;
     /* the listed general waves first, one per wave of the block: their long
      * load chains run beside the tiles */
-    if (NORM && (int)blockIdx.x < ngb) {
+    if ((int)blockIdx.x < ngb) {
         const int slot = blockIdx.x * (RT_TX * RT_TZ / 64) + ((int)threadIdx.x >> 6);
         if (slot < A.n_gen) residual_general_wave(a, A, ns, slot);
         return;
@@ -1528,13 +1527,9 @@ k_residual_tile(DevAsm a, DevBlock A, DevBlock C, DevBlock D, const unsigned cha
         f -= bu;
         const double F = f * cv;
         A.b[equ] = bu;
-        if (NORM) {
-            g.ru[un] = F;
-            vsum[0] = F * F; vsum[1] = 1.0;
-            A.F[equ] = scaled ? F * A.d[equ] : F;
-        } else {
-            A.F[equ] = F;
-        }
+        g.ru[un] = F;
+        vsum[0] = F * F; vsum[1] = 1.0;
+        A.F[equ] = scaled ? F * A.d[equ] : F;
     }
     if (fv) {
         /* z-momentum row of v(i, j) (zmom_inner, tag-free) */
@@ -1561,13 +1556,9 @@ k_residual_tile(DevAsm a, DevBlock A, DevBlock C, DevBlock D, const unsigned cha
         f -= bv;
         const double F = f * cv;
         A.b[eqv] = bv;
-        if (NORM) {
-            g.rv[vn] = F;
-            vsum[2] = F * F; vsum[3] = 1.0;
-            A.F[eqv] = scaled ? F * A.d[eqv] : F;
-        } else {
-            A.F[eqv] = F;
-        }
+        g.rv[vn] = F;
+        vsum[2] = F * F; vsum[3] = 1.0;
+        A.F[eqv] = scaled ? F * A.d[eqv] : F;
     }
     if (hc && eqp >= 0) {
         /* continuity row of centroid (i, j) (continuity_row, Assemble = 0) */
@@ -1581,22 +1572,16 @@ k_residual_tile(DevAsm a, DevBlock A, DevBlock C, DevBlock D, const unsigned cha
         const double F = f * cv;
         C.b[row] = rp;
         C.F[row] = F;
-        if (NORM) {
-            g.rp[cn] = F;
-            vsum[4] = F * F; vsum[5] = 1.0;
-            D.F[row] = scaled ? F * D.d[row] : F;
-        } else {
-            D.F[row] = F;
-        }
+        g.rp[cn] = F;
+        vsum[4] = F * F; vsum[5] = 1.0;
+        D.F[row] = scaled ? F * D.d[row] : F;
     }
-    if (NORM) {
-        block_sums<6>(vsum);
-        if (threadIdx.x == 0) {
+    block_sums<6>(vsum);
+    if (threadIdx.x == 0) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) ns.partial[q * ns.nsm + tile] = vsum[q];
-            ns.partial[4 * ns.nsm + tile] = vsum[4];
-            ns.partial[4 * ns.nsm + ns.nsc + tile] = vsum[5];
-        }
+        for (int q = 0; q < 4; q++) ns.partial[q * ns.nsm + tile] = vsum[q];
+        ns.partial[4 * ns.nsm + tile] = vsum[4];
+        ns.partial[4 * ns.nsm + ns.nsc + tile] = vsum[5];
     }
 }
 
@@ -2064,7 +2049,7 @@ int mdz_launch_residual_norms(int kind, const DevAsm &a, DevBlock *A, DevBlock *
         if ((size_t)(4 * (nt + ngen) + 2 * nt) <= partial_len) {
             NormSlots ns{partial, nt + ngen, nt, nt, A->gen_waves};
             const int ngb = mdz_div_up(ngen, RT_TX * RT_TZ / 64);
-            hipLaunchKernelGGL(k_residual_tile<true>, dim3(ngb + nt), dim3(RT_TX * RT_TZ), 0, s, a, *A, *C, *D,
+            hipLaunchKernelGGL(k_residual_tile, dim3(ngb + nt), dim3(RT_TX * RT_TZ), 0, s, a, *A, *C, *D,
                                (const unsigned char *)A->free_node, d_scaled, ntx, ngb, ns);
             hipLaunchKernelGGL(k_norms_final_slots, dim3(3), dim3(1024), 0, s, (const double *)partial, nt + ngen, nt,
                                out6, copy6);
