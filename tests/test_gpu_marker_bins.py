@@ -29,23 +29,35 @@ def _check_step(mdz, orc, hot, m, mk, nph):
 
 
 @pytest.mark.parametrize("itp", [1, 9])
-@pytest.mark.parametrize("crowd", [511, 512, 513, 3000])
-def test_crowded_cell(mdz, orc, hot, crowd, itp):
-    """One quarter cell with `crowd` markers besides the others: up to 512
-    are ordered in place, more go through the radix sort."""
-    print("case crowd", crowd, itp, flush=True)
+@pytest.mark.parametrize("active", [511, 512, 513, 3000])
+def test_crowded_bin(mdz, orc, hot, active, itp):
+    """One bin -- the quarter cell of the 1-node stencil, the centroid's and
+    the vertex's of the 9-node one -- holds `active` active markers: up to
+    512 are ordered in place, more go through the radix sort."""
+    print("case active", active, itp, flush=True)
     m = mdz.Model.lithosphere(30, 20, 4)
     _softening(m)
     m.m.model.itp_stencil = itp
     mk = seed_markers(mdz, m, (2, 2), seed=3, phase="layers")
     g, p = m.m.mesh.contents, m.m.model
     rng = np.random.default_rng(1)
-    x = p.xmin + (7 + rng.uniform(0.05, 0.45, crowd)) * g.dx
-    z = p.zmin + (5 + rng.uniform(0.55, 0.95, crowd)) * g.dz
-    perm = rng.permutation(mk.n + crowd)
+
+    def in_bins(k):
+        """active markers of k in each of the stencil's bins around cell (7, 5)'s upper left quarter"""
+        x, z = (k.x - p.xmin) / g.dx, (k.z - p.zmin) / g.dz
+        cell, vertex = (np.floor(x) == 7) & (np.floor(z) == 5), (np.rint(x) == 7) & (np.rint(z) == 6)
+        return [int((b & (k.phase != -1)).sum()) for b in ([cell & vertex] if itp == 1 else [cell, vertex])]
+
+    crowd = active - in_bins(mk)[0]
+    n = crowd + 200  # (200 inactive ones among them)
+    x = p.xmin + (7 + rng.uniform(0.05, 0.45, n)) * g.dx
+    z = p.zmin + (5 + rng.uniform(0.55, 0.95, n)) * g.dz
+    phase = np.concatenate([rng.integers(0, 3, crowd), np.full(n - crowd, -1)])
+    perm = rng.permutation(mk.n + n)
     mk = Markers(mdz, np.concatenate([mk.x, x])[perm], np.concatenate([mk.z, z])[perm],
-                 np.concatenate([mk.phase, rng.integers(-1, 3, crowd)])[perm],
-                 np.concatenate([mk.strain_pl, rng.exponential(1.0, crowd)])[perm])
+                 np.concatenate([mk.phase, phase])[perm],
+                 np.concatenate([mk.strain_pl, rng.exponential(1.0, n)])[perm])
+    assert in_bins(mk) == [active] * (1 if itp == 1 else 2)
     try:
         _check_step(mdz, orc, hot, m, mk, 3)
     finally:
