@@ -383,7 +383,13 @@ __device__ __forceinline__ void weight_grad(const unsigned short *Ds, const unsi
  * through the parameters' eight parts, in an order that depends on nothing.
  * Measured, batch 65 536: a step 43 us with its reduction and Adam (47 with
  * one group a wave), against 105 for one block per 64 samples that wrote
- * 1024 partial gradients, a reduction of 37 MB and Adam. */
+ * 1024 partial gradients, a reduction of 37 MB and Adam.
+ *
+ * Up to a tile per CU (batches of 8192) a tile has a block to itself: its
+ * other waves help to read the weights, and its gradient goes from the
+ * registers to the partials, without the eight rounds and their barriers.
+ * A step of 1024 samples takes 18 us, 26 with four tiles a block (25 for the
+ * one block per 64 samples), one of 8192 26 against 28 (31). */
 __global__ void __launch_bounds__(TWAVES * 64, 1) k_mlp_train_step(
     const float *__restrict__ X, const float *__restrict__ Y, long long n, long long first, unsigned long long mul,
     unsigned long long add, long long stride, int tiles, float inv_batch, DevMLPW w, float *__restrict__ partial,
@@ -407,7 +413,8 @@ __global__ void __launch_bounds__(TWAVES * 64, 1) k_mlp_train_step(
                    *Xs = Ds + 64 * TSW, *D4s = Xs + 16 * TSW;
     f32x4 g1[4] = {}, g2[4][4] = {}, g3[4][4] = {}, g4[4] = {};
     float gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f, gb4 = 0.0f, se = 0.0f;
-    int tile = blockIdx.x * TWAVES + wv;
+    const bool solo = (int)gridDim.x >= tiles; /* a block for each tile */
+    int tile = solo ? (wv == 0 ? (int)blockIdx.x : tiles) : blockIdx.x * TWAVES + wv;
     long long idx[2];
     float f[2][4], tgt[2][2] = {};
 #pragma unroll
@@ -437,6 +444,7 @@ __global__ void __launch_bounds__(TWAVES * 64, 1) k_mlp_train_step(
     static_assert(MLP_BP_TOTAL <= TWAVES * 64, "one bias a thread");
     if (threadIdx.x < MLP_BP_TOTAL) sB[threadIdx.x] = bl;
     __syncthreads();
+    if (solo && wv) return; /* (no barrier follows for the first wave) */
     for (; tile < tiles; tile += gridDim.x * TWAVES) {
         bf16x4 x[2][1];
         float t[2][2];
@@ -505,14 +513,9 @@ __global__ void __launch_bounds__(TWAVES * 64, 1) k_mlp_train_step(
         wave_lds_order();
     }
 
-    /* the block's gradient: wave wv adds part (2 wv + k) mod 8 in round k (the
-     * first two rounds are the first to touch a part) */
-    float *sum = (float *)sA;
-#pragma unroll 1
-    for (int k = 0; k < 8; k++) {
-        __syncthreads();
-        const int part = (2 * wv + k) & 7;
-        auto put = [&](int p, float v) { sum[p] = k > 1 ? sum[p] + v : v; };
+    float *P = partial + (size_t)blockIdx.x * MLP_NPARAMS;
+    /* part 0..7 of the wave's gradient: put(parameter, value) */
+    auto each = [&](int part, auto &&put) {
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             if (part == c) {
@@ -541,11 +544,24 @@ __global__ void __launch_bounds__(TWAVES * 64, 1) k_mlp_train_step(
         if (part == 1) put(MLP_OFF_B2 + l, gb2);
         if (part == 2) put(MLP_OFF_B3 + l, gb3);
         if (part == 3 && l < MLP_OUT) put(MLP_OFF_B4 + l, gb4);
-    }
+    };
     for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o, 64);
+    if (solo) {
+#pragma unroll
+        for (int part = 0; part < 8; part++) each(part, [&](int p, float v) { P[p] = v; });
+        if (l == 0) loss[blockIdx.x] = se;
+        return;
+    }
+    /* the block's gradient: wave wv adds part (2 wv + k) mod 8 in round k (the
+     * first two rounds are the first to touch a part) */
+    float *sum = (float *)sA;
+#pragma unroll 1
+    for (int k = 0; k < 8; k++) {
+        __syncthreads();
+        each((2 * wv + k) & 7, [&](int p, float v) { sum[p] = k > 1 ? sum[p] + v : v; });
+    }
     if (l == 0) sLoss[wv] = se;
     __syncthreads();
-    float *P = partial + (size_t)blockIdx.x * MLP_NPARAMS;
     for (int p = threadIdx.x; p < MLP_NPARAMS; p += TWAVES * 64) P[p] = sum[p];
     if (threadIdx.x == 0) {
         float s = 0.0f;
@@ -959,7 +975,7 @@ static AdamStep adam_step(mdz_mlp *n, float lr) {
 static int mlp_gradient(mdz_mlp *n, long long first, int count, unsigned long long mul, unsigned long long add,
                         double *loss_acc, const float *lr) {
     if (count < TSAMP || count % TSAMP) return mdz_error(MDZ_EINVAL, "batch must be a multiple of 64");
-    const int tiles = count / 32, nb = std::min(TBLOCKS, mdz_div_up(tiles, TWAVES));
+    const int tiles = count / 32, nb = tiles <= TBLOCKS ? tiles : std::min(TBLOCKS, mdz_div_up(tiles, TWAVES));
     if (nb > n->partial_blocks) {
         hipFree(n->partial);
         hipFree(n->loss);

@@ -104,6 +104,47 @@ def test_forward_and_gradient_against_oracle(mdz, hot, net):
         assert e_64 <= 5e-2, k
 
 
+def _gradient(mdz, hot, net, first, count):
+    g, loss = np.zeros(mo.NPARAMS, np.float32), C.c_double()
+    mdz.check(hot.mdz_mlp_gradient(net, first, count, g.ctypes.data_as(FP), C.byref(loss)))
+    return g.astype(np.float64), loss.value
+
+
+@pytest.mark.parametrize("count", [64, 1024, 8192, 8256])
+def test_gradient_of_small_batches(mdz, hot, net, count):
+    """Batches up to 8192 take a block for each tile of 32 samples, larger
+    ones four tiles a block; here with ragged last blocks (258 tiles).  A
+    BF16 rounding that falls the other way moves a sample's term by 2^-8 in
+    each of the four layers at most."""
+    mdz.check(hot.mdz_mlp_generate(net, 9000, 7))
+    mdz.check(hot.mdz_mlp_init(net, 4))
+    X, Y = _samples(mdz, hot, net, count, 128)
+    g, loss = _gradient(mdz, hot, net, 128, count)
+    go, lo = mo.gradient(_weights(mdz, hot, net).astype(np.float64), X, Y, bf=True)
+    assert loss == pytest.approx(lo, rel=1e-3)
+    for k, (o, n) in mo.OFF.items():
+        e = np.linalg.norm(g[o:o + n] - go[o:o + n]) / np.linalg.norm(go[o:o + n])
+        print(count, k, "%.2e" % e)
+        assert e <= 4 * 2.0 ** -8, k
+
+
+def test_gradient_is_the_mean_of_its_halves(mdz, hot, net):
+    """16384 samples (four tiles a block) against their halves (a block for
+    each tile), and those against batches of 64: the same terms -- the
+    counts' ratios are powers of two -- in another order of FP32 sums
+    (512 partials: 512 x 6e-8)."""
+    mdz.check(hot.mdz_mlp_generate(net, 16384, 8))
+    mdz.check(hot.mdz_mlp_init(net, 5))
+    whole, loss = _gradient(mdz, hot, net, 0, 16384)
+    for size in (8192, 64):
+        parts = [_gradient(mdz, hot, net, k, size) for k in range(0, 16384, size)]
+        assert loss == pytest.approx(sum(p[1] for p in parts), rel=3e-5)
+        mean = sum(p[0] for p in parts) / len(parts)
+        e = np.linalg.norm(whole - mean) / np.linalg.norm(mean)
+        print(size, "%.2e" % e)
+        assert e <= 3e-5
+
+
 def test_inference_form_against_oracle(mdz, hot, net):
     """The network the grid guess evaluates (inference form: log2(e) folded
     into the weights, K-permuted rows on 16x16x32 tiles) against the
