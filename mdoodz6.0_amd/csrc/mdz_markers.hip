@@ -23,9 +23,9 @@
  * million markers in random order over 2.0 million quarter cells: counts 0.31
  * ms, placement 0.28, order 0.16, the step's two gathers 0.17 and 0.16; a
  * radix sort of keys and records took 0.85 ms for each node family and the
- * six gathers 0.75 (the step 2.6 -> 1.15 ms).  A bin of more than BIN_LONG
- * markers (its ordering is quadratic) sends the call to a stable
- * radix sort instead.
+ * six gathers 0.75 (the step 2.6 -> 1.15 ms).  The ordering is quadratic in
+ * a bin's markers: where the bins hold more than BIN_DENSE on average, or
+ * one holds more than BIN_LONG, a stable radix sort takes the call.
  *
  * The step of a time step with the 1-node stencil bins once for both node
  * families: by quarter cell, the pair of a marker's nearest centroid and
@@ -70,7 +70,13 @@ struct BinGrid {
     }
 };
 
+/* BIN_LONG: most markers of a bin that the ordering pass takes; BIN_DENSE: markers a bin, on
+ * average, up to which the counting sort is the faster one.  Measured, steps of 8.0 million markers
+ * (1-node stencil) in random and in seeding order: 25 a quarter cell 1.25 and 1.18 ms against 1.35
+ * and 1.34 with the radix sort; 64 a quarter cell 1.58 and 1.92 against 1.53 and 1.48 (markers in
+ * seeding order meet in the counts' atomics) */
 #define BIN_LONG 512
+#define BIN_DENSE 32
 
 /* rank of every marker in its bin, in no particular order; counts per bin */
 __global__ void __launch_bounds__(256) k_marker_count(MarkerSet m, BinGrid g, int *__restrict__ count,
@@ -149,12 +155,16 @@ int mdz_markers_bin(MarkerDev &md, int fam, const NodeAxes &a, const NodeAxes *v
         const BinGrid g{a, quarter ? *v : a, quarter};
         const dim3 grid(mdz_div_up(md.n, 256)), blk(256);
         int *flag = md.scan + md.scan_len - 1, total = 0;
-        if (hipMemsetAsync(flag, 0, sizeof(int), s) != hipSuccess) return mdz_error(MDZ_EHIP, "marker binning: flag");
-        hipLaunchKernelGGL(k_marker_count, grid, blk, 0, s, md.set(), g, start, md.key, flag);
-        if (hipMemcpyAsync(md.long_bin, flag, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
-            mdz_scan_exclusive(start, bins + 1, md.scan, md.scan_len - 1, s, &total) != MDZ_OK)
-            return mdz_error(MDZ_EHIP, "marker binning: scan"); /* (the total's copy waits for the stream) */
-        if (!*md.long_bin) {
+        bool sort = md.n > (long long)BIN_DENSE * bins;
+        if (!sort) {
+            if (hipMemsetAsync(flag, 0, sizeof(int), s) != hipSuccess) return mdz_error(MDZ_EHIP, "marker binning: flag");
+            hipLaunchKernelGGL(k_marker_count, grid, blk, 0, s, md.set(), g, start, md.key, flag);
+            if (hipMemcpyAsync(md.long_bin, flag, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
+                mdz_scan_exclusive(start, bins + 1, md.scan, md.scan_len - 1, s, &total) != MDZ_OK)
+                return mdz_error(MDZ_EHIP, "marker binning: scan"); /* (the total's copy waits for the stream) */
+            sort = *md.long_bin != 0;
+        }
+        if (!sort) {
             hipLaunchKernelGGL(k_marker_place, grid, blk, 0, s, md.set(), (const double *)md.val, g,
                                (const int *)start, (const int *)md.key, md.rec_in);
             if (total > 0)

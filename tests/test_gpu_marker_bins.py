@@ -64,6 +64,20 @@ def test_crowded_bin(mdz, orc, hot, active, itp):
         m.free()
 
 
+@pytest.mark.parametrize("itp,per_cell", [(1, (11, 11)), (1, (12, 12)), (9, (5, 6)), (9, (6, 6))])
+def test_dense_bins(mdz, orc, hot, itp, per_cell):
+    """Markers a bin below and above the 32 at which the radix sort takes
+    over: 30.25 and 36 a quarter cell, 30 and 36 a centroid."""
+    m = mdz.Model.lithosphere(14, 11, 4)
+    _softening(m)
+    m.m.model.itp_stencil = itp
+    mk = seed_markers(mdz, m, per_cell, seed=6, phase="layers", inactive=0.05, outside=10)
+    try:
+        _check_step(mdz, orc, hot, m, mk, 3)
+    finally:
+        m.free()
+
+
 @pytest.mark.parametrize("nx,nz", [(3, 3), (4, 3), (33, 3), (65, 17)])
 def test_small_grids_and_markers_outside(mdz, orc, hot, nx, nz):
     m = mdz.Model.lithosphere(nx, nz, 4)
