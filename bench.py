@@ -63,7 +63,7 @@ def stage_kernels(shape, learned=False, fused=True, net_in_rheology=True):
             "dtensor_jacobian": d1,
             "jacobian_values": values(1, jac, 21, 6),
             "dtensor_picard_2": d0,
-            "residual": ["k_residual_tile<true>", "k_norms_final_slots"]}
+            "residual": ["k_residual_tile", "k_norms_final_slots"]}
 
 
 # The strain rates and the vertex interpolation of div_u, T, P, d and phi
@@ -314,7 +314,8 @@ def device_solve(mdz, hot, ncx, ncz, seed, penalty=1e5):
     iterations around GCR, preconditioned by the sparse Cholesky factor of the
     penalised Picard operator) on the blocks of one Newton-iteration unit of
     a lithosphere model; the second of two solves is reported (the first
-    one initialises the dense-algebra libraries).  Not the metric."""
+    one also analyses the pattern, allocates the factor and captures the
+    preconditioner's launches).  Not the metric."""
     m = mdz.Model.lithosphere(ncx, ncz, seed)
     m.m.model.penalty = penalty
     ctx = C.c_void_p()

@@ -484,8 +484,10 @@ int  mdz_ctx_iteration_histogram(mdz_ctx *ctx, long long *hist192);
  * else about 0), local iterations
  * (centroid and vertex rheology kernels), right-hand sides, D(Picard),
  * Picard values, D(Jacobian), Jacobian values, D(Picard), residual + norms;
- * ms[10] = whole unit.  An isotropic model (aniso = 0) runs one fused D
- * pass, timed as D(Jacobian); both D(Picard) stages are then 0. */
+ * ms[10] = the whole of them.  An isotropic model (aniso = 0) runs one
+ * fused D pass, timed as D(Jacobian); both D(Picard) stages are then 0.
+ * The stages are launched apart here; a unit takes the right-hand sides
+ * with the D pass, and on small grids both value passes, in one launch. */
 int  mdz_ctx_stage_times(mdz_ctx *ctx, int reps, double *ms11);
 /* Mean milliseconds per unit over `reps` back-to-back units. */
 int  mdz_ctx_time_units(mdz_ctx *ctx, int reps, double *ms_per_unit);
