@@ -32,6 +32,8 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <new>
+
 #include "../../include/mdoodz_hot.h"
 #include "mdz_factor.h"
 #include "mdz_factor_plan.h"
@@ -703,7 +705,8 @@ static void nd_free(NdBuf<T> &b) {
 
 int mdz_factor_create(MdzFactor **out, hipStream_t s) {
     if (!out) return mdz_error(MDZ_EINVAL, "factor: null output");
-    *out = new MdzFactor();
+    *out = new (std::nothrow) MdzFactor();
+    if (!*out) return mdz_error(MDZ_ENOMEM, "factor: host memory");
     (*out)->s = s;
     return MDZ_OK;
 }

@@ -6,7 +6,6 @@
 #include <algorithm>
 #include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -32,7 +31,7 @@ void mdz_host_parallel(long long n, long long grain, Fn &&fn) {
     int started = 1;
     try {
         for (; started < nt; started++) th.emplace_back(chunk, started);
-    } catch (const std::system_error &) {
+    } catch (...) { /* no thread, or no memory for one */
     }
     chunk(0);
     for (int t = started; t < nt; t++) chunk(t);

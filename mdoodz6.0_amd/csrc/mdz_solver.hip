@@ -42,6 +42,7 @@
 #include <algorithm>
 #include <chrono>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "mdz_factor.h"
@@ -517,7 +518,8 @@ void mdz_solver_pdiag(int np, const int *cont_node, const int *comp_cells, const
 /* ------------------------------------------------------------------ */
 int mdz_solver_create(MdzSolver **out, hipStream_t s) {
     if (!out) return sv_err(MDZ_EINVAL, "solver: null output");
-    MdzSolver *S = new MdzSolver();
+    MdzSolver *S = new (std::nothrow) MdzSolver();
+    if (!S) return sv_err(MDZ_ENOMEM, "solver: host memory");
     S->s = s;
     const int rc = mdz_factor_create(&S->fac, s);
     if (rc) {

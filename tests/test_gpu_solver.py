@@ -217,8 +217,7 @@ def test_factor_is_an_exact_inverse(mdz, orc, hot):
 
 def test_killer_solver_dropin(mdz, orc, hot):
     """The drop-in on host blocks returns the context solve's correction
-    (to 1e-10: the library's factorisation kernels need not be bitwise
-    reproducible)."""
+    (to 1e-10)."""
     m = mdz.Model.lithosphere(96, 48, 2)
     m.m.model.penalty = 1e5
     gpu = None
